@@ -229,26 +229,11 @@ __global__ void k_weighted(const uint32_t* states, int64_t count, const double* 
   out[i] = acc;
 }
 
-__device__ inline double u_term(const HvArgs& a, uint32_t both) {
-  if (a.u_mode == 1) return a.u_uniform * (double)popc32(both);
-  if (a.u_mode == 2) {
-    double acc = 0.0;
-    uint32_t m = both & a.u_mask;
-    while (m) {
-      const int p = __builtin_ctz(m);
-      acc += a.u_site[p];
-      m &= m - 1;
-    }
-    return acc;
-  }
-  return 0.0;
-}
-
 __global__ void k_diagonal(HvArgs a, double* diag) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= a.num_up * a.num_dn) return;
   const int64_t iu = k / a.num_dn, id = k - iu * a.num_dn;
-  diag[k] = a.d_up[iu] + a.d_dn[id] + u_term(a, a.st_up[iu] & a.st_dn[id]);
+  diag[k] = a.d_up[iu] + a.d_dn[id] + hv_u_term(a, a.st_up[iu] & a.st_dn[id]);
 }
 
 // Dense H (row-major, H[target][origin]).  One thread per row: diagonal plus the
@@ -260,7 +245,7 @@ __global__ void k_dense(HvArgs a, double* h) {
   const int64_t iu = row / a.num_dn, id = row - iu * a.num_dn;
   double* hr = h + row * D;
   for (int64_t c = 0; c < D; ++c) hr[c] = 0.0;
-  hr[row] = a.d_up[iu] + a.d_dn[id] + u_term(a, a.st_up[iu] & a.st_dn[id]);
+  hr[row] = a.d_up[iu] + a.d_dn[id] + hv_u_term(a, a.st_up[iu] & a.st_dn[id]);
   const int cu = a.up_cnt[iu];
   for (int k = 0; k < cu; ++k) hr[(int64_t)a.up_col[iu * a.up_w + k] * a.num_dn + id] += a.up_val[iu * a.up_w + k];
   const int cd = a.dn_cnt[id];

@@ -250,6 +250,22 @@ struct HvArgs {
 
 HvArgs make_hv_args(const ed_op* op);
 
+// Interaction energy of a state whose doubly occupied sites are `both`.
+__device__ __forceinline__ double hv_u_term(const HvArgs& a, uint32_t both) {
+  if (a.u_mode == 1) return a.u_uniform * (double)popc32(both);
+  if (a.u_mode == 2) {
+    double acc = 0.0;
+    uint32_t m = both & a.u_mask;
+    while (m) {
+      const int p = __builtin_ctz(m);
+      acc += a.u_site[p];
+      m &= m - 1;
+    }
+    return acc;
+  }
+  return 0.0;
+}
+
 // Lanczos epilogue: y = s_j * H x - c_j * xprev, partial <y, x>.
 struct HvEpilogue {
   const double* xprev = nullptr;  // may be null
@@ -270,9 +286,43 @@ struct HvEpilogue {
 int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const HvEpilogue& epi,
                   hipStream_t stream, int* num_partials);
 int matvec_num_partials(const ed_op* op, int64_t ld);
+// Whether an H.v on rows of this stride runs as the single fused pass.
+bool matvec_is_fused(const ed_op* op, int64_t ld);
 // Row stride the library's own vectors use: num_dn rounded up to 16 doubles
 // (128-byte rows) where the two-pass sweep runs, num_dn otherwise.
 int64_t vector_ld(const ed_op* op);
+
+// Device-resident scalars of a Lanczos run of at most M steps.
+struct LzCoef {
+  double* alpha;  // [M]
+  double* beta;   // [M+1]
+  double* scale;  // [M+1]
+  double* cprev;  // [M+1]  beta_j * s_{j-1}
+  double* misc;   // [16]   0: breakdown flag, 1: one, 2..: scratch scalars
+};
+
+// beta_{j+1} = sqrt(S) from S = |w|^2, zero (breakdown) where it falls below
+// 1e-12 of ref = |alpha_j| + beta_j, is not finite (*bad) or the run had
+// broken down before.
+__device__ __forceinline__ double lanczos_beta(double S, double ref, bool broken, bool* bad) {
+  const double b = sqrt(fmax(S, 0.0));
+  *bad = !std::isfinite(b);
+  return broken || !(b > 1e-12 * ref) || *bad ? 0.0 : b;
+}
+
+// Fully reorthogonalised steps (ed_reorth.hip): blocks of 64 * sub states.
+struct ReorthGrid {
+  int blocks, sub;
+};
+ReorthGrid reorth_grid(int64_t D);
+bool reorth_available();                // the kernels' LDS is granted
+constexpr int kReorthMaxVectors = 256;  // basis vectors a step's kernels hold in LDS
+// Step j < kReorthMaxVectors from V_0..V_j (vectors of D doubles, contiguous
+// rows) into V_{j+1}: alpha_j, and |V_{j+1}|^2 as `blocks` partials in nout.
+// beta_j, s_j from the partials npart of the previous step (j > 0; may be
+// nout).  part, part2: kReorthMaxVectors * blocks doubles each.
+int launch_reorth_step(const ed_op* op, const double* V, int64_t D, int j, LzCoef c, double* part, double* part2,
+                       const double* npart, double* nout, hipStream_t s);
 
 // Deterministic reductions (ed_lanczos.hip).
 int launch_reduce(const double* partial, int n, double* out, int op_kind, hipStream_t stream);

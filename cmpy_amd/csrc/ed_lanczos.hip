@@ -27,28 +27,16 @@ namespace ed {
 
 enum RedKind { RED_NORM0 = 0, RED_ALPHA = 1, RED_BETA = 2, RED_SUM_TO = 3, RED_SQRT_TO = 4 };
 
-struct LzCoef {
-  double* alpha;  // [M]
-  double* beta;   // [M+1]
-  double* scale;  // [M+1]
-  double* cprev;  // [M+1]  beta_j * s_{j-1}
-  double* misc;   // [16]   0: breakdown flag, 1: one, 2..: scratch scalars
-};
-
 constexpr int kRedThreads = 1024;
 constexpr int kVecThreads = 256;
 
-// beta_{j+1} = sqrt(S) from S = |w|^2, zero (and the breakdown flag set)
-// where it falls below 1e-12 of |alpha_j| + beta_j or is not finite; then
+// beta_{j+1} (lanczos_beta, with the breakdown and non-finite flags), then
 // scale_{j+1} = 1/beta_{j+1} and cprev_{j+1} = beta_{j+1} scale_j.
 __device__ __forceinline__ void finish_beta(LzCoef c, int j, double S) {
-  double b = sqrt(fmax(S, 0.0));
-  const double ref = fabs(c.alpha[j]) + (j > 0 ? c.beta[j] : 0.0);
-  if (c.misc[0] != 0.0 || !(b > 1e-12 * ref) || !isfinite(b)) {
-    if (!isfinite(b)) c.misc[3] = 1.0;
-    b = 0.0;
-    c.misc[0] = 1.0;
-  }
+  bool bad;
+  const double b = lanczos_beta(S, fabs(c.alpha[j]) + (j > 0 ? c.beta[j] : 0.0), c.misc[0] != 0.0, &bad);
+  if (bad) c.misc[3] = 1.0;
+  if (b == 0.0) c.misc[0] = 1.0;
   c.beta[j + 1] = b;
   c.scale[j + 1] = b > 0.0 ? 1.0 / b : 0.0;
   c.cprev[j + 1] = b * c.scale[j];
@@ -532,14 +520,16 @@ void tri_lowest_vector(const double* a, const double* b, int m, double lam, std:
 // Partials: region A (npart doubles: the H.v sweep's and the Gram-Schmidt
 // dot products'), M + 2 coefficients, region B (npart2 doubles: the vector
 // updates' |w|^2), then with reorthogonalisation the orthogonality estimate
-// (3 (M + 2) doubles and two flags).
+// (3 (M + 2) doubles and two flags) and the three-launch step's partials (two
+// sets of dots and |w|^2).
 struct LzLayout {
-  int64_t coef_off, part_off, part2_off, pro_off, vec_off, total;
+  int64_t coef_off, part_off, part2_off, pro_off, dots_off, vec_off, total;
   int64_t D;           // doubles per stored vector: nu rows of ld (zeros past nd)
   int64_t nu, nd, ld;  // rows, states per row, row stride
   int M;
   int nvec;
   int npart, npart2;
+  int64_t ndots;  // doubles of one set of the three-launch step's dots
 };
 
 static int64_t align256(int64_t b) { return (b + 255) & ~int64_t(255); }
@@ -563,7 +553,10 @@ static LzLayout lz_layout(const ed_op* op, int M, int reorth, int want_vector, i
   L.part2_off = align256(L.part_off + sizeof(double) * (int64_t)(L.npart + M + 2));
   L.pro_off = align256(L.part2_off + sizeof(double) * (int64_t)L.npart2);
   const int64_t pro_bytes = reorth ? (int64_t)sizeof(double) * (3 * ((int64_t)M + 2) + 1) : 0;
-  L.vec_off = align256(L.pro_off + pro_bytes);
+  L.dots_off = align256(L.pro_off + pro_bytes);
+  const int64_t rb = reorth_grid(L.D).blocks;
+  L.ndots = kReorthMaxVectors * rb;
+  L.vec_off = align256(L.dots_off + (reorth ? (int64_t)sizeof(double) * (2 * L.ndots + rb) : 0));
   L.total = L.vec_off + align256(sizeof(double) * L.D) * L.nvec;
   return L;
 }
@@ -677,10 +670,32 @@ struct ReorthCtx {
   double* part2;  // region B
   int64_t chunks, chunk;
   int gx;         // k_multidot blocks along the chunks (dot partials per vector)
+  // three-launch steps (ed_reorth.hip): their partials, and the step whose
+  // beta is still only a set of partials (-1: none)
+  double *dots, *dots2, *norms;
+  int blocks;
+  bool three = false;
+  int pending = -1;
 };
 
-static ReorthCtx reorth_ctx(char* base, const LzLayout& L, double* part) {
+// Sectors up to this many states take the three-launch step, whose H.v deals
+// a state's hops over the waves of its block; beyond it k_reorth_hv's gathers
+// are no match for the sweep of a whole sector (12-site chain, 853,776 states:
+// 20 us).  A full solve, seven launches a step before: 4,900 states (ground
+// state and two 200-step fractions) 28.1 -> 10.9 ms, 400 states 17.6 -> 10.2
+// ms, 63,504 states (ground state) 6.5 -> 4.2 ms.
+constexpr int64_t kReorthMaxStates = int64_t(1) << 18;
+
+// three: the three-launch steps may be used (full reorthogonalisation, no
+// timing of the H.v).
+static ReorthCtx reorth_ctx(const ed_op* op, char* base, const LzLayout& L, double* part, bool three) {
   ReorthCtx r;
+  r.dots = reinterpret_cast<double*>(base + L.dots_off);
+  r.dots2 = r.dots + L.ndots;
+  r.norms = r.dots2 + L.ndots;
+  r.blocks = reorth_grid(L.D).blocks;
+  r.three = three && L.ld == L.nd && L.D <= kReorthMaxStates && matvec_is_fused(op, L.ld) &&
+            reorth_available();
   r.V = vec_ptr(base, L, 0);
   r.w = vec_ptr(base, L, L.M + 1);
   r.coefs = part + L.npart;
@@ -793,6 +808,16 @@ static int pro_init(ProState& pro, char* base, const LzLayout& L, hipStream_t s)
   return ED_OK;
 }
 
+// beta_{j+1} of a three-launch step whose next step has not formed it.
+static int reorth_finish(LzCoef c, ReorthCtx& r, hipStream_t s) {
+  if (r.pending < 0) return ED_OK;
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, r.norms, r.blocks, (int)RED_BETA, c, r.pending,
+                     nullptr);
+  r.pending = -1;
+  ED_HIP(hipGetLastError());
+  return ED_OK;
+}
+
 // Step j, with the basis kept unnormalised (v_i = scale_i V_i, as the
 // three-vector recurrence keeps its vectors): W = V_{j+1} = s_j H V_j -
 // beta_j s_{j-1} V_{j-1}; alpha_j = s_j <W, V_j> (formed in the update);
@@ -804,9 +829,15 @@ static int pro_init(ProState& pro, char* base, const LzLayout& L, hipStream_t s)
 // the two H.v sweeps, the update, then with a ProState the estimate (which
 // sets beta_{j+1} when no pass is due) and three gated kernels (dots,
 // combination, beta); without, two passes of (dots, combination) and beta.
-static int reorth_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, const ReorthCtx& r, int j,
+static int reorth_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, ReorthCtx& r, int j,
                        hipStream_t s, EventTimer* tm, const ProState* pro = nullptr) {
   const int64_t D = L.D;
+  if (r.three && j < kReorthMaxVectors) {
+    ED_TRY(launch_reorth_step(op, r.V, D, j, c, r.dots, r.dots2, r.norms, r.norms, s));
+    r.pending = j;
+    return ED_OK;
+  }
+  ED_TRY(reorth_finish(c, r, s));
   const int vb = vec_blocks(D);
   double* vj = r.V + (int64_t)j * D;
   double* w = r.V + (int64_t)(j + 1) * D;
@@ -975,7 +1006,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
     }
   } else {
     // full or partial reorthogonalisation: V holds normalised basis vectors
-    const ReorthCtx rc = reorth_ctx(base, L, part);
+    ReorthCtx rc = reorth_ctx(op, base, L, part, cfg->reorth == 1 && !tm.on);
     double* V = rc.V;
     double* coefs = rc.coefs;
     ED_TRY(reorth_start(L, c, part, rc, v0_dev, cfg->seed, s));
@@ -988,6 +1019,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
       const bool last = (j + 1 == M);
       const bool due = !cfg->fixed_iter && steps >= cfg->min_iter && (steps % cfg->check_every == 0);
       if (due || last) {
+        ED_TRY(reorth_finish(c, rc, s));
         ED_TRY(check(steps));
         if (breakdown || ritz <= cfg->tol) {
           converged = true;
@@ -1071,11 +1103,12 @@ extern "C" int ed_lanczos_coeffs(ed_op* op, const double* v0_dev, int32_t nsteps
   const int vb = vec_blocks(D);
   hipLaunchKernelGGL(k_init_misc, dim3(1), dim3(64), 0, s, c.misc);
   if (reorth) {
-    const ReorthCtx rc = reorth_ctx(base, L, part);
+    ReorthCtx rc = reorth_ctx(op, base, L, part, reorth == 1);
     ED_TRY(reorth_start(L, c, part, rc, v0_dev, 0, s));
     ProState pro{nullptr, nullptr, M};
     if (reorth == 2) ED_TRY(pro_init(pro, base, L, s));
     for (int j = 0; j < M; ++j) ED_TRY(reorth_step(op, L, c, part, rc, j, s, nullptr, reorth == 2 ? &pro : nullptr));
+    ED_TRY(reorth_finish(c, rc, s));
     // basis vector j is rc.V + j D, scaled by scale_j
     if (basis_dev) launch_compact(L, s, basis_dev, rc.V, D, M, c.scale, 0);
   } else {

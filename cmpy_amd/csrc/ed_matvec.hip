@@ -17,21 +17,6 @@
 
 namespace ed {
 
-__device__ __forceinline__ double u_term_dev(const HvArgs& a, uint32_t both) {
-  if (a.u_mode == 1) return a.u_uniform * (double)popc32(both);
-  if (a.u_mode == 2) {
-    double acc = 0.0;
-    uint32_t m = both & a.u_mask;
-    while (m) {
-      const int p = __builtin_ctz(m);
-      acc += a.u_site[p];
-      m &= m - 1;
-    }
-    return acc;
-  }
-  return 0.0;
-}
-
 __device__ __forceinline__ double block_sum_256(double v, double* red) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
@@ -71,7 +56,7 @@ __global__ __launch_bounds__(256) void k_hv(HvArgs a, const double* __restrict__
       const int64_t iu = r0 + r;
       if (iu < a.num_up) {
         xo[r] = x[iu * ld + id];
-        acc[r] = (a.d_up[iu] + ddn + u_term_dev(a, a.st_up[iu] & sdn)) * xo[r];
+        acc[r] = (a.d_up[iu] + ddn + hv_u_term(a, a.st_up[iu] & sdn)) * xo[r];
       } else {
         xo[r] = 0.0;
         acc[r] = 0.0;
@@ -1541,6 +1526,8 @@ int matvec_num_partials(const ed_op* op, int64_t ld) {
   grid_shape(op, pick_rb(op), ld, &nrb, &nct);
   return (int)(nrb * nct);
 }
+
+bool matvec_is_fused(const ed_op* op, int64_t ld) { return !plan_two_pass(op, ld).ok; }
 
 int64_t vector_ld(const ed_op* op) {
   const int64_t nd = op->num_dn;
