@@ -161,6 +161,8 @@ struct Hv2Args {
   int32_t up_quad_stride;
   const double* hop;
   int32_t nb;
+  const double* up_val;         // [nu][up_w] hop values, sign included
+  const double* dn_val;         // [dn_w][nd]
   int32_t u_mode;
   double u_uniform;
   uint32_t u_mask;
@@ -630,6 +632,148 @@ __global__ __launch_bounds__(kRowThreads) void k_hv_rows_held(Hv2Args a, int row
   if (e.partial) {
     const double s = block_sum_n<kRowThreads>(dot, red);
     if (threadIdx.x == 0) e.partial[blockIdx.x] = s;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Single fused pass on staged rows: a block stages RB rows of x in LDS and
+// each of its waves takes 64-column chunks of them.  Up hops are read from x
+// itself (one list per row, wave-uniform: scalar loads; every hop a contiguous
+// 64-column piece of another row, eight in flight), dn hops are LDS gathers
+// through the packed column-major table, whose entries serve all RB rows.
+// Blocks go to XCDs in contiguous runs of rows, whose hop sources lie mostly
+// near them.  blockIdx.y picks the vector.  Every wave has a chunk (at most
+// nch waves a block).
+// ---------------------------------------------------------------------------
+constexpr int kTileDn = 4;  // dn slots per step; the next step's entries are loaded ahead
+
+template <int RB, bool UNI, bool LZ>
+__global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __restrict__ x, double* __restrict__ y,
+                                                  HvEpilogue e, int nrg, int per_xcd, int64_t vstride) {
+  extern __shared__ double rows[];  // [RB][nd]
+  __shared__ double red[16];
+  const int rg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if (rg >= nrg) {  // the whole block
+    if (LZ && e.partial && threadIdx.x == 0) e.partial[blockIdx.x] = 0.0;
+    return;
+  }
+  const int nd = (int)a.nd, nt = (int)blockDim.x;
+  const int64_t ld = a.ld;
+  const int r0 = rg * RB;
+  const int R = (int)a.nu - r0 < RB ? (int)a.nu - r0 : RB;
+  x += (int64_t)blockIdx.y * vstride;
+  y += (int64_t)blockIdx.y * vstride;
+  for (int k = threadIdx.x; k < nd; k += nt) {
+    double v[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) v[r] = x[(int64_t)(r0 + (r < R ? r : 0)) * ld + k];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) rows[r * nd + k] = v[r];
+  }
+  zero_row_pads(y, r0, R, nd, ld);
+  const double t = UNI ? a.hop[0] : 1.0;
+  const double sx = LZ && e.sx ? *e.sx : 1.0;
+  const double cp = LZ && e.cprev ? *e.cprev : 0.0;
+  const double cs = LZ && e.cself ? *e.cself : 0.0;
+  const double ps = LZ ? e.psi_y * sx : 0.0;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  constexpr int UP = RB == 4 ? 4 : 8;  // up hops of a row whose loads are in flight together
+  int cu[RB], cmax = 0;
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    cu[r] = r < R ? uniform_load(a.up_cnt + (r0 + r)) : 0;
+    cmax = cmax > cu[r] ? cmax : cu[r];
+  }
+  double dot = 0.0;
+  bool first = true;
+  for (int c0 = wave * 64; c0 < nd; c0 += nt) {
+    const int id = c0 + lane;
+    const bool act = id < nd;
+    const int ids = act ? id : nd - 1;
+    const int cnt = act ? a.dn_cnt[ids] : 0;
+    const uint32_t sdn = a.st_dn[ids];
+    const double ddn = a.d_dn[ids];
+    double acc[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) acc[r] = 0.0;
+    for (int e0 = 0; e0 < cmax; e0 += UP) {
+      double g[RB][UP], v[RB][UP];
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int q = 0; q < UP; ++q) {
+          const int64_t k = (int64_t)(r0 + (r < R ? r : 0)) * a.up_w + (e0 + q < cu[r] ? e0 + q : 0);
+          const uint32_t en = uniform_load(a.up_pk + k);
+          const double h = UNI ? ((en & 0x80000000u) ? -1.0 : 1.0) : uniform_load(a.up_val + k);
+          v[r][q] = e0 + q < cu[r] ? h : 0.0;
+          g[r][q] = (x + (int64_t)hop_target(en) * ld)[ids];
+        }
+#pragma unroll
+      for (int r = 0; r < RB; ++r)
+#pragma unroll
+        for (int q = 0; q < UP; ++q) acc[r] = fma(v[r][q], g[r][q], acc[r]);
+    }
+    if (first) __syncthreads();  // every wave passes here once
+    first = false;
+    const int w1 = a.dn_w - 1;
+    uint32_t en[kTileDn];
+    double vl[kTileDn];
+#pragma unroll
+    for (int q = 0; q < kTileDn; ++q) {
+      const int64_t k = (int64_t)(q < w1 ? q : w1) * nd + ids;
+      en[q] = a.dn_pk[k];
+      if (!UNI) vl[q] = a.dn_val[k];
+    }
+    for (int e0 = 0; __ballot(e0 < cnt); e0 += kTileDn) {
+      uint32_t cur[kTileDn];
+      double v[kTileDn];
+#pragma unroll
+      for (int q = 0; q < kTileDn; ++q) {
+        cur[q] = en[q];
+        const double h = UNI ? ((en[q] & 0x80000000u) ? -1.0 : 1.0) : vl[q];
+        v[q] = e0 + q < cnt ? h : 0.0;
+        const int n = e0 + kTileDn + q;
+        const int64_t k = (int64_t)(n < w1 ? n : w1) * nd + ids;
+        en[q] = a.dn_pk[k];
+        if (!UNI) vl[q] = a.dn_val[k];
+      }
+#pragma unroll
+      for (int q = 0; q < kTileDn; ++q) {
+        const int tg = hop_target(cur[q]);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) acc[r] = fma(v[q], rows[r * nd + tg], acc[r]);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      if (r < R && act) {
+        const int iu = r0 + r;
+        const int64_t k = (int64_t)iu * ld + id;
+        const double xo = rows[r * nd + id];
+        const double h = (a.d_up[iu] + ddn + u_term2(a, a.st_up[iu] & sdn)) * xo + t * acc[r];
+        if (LZ) {
+          double v = sx * (h - cs * xo);
+          if (e.xprev) v -= cp * e.xprev[k];
+          y[k] = v;
+          if (e.psi) e.psi[k] += ps * xo;
+          dot += v * xo;
+        } else {
+          y[k] = h;
+        }
+      }
+    }
+  }
+  if (LZ && e.partial) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) dot += __shfl_down(dot, off, 64);
+    if (lane == 0) red[wave] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double s = 0.0;
+      for (int w = 0; w < nt / 64; ++w) s += red[w];
+      e.partial[blockIdx.x] = s;
+    }
   }
 }
 
@@ -1269,6 +1413,8 @@ static Hv2Args make_hv2_args(const ed_op* op, int64_t ld) {
   a.up_quad_stride = op->up.quad_stride;
   a.hop = op->hop_dev;
   a.nb = op->num_bonds;
+  a.up_val = op->up.val_rm;
+  a.dn_val = op->dn.val_cm;
   a.u_mode = op->u_mode;
   a.u_uniform = op->u_uniform;
   a.u_mask = op->u_mask;
@@ -1361,13 +1507,64 @@ static ColKernel col_kernel_split(int tw, int maxl) {
 
 constexpr int64_t kMinRowBlocks = 512;
 
-// Below this many states the single fused pass (k_hv) is the faster sweep:
-// its rows gather their up-hop sources straight from x, which at this size
-// stays in the caches, and it is one launch instead of two.  Measured
-// back-to-back on MI355X: 12-site chain (6,6), D = 853,776: 19.0 us fused
-// against 26.5 us in two passes; 14-site chain (7,7), D = 11.8 M: 208 against
-// 177 us; 4x4 (5,5), D = 19.1 M: 1063 against 307 us (break-even near 3 M).
-constexpr int64_t kTwoPassMinStates = int64_t(1) << 21;
+// Fused pass on staged rows (k_hv_tile): where the packed tables exist and a
+// row fits the LDS budget.
+struct TilePlan {
+  bool ok;
+  int rb, threads, nrg, per_xcd;
+  size_t lds_bytes;
+  int grid() const { return 8 * per_xcd; }
+};
+using TileKernel = void (*)(Hv2Args, const double*, double*, HvEpilogue, int, int, int64_t);
+
+template <int RB>
+static TileKernel tile_kernel_rb(bool uni, bool lz) {
+  if (uni) return lz ? k_hv_tile<RB, true, true> : k_hv_tile<RB, true, false>;
+  return lz ? k_hv_tile<RB, false, true> : k_hv_tile<RB, false, false>;
+}
+
+static TileKernel tile_kernel(int rb, bool uni, bool lz) {
+  return rb == 4 ? tile_kernel_rb<4>(uni, lz) : rb == 2 ? tile_kernel_rb<2>(uni, lz) : tile_kernel_rb<1>(uni, lz);
+}
+
+constexpr int64_t kTileWaves = 2048;    // waves that keep the chip busy (2 per SIMD)
+constexpr size_t kTileLds = 64 * 1024;  // granted without an attribute, and two blocks fit a CU
+constexpr int kTileMaxThreads = 1024;
+
+// Rows per block: as many as keep kTileWaves waves in flight, up to four (the
+// dn table's entries are read once for all of a block's rows; 12-site chain:
+// 14.1 us with four rows, 15.2 with two, 16.7 with one).
+
+static TilePlan plan_tile(const ed_op* op) {
+  TilePlan p{};
+  if (!op->packed || op->size == 0) return p;
+  const int64_t nch = (op->num_dn + 63) / 64;
+  const int64_t iters = (nch + kTileMaxThreads / 64 - 1) / (kTileMaxThreads / 64);
+  const int64_t waves = (nch + iters - 1) / iters;
+  p.threads = (int)waves * 64;
+  p.rb = 4;
+  for (; p.rb > 1; p.rb /= 2)
+    if (p.rb * op->num_dn * sizeof(double) <= kTileLds - 128 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
+  p.lds_bytes = p.rb * op->num_dn * sizeof(double);
+  if (p.lds_bytes > kTileLds - 128) return p;  // the kernel has static LDS of its own
+  p.nrg = (int)((op->num_up + p.rb - 1) / p.rb);
+  p.per_xcd = (p.nrg + 7) / 8;
+  p.ok = true;
+  return p;
+}
+
+// Below this many states the single fused pass is the faster sweep: its rows
+// gather their up-hop sources straight from x, which at this size stays in the
+// last-level cache, and it is one launch instead of two.  Measured with
+// k_hv_tile against two passes: 12-site chain (6,6), D = 853,776: 14.1 against
+// 27.1 us; 13-site chain (6,5), 2.2 M: 30.6 against 50.4; 4x4 (4,4), 3.3 M: 57
+// against 73; 14-site chain (7,7), 11.8 M: 165 against 185 (1+13-site impurity:
+// 147 against 192); 4x4 (5,5), 19 M: 439 against 316; 15-site chain (7,7), 41 M:
+// 745 against 634.
+constexpr int64_t kTwoPassMinStates = int64_t(1) << 24;
+// The same for rows that do not fit k_hv_tile's LDS (k_hv otherwise: 4x4 (5,5)
+// 1063 against 316 us, 12-site chain 19.0 against 27.1).
+constexpr int64_t kTwoPassMinStatesLongRows = int64_t(1) << 21;
 
 // Two-pass plan.  Kernels: sign-split tables when hopping is uniform and the
 // tables exist (CMPY_AMD_HV_SPLIT=0 turns them off), general packed tables
@@ -1378,7 +1575,7 @@ static TwoPassPlan plan_two_pass(const ed_op* op, int64_t ld) {
   p.ok = false;
   const int mode = op->hv_mode >= 0 ? op->hv_mode : env_int("CMPY_AMD_HV_MODE", -1);
   if (!op->packed || mode == 0) return p;
-  if (mode < 0 && op->size < kTwoPassMinStates) return p;
+  if (mode < 0 && op->size < (plan_tile(op).ok ? kTwoPassMinStates : kTwoPassMinStatesLongRows)) return p;
   const int maxh_up = maxh_for(op->max_hops_up);
   if (!maxh_up || !maxh_for(op->max_hops_dn)) return p;
   bool uni = op->num_bonds > 0;
@@ -1522,6 +1719,8 @@ static void grid_shape(const ed_op* op, int rb, int64_t ld, int64_t* nrb, int64_
 int matvec_num_partials(const ed_op* op, int64_t ld) {
   const TwoPassPlan p = plan_two_pass(op, ld);
   if (p.ok) return (int)(p.col_first ? p.grid_r : p.grid_r + p.grid_c);
+  const TilePlan tp = plan_tile(op);
+  if (tp.ok) return tp.grid();
   int64_t nrb, nct;
   grid_shape(op, pick_rb(op), ld, &nrb, &nct);
   return (int)(nrb * nct);
@@ -1551,17 +1750,47 @@ static void launch_rb(int rb, const HvArgs& a, const double* x, double* y, const
   }
 }
 
+static int launch_tile(const ed_op* op, const TilePlan& p, const double* x, double* y, int64_t ld, int64_t nvec,
+                       bool lz, const HvEpilogue& epi, hipStream_t s) {
+  hipLaunchKernelGGL(tile_kernel(p.rb, op->uniform_hop && op->num_bonds > 0, lz),
+                     dim3((unsigned)p.grid(), (unsigned)nvec), dim3((unsigned)p.threads), p.lds_bytes, s,
+                     make_hv2_args(op, ld), x, y, epi, p.nrg, p.per_xcd, op->num_up * ld);
+  ED_HIP(hipGetLastError());
+  return ED_OK;
+}
+
+// y = H x for nvec vectors one after another: one launch where the fused pass
+// on staged rows applies.
+static int matvec_block(const ed_op* op, const double* x, double* y, int64_t ld, int64_t nvec, hipStream_t s) {
+  const HvEpilogue none{nullptr, nullptr, nullptr, nullptr};
+  const int64_t n = op->num_up * ld;
+  const TilePlan tp = plan_two_pass(op, ld).ok ? TilePlan{} : plan_tile(op);
+  const int64_t step = tp.ok ? 65535 : 1;
+  for (int64_t v = 0; v < nvec; v += step) {
+    if (tp.ok)
+      ED_TRY(launch_tile(op, tp, x + v * n, y + v * n, ld, std::min(step, nvec - v), false, none, s));
+    else
+      ED_TRY(launch_matvec(op, x + v * n, y + v * n, ld, none, s, nullptr));
+  }
+  return ED_OK;
+}
+
 int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const HvEpilogue& epi, hipStream_t s,
                   int* num_partials) {
   const TwoPassPlan p = plan_two_pass(op, ld);
   if (p.ok) return launch_two_pass(op, p, x, y, ld, epi, s, num_partials);
+  const bool lz = epi.xprev || epi.sx || epi.cprev || epi.partial || epi.cself || epi.psi;
+  const TilePlan tp = plan_tile(op);
+  if (tp.ok) {
+    if (num_partials) *num_partials = tp.grid();
+    return launch_tile(op, tp, x, y, ld, 1, lz, epi, s);
+  }
   HvArgs a = make_hv_args(op);
   a.ld = ld;
   const int rb = pick_rb(op);
   int64_t nrb, nct;
   grid_shape(op, rb, ld, &nrb, &nct);
   ED_REQUIRE(nrb * nct < (1ll << 31), "grid too large");
-  const bool lz = epi.xprev || epi.sx || epi.cprev || epi.partial || epi.cself || epi.psi;
   if (lz)
     launch_rb<true>(rb, a, x, y, epi, nrb, nct, s);
   else
@@ -1609,10 +1838,7 @@ extern "C" int ed_op_matvec(ed_op* op, const double* x_dev, double* y_dev, int64
   const char* yb = (const char*)y_dev;
   ED_REQUIRE(xb + sizeof(double) * D * nvec <= yb || yb + sizeof(double) * D * nvec <= xb,
              "x and y overlap");
-  HvEpilogue none{nullptr, nullptr, nullptr, nullptr};
-  for (int64_t v = 0; v < nvec; ++v)
-    ED_TRY(launch_matvec(op, x_dev + v * D, y_dev + v * D, op->num_dn, none, as_stream(stream), nullptr));
-  return ED_OK;
+  return matvec_block(op, x_dev, y_dev, op->num_dn, nvec, as_stream(stream));
 }
 
 extern "C" int ed_op_matvec_ld(ed_op* op, const double* x_dev, double* y_dev, int64_t ld, int64_t nvec,
@@ -1626,10 +1852,7 @@ extern "C" int ed_op_matvec_ld(ed_op* op, const double* x_dev, double* y_dev, in
   const char* xb = (const char*)x_dev;
   const char* yb = (const char*)y_dev;
   ED_REQUIRE(xb + sizeof(double) * n * nvec <= yb || yb + sizeof(double) * n * nvec <= xb, "x and y overlap");
-  HvEpilogue none{nullptr, nullptr, nullptr, nullptr};
-  for (int64_t v = 0; v < nvec; ++v)
-    ED_TRY(launch_matvec(op, x_dev + v * n, y_dev + v * n, ld, none, as_stream(stream), nullptr));
-  return ED_OK;
+  return matvec_block(op, x_dev, y_dev, ld, nvec, as_stream(stream));
 }
 
 extern "C" int ed_op_vector_ld(const ed_op* op, int64_t* ld) {

@@ -1,0 +1,41 @@
+"""H.v through the fused pass on staged rows at the edges of its layout: rows shorter than, equal to and just past a
+wave's 64 columns and past one pass of a block, row counts that leave a partial row group or whole idle blocks,
+one, two and four rows per block, uniform and per-bond hopping, several vectors in one call, padded strides.
+
+Against the oracle's operator to 1e-13 of the largest entry (the bound of every H.v path)."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ed_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ns,nu,nd", [(1, 0, 1), (4, 2, 0), (4, 0, 2), (6, 3, 1), (8, 4, 4), (8, 1, 3), (9, 2, 4),
+                                      (10, 5, 5), (11, 3, 5), (13, 6, 3), (13, 4, 6), (14, 2, 7)])
+def test_fused_rows_vs_oracle(gpu, ns, nu, nd, uniform):
+    from cmpy_amd import SectorHamiltonOperator
+
+    rng = np.random.default_rng(ns * 100 + nu * 10 + nd)
+    bonds = [(i, j) for i in range(ns) for j in range(i + 1, ns) if j == i + 1 or rng.random() < 0.3]
+    hops = np.full(len(bonds), -0.7) if uniform else rng.uniform(-1, 1, len(bonds))
+    eps, u = rng.uniform(-1, 1, ns), rng.uniform(0, 4, ns)
+    op = SectorHamiltonOperator(ns, nu, nd, bonds, hops, eps, u, ns)
+    ref = O.SectorOperator(ns, nu, nd, bonds, hops, eps, u, ns)
+    nvec = 3
+    x = rng.standard_normal((nvec, ref.size))
+    want = np.stack([ref.matvec(v) for v in x])
+    tol = 1e-13 * max(np.abs(want).max(), 1.0)
+    got = op.matvec_device(torch.from_numpy(x).cuda()).cpu().numpy()
+    assert np.abs(got - want).max() <= tol
+    ld = op.num_dn + 3
+    xp = np.full((nvec, op.num_up, ld), np.nan)
+    xp[:, :, :op.num_dn] = x.reshape(nvec, op.num_up, op.num_dn)
+    yp = torch.full((nvec, op.num_up, ld), float("nan"), dtype=torch.float64, device="cuda")
+    op.matvec_device_ld(torch.from_numpy(xp).cuda(), ld, out=yp)
+    yp = yp.cpu().numpy()
+    assert np.all(yp[:, :, op.num_dn:] == 0.0)
+    assert np.abs(yp[:, :, :op.num_dn].reshape(nvec, -1) - want).max() <= tol
