@@ -266,32 +266,6 @@ __device__ __forceinline__ double hv_u_term(const HvArgs& a, uint32_t both) {
   return 0.0;
 }
 
-// Lanczos epilogue: y = s_j * H x - c_j * xprev, partial <y, x>.
-struct HvEpilogue {
-  const double* xprev = nullptr;  // may be null
-  const double* sx = nullptr;     // device scalar: scale of x (null = 1)
-  const double* cprev = nullptr;  // device scalar: coefficient of xprev (null = 0)
-  double* partial = nullptr;      // per-block partial dots (null = none)
-  // Recurrence with known coefficients (the eigenvector's second pass):
-  // y = H (sx x) - cself sx x - cprev xprev, and psi += psi_y sx x over the
-  // sector entries (row padding untouched).  Applied by the row pass.
-  const double* cself = nullptr;  // device scalar (null = 0)
-  double* psi = nullptr;          // null = none
-  double psi_y = 0.0;
-};
-
-// Launch helpers implemented in ed_matvec.hip.  Vectors are stored row by
-// row at a stride of ld >= num_dn doubles; the H.v writes zeros into y's
-// entries num_dn .. ld-1 of every row and never reads those of x.
-int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const HvEpilogue& epi,
-                  hipStream_t stream, int* num_partials);
-int matvec_num_partials(const ed_op* op, int64_t ld);
-// Whether an H.v on rows of this stride runs as the single fused pass.
-bool matvec_is_fused(const ed_op* op, int64_t ld);
-// Row stride the library's own vectors use: num_dn rounded up to 16 doubles
-// (128-byte rows) where the two-pass sweep runs, num_dn otherwise.
-int64_t vector_ld(const ed_op* op);
-
 // Device-resident scalars of a Lanczos run of at most M steps.
 struct LzCoef {
   double* alpha;  // [M]
@@ -310,6 +284,82 @@ __device__ __forceinline__ double lanczos_beta(double S, double ref, bool broken
   return broken || !(b > 1e-12 * ref) || *bad ? 0.0 : b;
 }
 
+// beta_{j+1}, scale_{j+1} and cprev_{j+1} from partials of |w|^2 of step j that
+// an earlier launch left: n[0] of them, or n[1] where *which is set.
+struct HvBeta {
+  const double* part = nullptr;
+  int n[2] = {0, 0};
+  const int* which = nullptr;  // null: n[0]
+  LzCoef c{};
+  int j = -1;                  // -1: nothing to form
+};
+
+// The calling thread's share of the partials' sum, thread `at` of `step`.
+__device__ __forceinline__ double beta_share(const HvBeta& b, int at, int step) {
+  const int n = b.which && *b.which ? b.n[1] : b.n[0];
+  double S = 0.0;
+  for (int i = at; i < n; i += step) S += b.part[i];
+  return S;
+}
+
+// scale_{j+1} from the whole sum S, and cprev_{j+1} in *cp; one thread of the
+// launch stores the results and the flags of a broken run, which are not read
+// here, so blocks need no order among them.
+__device__ __forceinline__ double beta_scale(const HvBeta& b, double S, bool store, double* cp) {
+  bool bad;
+  const double sj = b.c.scale[b.j];
+  const double bt = lanczos_beta(S, fabs(b.c.alpha[b.j]) + (b.j > 0 ? b.c.beta[b.j] : 0.0), sj == 0.0, &bad);
+  const double sn = bt > 0.0 ? 1.0 / bt : 0.0;
+  *cp = bt * sj;
+  if (store) {
+    if (bad) b.c.misc[3] = 1.0;
+    if (bt == 0.0) b.c.misc[0] = 1.0;
+    b.c.beta[b.j + 1] = bt;
+    b.c.scale[b.j + 1] = sn;
+    b.c.cprev[b.j + 1] = bt * sj;
+  }
+  return sn;
+}
+
+// Both, by every wave of the block for itself.
+__device__ __forceinline__ double form_beta(const HvBeta& b, bool store, double* cp) {
+  double S = beta_share(b, threadIdx.x & 63, 64);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) S += __shfl_xor(S, off, 64);
+  return beta_scale(b, S, store && threadIdx.x == 0, cp);
+}
+
+// Lanczos epilogue: y = s_j * H x - c_j * xprev, partial <y, x>.
+struct HvEpilogue {
+  const double* xprev = nullptr;  // may be null
+  const double* sx = nullptr;     // device scalar: scale of x (null = 1)
+  const double* cprev = nullptr;  // device scalar: coefficient of xprev (null = 0)
+  double* partial = nullptr;      // per-block partial dots (null = none)
+  // Recurrence with known coefficients (the eigenvector's second pass):
+  // y = H (sx x) - cself sx x - cprev xprev, and psi += psi_y sx x over the
+  // sector entries (row padding untouched).  Applied by the row pass.
+  const double* cself = nullptr;  // device scalar (null = 0)
+  double* psi = nullptr;          // null = none
+  double psi_y = 0.0;
+  // sx and cprev's values formed by the H.v itself first (matvec_forms_beta);
+  // sx and cprev then point at the entries it stores them in.
+  HvBeta beta;
+};
+
+// Launch helpers implemented in ed_matvec.hip.  Vectors are stored row by
+// row at a stride of ld >= num_dn doubles; the H.v writes zeros into y's
+// entries num_dn .. ld-1 of every row and never reads those of x.
+int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const HvEpilogue& epi,
+                  hipStream_t stream, int* num_partials);
+int matvec_num_partials(const ed_op* op, int64_t ld);
+// Whether an H.v on rows of this stride runs as the single fused pass, and
+// whether that pass forms a pending beta (HvEpilogue::beta).
+bool matvec_is_fused(const ed_op* op, int64_t ld);
+bool matvec_forms_beta(const ed_op* op, int64_t ld);
+// Row stride the library's own vectors use: num_dn rounded up to 16 doubles
+// (128-byte rows) where the two-pass sweep runs, num_dn otherwise.
+int64_t vector_ld(const ed_op* op);
+
 // Fully reorthogonalised steps (ed_reorth.hip): blocks of 64 * sub states.
 struct ReorthGrid {
   int blocks, sub;
@@ -319,10 +369,10 @@ bool reorth_available();                // the kernels' LDS is granted
 constexpr int kReorthMaxVectors = 256;  // basis vectors a step's kernels hold in LDS
 // Step j < kReorthMaxVectors from V_0..V_j (vectors of D doubles, contiguous
 // rows) into V_{j+1}: alpha_j, and |V_{j+1}|^2 as `blocks` partials in nout.
-// beta_j, s_j from the partials npart of the previous step (j > 0; may be
-// nout).  part, part2: kReorthMaxVectors * blocks doubles each.
+// prev: the previous step's beta where it is still a set of partials (which
+// may be nout's).  part, part2: kReorthMaxVectors * blocks doubles each.
 int launch_reorth_step(const ed_op* op, const double* V, int64_t D, int j, LzCoef c, double* part, double* part2,
-                       const double* npart, double* nout, hipStream_t s);
+                       const HvBeta& prev, double* nout, hipStream_t s);
 
 // Deterministic reductions (ed_lanczos.hip).
 int launch_reduce(const double* partial, int n, double* out, int op_kind, hipStream_t stream);

@@ -22,25 +22,15 @@
 
 #include <algorithm>
 #include <chrono>
+#include <type_traits>
 
 namespace ed {
 
-enum RedKind { RED_NORM0 = 0, RED_ALPHA = 1, RED_BETA = 2, RED_SUM_TO = 3, RED_SQRT_TO = 4 };
+enum RedKind { RED_NORM0 = 0, RED_ALPHA = 1, RED_SUM_TO = 3, RED_SQRT_TO = 4 };
 
 constexpr int kRedThreads = 1024;
 constexpr int kVecThreads = 256;
-
-// beta_{j+1} (lanczos_beta, with the breakdown and non-finite flags), then
-// scale_{j+1} = 1/beta_{j+1} and cprev_{j+1} = beta_{j+1} scale_j.
-__device__ __forceinline__ void finish_beta(LzCoef c, int j, double S) {
-  bool bad;
-  const double b = lanczos_beta(S, fabs(c.alpha[j]) + (j > 0 ? c.beta[j] : 0.0), c.misc[0] != 0.0, &bad);
-  if (bad) c.misc[3] = 1.0;
-  if (b == 0.0) c.misc[0] = 1.0;
-  c.beta[j + 1] = b;
-  c.scale[j + 1] = b > 0.0 ? 1.0 / b : 0.0;
-  c.cprev[j + 1] = b * c.scale[j];
-}
+typedef double v2d __attribute__((ext_vector_type(2)));
 
 __global__ __launch_bounds__(kRedThreads) void k_reduce(const double* __restrict__ partial, int n,
                                                         int kind, LzCoef c, int j, double* out) {
@@ -66,9 +56,6 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce(const double* __restrict
     }
     case RED_ALPHA:
       c.alpha[j] = c.scale[j] * S;
-      break;
-    case RED_BETA:
-      finish_beta(c, j, S);
       break;
     case RED_SUM_TO:
       *out = S;
@@ -189,8 +176,6 @@ __global__ __launch_bounds__(kVecThreads) void k_update(double* __restrict__ w, 
   }
 }
 
-typedef double v2d __attribute__((ext_vector_type(2)));
-
 // k_update on pairs of doubles (16-byte loads and stores; all pointers
 // 16-byte aligned, D2 = D / 2 with D even).  NT: u and w streamed with
 // nontemporal hints, for vectors far larger than the caches (the next step
@@ -276,36 +261,46 @@ __global__ __launch_bounds__(kVecThreads) void k_resid(const double* __restrict_
 
 // Block (c0, g) sums <V_i, w> for the kDotGroup vectors i of group g (then
 // g + gridDim.y, ...) over the chunks c = c0, c0 + gridDim.x, ... < nchunks,
-// into partial[i * gridDim.x + c0]: one read of w serves a group, and each
-// thread keeps kDotGroup + 1 loads in flight (a bounded grid, so a gated-off
-// launch costs one small dispatch).  gate (optional): skip the whole launch
-// unless *gate != 0 (partial reorthogonalisation decides on the device
-// whether a step needs it).
-constexpr int kMultidotRows = 32;    // blocks along the vector groups
-constexpr int kMultidotChunks = 32;  // blocks along the chunks
-constexpr int kDotGroup = 4;
-__global__ __launch_bounds__(kVecThreads) void k_multidot(const double* __restrict__ V, int64_t D,
-                                                          const double* __restrict__ w, int64_t chunk,
-                                                          double* partial, int nchunks, int nv, const int* gate) {
-  if (gate && *gate == 0) return;
+// into partial[i * gridDim.x + c0]: one read of w serves a group.  V2: pairs
+// of doubles (D and chunk even, every vector 16-byte aligned).  Eight vectors
+// by 16-byte loads keep 18 of them in flight per thread; with four vectors and
+// 8-byte loads the dots of an 853,776-state basis ran at 3.8 TB/s, half the
+// rate of the combination that follows.
+constexpr int kDotGroup = 8;
+// Blocks of a dots launch: two a CU, the register limit; the blocks along the
+// chunks follow from it, so that every CU gets the same share (a fixed 32
+// left 288 blocks on 256 CUs for a basis of 70 vectors).
+constexpr int kDotBlocks = 512;
+static dim3 dot_grid(int nchunks, int nv) {
+  const int ngroups = (nv + kDotGroup - 1) / kDotGroup;
+  return dim3((unsigned)std::min(nchunks, std::max(8, kDotBlocks / ngroups)), (unsigned)std::min(ngroups, 65535));
+}
+
+__device__ __forceinline__ double dot_step(v2d v, v2d w, double acc) { return fma(v.y, w.y, fma(v.x, w.x, acc)); }
+__device__ __forceinline__ double dot_step(double v, double w, double acc) { return fma(v, w, acc); }
+
+template <bool V2>
+__device__ void basis_dots(const double* __restrict__ V, int64_t D, const double* __restrict__ w, int64_t chunk,
+                           double* __restrict__ partial, int nchunks, int nv) {
+  using T = std::conditional_t<V2, v2d, double>;
+  constexpr int E = V2 ? 2 : 1;
   __shared__ double sh[kDotGroup][kVecThreads / 64];
   const int ngroups = (nv + kDotGroup - 1) / kDotGroup;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int g = blockIdx.y; g < ngroups; g += gridDim.y) {
     const int i0 = g * kDotGroup;
     const int nq = min(kDotGroup, nv - i0);
-    const double* v0 = V + (int64_t)i0 * D;
     double acc[kDotGroup];
 #pragma unroll
     for (int q = 0; q < kDotGroup; ++q) acc[q] = 0.0;
     for (int c = blockIdx.x; c < nchunks; c += gridDim.x) {
       const int64_t k0 = (int64_t)c * chunk, k1 = std::min<int64_t>(D, k0 + chunk);
 #pragma unroll 2
-      for (int64_t k = k0 + threadIdx.x; k < k1; k += blockDim.x) {
-        const double wk = w[k];
+      for (int64_t k = k0 / E + threadIdx.x; k < k1 / E; k += kVecThreads) {
+        const T wk = ((const T*)w)[k];
 #pragma unroll
-        for (int q = 0; q < kDotGroup; ++q)
-          if (q < nq) acc[q] += v0[(int64_t)q * D + k] * wk;
+        for (int q = 0; q < kDotGroup; ++q)  // past the last vector: read again, not stored
+          acc[q] = dot_step(((const T*)(V + (int64_t)(i0 + (q < nq ? q : 0)) * D))[k], wk, acc[q]);
       }
     }
 #pragma unroll
@@ -323,6 +318,13 @@ __global__ __launch_bounds__(kVecThreads) void k_multidot(const double* __restri
     }
     __syncthreads();  // sh is reused by the next group
   }
+}
+
+template <bool V2>
+__global__ __launch_bounds__(kVecThreads) void k_multidot(const double* __restrict__ V, int64_t D,
+                                                          const double* __restrict__ w, int64_t chunk,
+                                                          double* __restrict__ partial, int nchunks, int nv) {
+  basis_dots<V2>(V, D, w, chunk, partial, nchunks, nv);
 }
 
 // One classical Gram-Schmidt pass against the stored basis v_i = scale_i V_i:
@@ -356,15 +358,10 @@ __global__ __launch_bounds__(kVecThreads) void k_gs_update(const double* __restr
   if (threadIdx.x == 0) wpart[blockIdx.x] = t;
 }
 
-// beta_{j+1} from n partials of |w|^2 (finish_beta), unless *gate == 0.
-__global__ __launch_bounds__(kRedThreads) void k_beta_gated(const double* __restrict__ partial, int n, LzCoef c,
-                                                            int j, const int* gate) {
-  if (*gate == 0) return;
-  __shared__ double sh[kRedThreads / 64];
-  double v = 0.0;
-  for (int i = threadIdx.x; i < n; i += kRedThreads) v += partial[i];
-  const double S = block_sum(v, sh);
-  if (threadIdx.x == 0) finish_beta(c, j, S);
+// beta_{j+1} of a step whose H.v-formed beta is needed before the next step.
+__global__ __launch_bounds__(64) void k_form_beta(HvBeta b) {
+  double cp;
+  form_beta(b, true, &cp);
 }
 
 // w -= sum_i coef_i V_i   (sign = -1)   or   w = sum_i coef_i V_i (sign = 0)
@@ -520,7 +517,7 @@ void tri_lowest_vector(const double* a, const double* b, int m, double lam, std:
 // Partials: region A (npart doubles: the H.v sweep's and the Gram-Schmidt
 // dot products'), M + 2 coefficients, region B (npart2 doubles: the vector
 // updates' |w|^2), then with reorthogonalisation the orthogonality estimate
-// (3 (M + 2) doubles and two flags) and the three-launch step's partials (two
+// (3 (M + 2) doubles and four flags) and the three-launch step's partials (two
 // sets of dots and |w|^2).
 struct LzLayout {
   int64_t coef_off, part_off, part2_off, pro_off, dots_off, vec_off, total;
@@ -552,7 +549,7 @@ static LzLayout lz_layout(const ed_op* op, int M, int reorth, int want_vector, i
   L.part_off = align256(L.coef_off + sizeof(double) * (4 * (int64_t)M + 4 + 16));
   L.part2_off = align256(L.part_off + sizeof(double) * (int64_t)(L.npart + M + 2));
   L.pro_off = align256(L.part2_off + sizeof(double) * (int64_t)L.npart2);
-  const int64_t pro_bytes = reorth ? (int64_t)sizeof(double) * (3 * ((int64_t)M + 2) + 1) : 0;
+  const int64_t pro_bytes = reorth ? (int64_t)sizeof(double) * (3 * ((int64_t)M + 2) + 2) : 0;
   L.dots_off = align256(L.pro_off + pro_bytes);
   const int64_t rb = reorth_grid(L.D).blocks;
   L.ndots = kReorthMaxVectors * rb;
@@ -625,15 +622,35 @@ struct EventTimer {
   }
 };
 
+// A beta still held as partials, formed now (before the coefficients are read).
+static int flush_beta(HvBeta& pend, hipStream_t s) {
+  if (pend.j < 0) return ED_OK;
+  hipLaunchKernelGGL(k_form_beta, dim3(1), dim3(64), 0, s, pend);
+  pend.j = -1;
+  ED_HIP(hipGetLastError());
+  return ED_OK;
+}
+
+// Hands a pending beta to the H.v described by e, where its kernel forms it.
+static int pass_beta(const ed_op* op, const LzLayout& L, HvBeta& pend, HvEpilogue& e, hipStream_t s) {
+  if (!matvec_forms_beta(op, L.ld)) return flush_beta(pend, s);
+  e.beta = pend;
+  pend.j = -1;
+  return ED_OK;
+}
+
 // One step of the three-vector recurrence: H.v with the epilogue (partials
 // of <w, u_j> into part), the update with alpha_j formed in it (|w|^2
 // partials into part2), beta_{j+1}.  Without reduce (the eigenvector's
 // second pass) alpha_j and beta_{j+1} are already known, and the H.v's
 // epilogue applies alpha_j and accumulates psi itself: no update pass.
+// pend: the beta that the previous step left as partials (formed here, or by
+// the H.v's own blocks), and on return this step's.
 static int run_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, double* part2, double* u_prev,
                     double* u_cur, double* w, int j, hipStream_t s, EventTimer* tm, double* psi, double yj,
-                    bool reduce) {
+                    bool reduce, HvBeta& pend) {
   HvEpilogue e;
+  ED_TRY(pass_beta(op, L, pend, e, s));
   e.xprev = j > 0 ? u_prev : nullptr;
   e.sx = c.scale + j;
   e.cprev = c.cprev + j;
@@ -656,7 +673,7 @@ static int run_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, double
   if (reduce) {
     const int ub = update_blocks(L.D);
     launch_update(ub, s, w, u_cur, L.D, c.alpha + j, c.scale + j, psi, yj, part2, part, np);
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part2, ub, (int)RED_BETA, c, j, nullptr);
+    pend = HvBeta{part2, {ub, ub}, nullptr, c, j};
   }
   ED_HIP(hipGetLastError());
   return ED_OK;
@@ -669,13 +686,12 @@ struct ReorthCtx {
   double* coefs;
   double* part2;  // region B
   int64_t chunks, chunk;
-  int gx;         // k_multidot blocks along the chunks (dot partials per vector)
-  // three-launch steps (ed_reorth.hip): their partials, and the step whose
-  // beta is still only a set of partials (-1: none)
+  // three-launch steps (ed_reorth.hip) and their partials
   double *dots, *dots2, *norms;
   int blocks;
   bool three = false;
-  int pending = -1;
+  HvBeta pend;  // the last step's beta while it is a set of partials
+  bool pairs;   // the vectors can be read as pairs of doubles
 };
 
 // Sectors up to this many states take the three-launch step, whose H.v deals
@@ -701,8 +717,8 @@ static ReorthCtx reorth_ctx(const ed_op* op, char* base, const LzLayout& L, doub
   r.coefs = part + L.npart;
   r.part2 = reinterpret_cast<double*>(base + L.part2_off);
   r.chunks = std::min<int64_t>((L.D + 4095) / 4096, 256);
-  r.chunk = (L.D + r.chunks - 1) / r.chunks;
-  r.gx = (int)std::min<int64_t>(r.chunks, kMultidotChunks);
+  r.chunk = ((L.D + r.chunks - 1) / r.chunks + 1) / 2 * 2;
+  r.pairs = L.D % 2 == 0;
   return r;
 }
 
@@ -724,11 +740,11 @@ static int reorth_start(const LzLayout& L, LzCoef c, double* part, const ReorthC
 // with w_{k,k} = 1 and w_{k+1,k} = eps.  When max_k |w_{j+1,k}| passes
 // sqrt(eps) the new vector is orthogonalised against all previous ones (and
 // so is the next one), and its row is reset to eps.  Rows live in om[3][M+2]
-// (row r at (r % 3)); flags[0] = orthogonalise this step, flags[1] = the
-// next step must too.
+// (row r at (r % 3)); flags[2 (j & 1)] = step j is orthogonalised, flags[2 (j &
+// 1) + 1] = the next step must be too.
 struct ProState {
   double* om;   // [3][M + 2]
-  int* flags;   // [2]
+  int* flags;   // [4]
   int M;
 };
 
@@ -739,64 +755,69 @@ __global__ __launch_bounds__(256) void k_pro_init(ProState p) {
   for (int i = threadIdx.x; i < 3 * (p.M + 2); i += blockDim.x) p.om[i] = 0.0;
   if (threadIdx.x == 0) {
     p.om[0] = 1.0;  // w_{0,0}
-    p.flags[0] = 0;
-    p.flags[1] = 0;
+    for (int i = 0; i < 4; ++i) p.flags[i] = 0;
   }
 }
 
-// bt = |w| before orthogonalisation, summed here from the np partials of
-// |w|^2 that the vector update left.  On a step that needs no Gram-Schmidt
-// this |w| is final: beta_{j+1} is set here (finish_beta), and the gated
-// kernels after it do nothing.  One block of 256 threads.
-__global__ __launch_bounds__(256) void k_pro_omega(ProState p, LzCoef c, int j, const double* __restrict__ wpart,
-                                                   int np) {
+// Step j's estimate, and where it asks for it the dots <V_i, w>, i <= j (see
+// basis_dots).  bt = |w| before orthogonalisation is summed from the np
+// partials of |w|^2 that the vector update left.  Every block forms the same
+// estimate from what earlier launches wrote and block (0, 0) records it, so the
+// decision costs no launch of its own; a step that needs no pass ends here.
+template <bool V2>
+__global__ __launch_bounds__(kVecThreads) void k_pro_dots(ProState p, LzCoef c, int j, const double* __restrict__ wpart,
+                                                          int np, const double* __restrict__ V, int64_t D,
+                                                          const double* __restrict__ w, int64_t chunk,
+                                                          double* __restrict__ partial, int nchunks) {
   const double* __restrict__ alpha = c.alpha;
   const double* __restrict__ beta = c.beta;
-  __shared__ double sh[256 / 64];
-  __shared__ int decide;
-  __shared__ double bt_sh;
+  __shared__ double sh[2 * (kVecThreads / 64)];
   const int W = p.M + 2;
   const double* cur = p.om + (int64_t)(j % 3) * W;
   const double* prev = p.om + (int64_t)((j + 2) % 3) * W;
   double* nxt = p.om + (int64_t)((j + 1) % 3) * W;
+  const int force = p.flags[2 * ((j + 1) & 1) + 1];
+  const bool lead = blockIdx.x == 0 && blockIdx.y == 0;
   const double eps = 2.220446049250313e-16;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   double w2 = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) w2 += wpart[i];
-  w2 = block_sum(w2, sh);
-  if (threadIdx.x == 0) bt_sh = sqrt(fmax(w2, 0.0));
+  for (int i = threadIdx.x; i < np; i += kVecThreads) w2 += wpart[i];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) w2 += __shfl_down(w2, off, 64);
+  if (lane == 0) sh[wave] = w2;
   __syncthreads();
-  const double bt = bt_sh;
+  w2 = 0.0;
+  for (int v = 0; v < kVecThreads / 64; ++v) w2 += sh[v];
+  const double bt = sqrt(fmax(w2, 0.0));
   double mx = 0.0;
   if (bt > 0.0) {
-    for (int k = threadIdx.x; k < j; k += blockDim.x) {
+    for (int k = threadIdx.x; k < j; k += kVecThreads) {
       double t = beta[k + 1] * cur[k + 1] + (alpha[k] - alpha[j]) * cur[k] - beta[j] * prev[k];
       if (k > 0) t += beta[k] * cur[k - 1];
       t += (t >= 0.0 ? 1.0 : -1.0) * eps * (beta[k + 1] + bt) * 0.3;
       const double o = t / bt;
-      nxt[k] = o;
+      if (lead) nxt[k] = o;
       mx = fmax(mx, fabs(o));
     }
   }
-  // block maximum
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_down(mx, off, 64));
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = mx;
+  if (lane == 0) sh[kVecThreads / 64 + wave] = mx;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double m = 0.0;
-    for (int w = 0; w < 4; ++w) m = fmax(m, sh[w]);
-    const int force = p.flags[1];
-    const int re = bt > 0.0 && (m > 1.4901161193847656e-08 || force);
-    p.flags[0] = re;
-    p.flags[1] = re && !force;
-    decide = re;
-    nxt[j] = eps;
-    nxt[j + 1] = 1.0;
-    if (!re) finish_beta(c, j, w2);
+  mx = 0.0;
+  for (int v = 0; v < kVecThreads / 64; ++v) mx = fmax(mx, sh[kVecThreads / 64 + v]);
+  const bool re = bt > 0.0 && (mx > 1.4901161193847656e-08 || force);
+  if (lead) {
+    if (threadIdx.x == 0) {
+      p.flags[2 * (j & 1)] = re;
+      p.flags[2 * (j & 1) + 1] = re && !force;
+      nxt[j] = eps;
+      nxt[j + 1] = 1.0;
+    }
+    if (re)
+      for (int k = threadIdx.x; k < j; k += kVecThreads) nxt[k] = eps;  // the thread that wrote nxt[k]
   }
-  __syncthreads();
-  if (decide)
-    for (int k = threadIdx.x; k < j; k += blockDim.x) nxt[k] = eps;
+  if (re) basis_dots<V2>(V, D, w, chunk, partial, nchunks, j + 1);
 }
 
 static int pro_init(ProState& pro, char* base, const LzLayout& L, hipStream_t s) {
@@ -808,16 +829,6 @@ static int pro_init(ProState& pro, char* base, const LzLayout& L, hipStream_t s)
   return ED_OK;
 }
 
-// beta_{j+1} of a three-launch step whose next step has not formed it.
-static int reorth_finish(LzCoef c, ReorthCtx& r, hipStream_t s) {
-  if (r.pending < 0) return ED_OK;
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, r.norms, r.blocks, (int)RED_BETA, c, r.pending,
-                     nullptr);
-  r.pending = -1;
-  ED_HIP(hipGetLastError());
-  return ED_OK;
-}
-
 // Step j, with the basis kept unnormalised (v_i = scale_i V_i, as the
 // three-vector recurrence keeps its vectors): W = V_{j+1} = s_j H V_j -
 // beta_j s_{j-1} V_{j-1}; alpha_j = s_j <W, V_j> (formed in the update);
@@ -825,19 +836,19 @@ static int reorth_finish(LzCoef c, ReorthCtx& r, hipStream_t s) {
 // every step, or, with a ProState, one pass where the orthogonality estimate
 // asks for it (the basis is then semi-orthogonal, |<v_i, v_k>| <= sqrt(eps),
 // and W's components along it are O(sqrt(eps) |W|), so one pass leaves
-// O(eps)); beta_{j+1} = |W|, scale_{j+1} = 1/beta_{j+1}.  Launches per step:
-// the two H.v sweeps, the update, then with a ProState the estimate (which
-// sets beta_{j+1} when no pass is due) and three gated kernels (dots,
-// combination, beta); without, two passes of (dots, combination) and beta.
+// O(eps)); beta_{j+1} = |W|, scale_{j+1} = 1/beta_{j+1}.  beta_{j+1}
+// stays a set of partials until the next step's H.v (or the host) needs it.
+// Launches per step: the H.v, the update, then with a ProState the estimate
+// with the dots and the gated combination; without, two passes of (dots,
+// combination).
 static int reorth_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, ReorthCtx& r, int j,
                        hipStream_t s, EventTimer* tm, const ProState* pro = nullptr) {
   const int64_t D = L.D;
   if (r.three && j < kReorthMaxVectors) {
-    ED_TRY(launch_reorth_step(op, r.V, D, j, c, r.dots, r.dots2, r.norms, r.norms, s));
-    r.pending = j;
+    ED_TRY(launch_reorth_step(op, r.V, D, j, c, r.dots, r.dots2, r.pend, r.norms, s));
+    r.pend = HvBeta{r.norms, {r.blocks, r.blocks}, nullptr, c, j};
     return ED_OK;
   }
-  ED_TRY(reorth_finish(c, r, s));
   const int vb = vec_blocks(D);
   double* vj = r.V + (int64_t)j * D;
   double* w = r.V + (int64_t)(j + 1) * D;
@@ -846,6 +857,7 @@ static int reorth_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, Reo
   e.sx = c.scale + j;
   e.cprev = c.cprev + j;
   e.partial = part;
+  ED_TRY(pass_beta(op, L, r.pend, e, s));
   if (tm && tm->on) {
     hipEvent_t a = tm->next();
     if (a) ED_HIP(hipEventRecord(a, s));
@@ -858,23 +870,21 @@ static int reorth_step(ed_op* op, const LzLayout& L, LzCoef c, double* part, Reo
   }
   const int ub = update_blocks(D);
   launch_update(ub, s, w, vj, D, c.alpha + j, c.scale + j, nullptr, 0.0, r.part2, part, np);
-  const int* gate = nullptr;
-  if (pro) {
-    hipLaunchKernelGGL(k_pro_omega, dim3(1), dim3(256), 0, s, *pro, c, j, r.part2, ub);
-    gate = pro->flags;
-  }
   const int gb = std::min(vb, kAxpyBlocks);
+  const int* gate = pro ? pro->flags + 2 * (j & 1) : nullptr;
+  const dim3 dg = dot_grid((int)r.chunks, j + 1);
   for (int pass = 0; pass < (pro ? 1 : 2); ++pass) {
-    hipLaunchKernelGGL(k_multidot,
-                       dim3((unsigned)r.gx, (unsigned)std::min((j + kDotGroup) / kDotGroup, kMultidotRows)),
-                       dim3(kVecThreads), 0, s, r.V, D, w, r.chunk, part, (int)r.chunks, j + 1, gate);
+    if (pro)
+      hipLaunchKernelGGL(r.pairs ? k_pro_dots<true> : k_pro_dots<false>, dg, dim3(kVecThreads), 0, s, *pro, c, j,
+                         r.part2, ub, r.V, D, w, r.chunk, part, (int)r.chunks);
+    else
+      hipLaunchKernelGGL(r.pairs ? k_multidot<true> : k_multidot<false>, dg, dim3(kVecThreads), 0, s, r.V, D, w,
+                         r.chunk, part, (int)r.chunks, j + 1);
     hipLaunchKernelGGL(k_gs_update, dim3((unsigned)gb), dim3(kVecThreads), sizeof(double) * (j + 1), s, r.V, j + 1,
-                       D, part, r.gx, c.scale, w, r.part2, gate);
+                       D, part, (int)dg.x, c.scale, w, r.part2, gate);
   }
-  if (pro)
-    hipLaunchKernelGGL(k_beta_gated, dim3(1), dim3(kRedThreads), 0, s, r.part2, gb, c, j, gate);
-  else
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, r.part2, gb, (int)RED_BETA, c, j, nullptr);
+  // |w|^2 from the update's partials, or the pass's where one ran
+  r.pend = HvBeta{r.part2, {pro ? ub : gb, gb}, gate, c, j};
   ED_HIP(hipGetLastError());
   return ED_OK;
 }
@@ -965,8 +975,9 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
     ED_HIP(hipGetLastError());
     int ip = 2, ic = 0, iw = 1;  // u_prev, u_cur, w
     int steps = 0;
+    HvBeta pend;
     for (int j = 0; j < M; ++j) {
-      ED_TRY(run_step(op, L, c, part, part2, u[ip], u[ic], u[iw], j, s, &tm, nullptr, 0.0, true));
+      ED_TRY(run_step(op, L, c, part, part2, u[ip], u[ic], u[iw], j, s, &tm, nullptr, 0.0, true, pend));
       steps = j + 1;
       const int old_p = ip;
       ip = ic;
@@ -975,6 +986,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
       const bool last = (j + 1 == M);
       const bool due = !cfg->fixed_iter && steps >= cfg->min_iter && (steps % cfg->check_every == 0);
       if (due || last) {
+        ED_TRY(flush_beta(pend, s));
         ED_TRY(check(steps));
         if (breakdown || ritz <= cfg->tol) {
           converged = true;
@@ -992,7 +1004,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
       iw = 1;
       for (int j = 0; j < m; ++j) {
         if (j + 1 < m) {
-          ED_TRY(run_step(op, L, c, part, part2, u[ip], u[ic], u[iw], j, s, nullptr, psi, y[j], false));
+          ED_TRY(run_step(op, L, c, part, part2, u[ip], u[ic], u[iw], j, s, nullptr, psi, y[j], false, pend));
         } else {
           // last vector: accumulate only (w is scratch)
           launch_update(vb, s, u[iw], u[ic], D, c.misc + 2, c.scale + j, psi, y[j], nullptr);
@@ -1019,7 +1031,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
       const bool last = (j + 1 == M);
       const bool due = !cfg->fixed_iter && steps >= cfg->min_iter && (steps % cfg->check_every == 0);
       if (due || last) {
-        ED_TRY(reorth_finish(c, rc, s));
+        ED_TRY(flush_beta(rc.pend, s));
         ED_TRY(check(steps));
         if (breakdown || ritz <= cfg->tol) {
           converged = true;
@@ -1108,7 +1120,7 @@ extern "C" int ed_lanczos_coeffs(ed_op* op, const double* v0_dev, int32_t nsteps
     ProState pro{nullptr, nullptr, M};
     if (reorth == 2) ED_TRY(pro_init(pro, base, L, s));
     for (int j = 0; j < M; ++j) ED_TRY(reorth_step(op, L, c, part, rc, j, s, nullptr, reorth == 2 ? &pro : nullptr));
-    ED_TRY(reorth_finish(c, rc, s));
+    ED_TRY(flush_beta(rc.pend, s));
     // basis vector j is rc.V + j D, scaled by scale_j
     if (basis_dev) launch_compact(L, s, basis_dev, rc.V, D, M, c.scale, 0);
   } else {
@@ -1117,15 +1129,18 @@ extern "C" int ed_lanczos_coeffs(ed_op* op, const double* v0_dev, int32_t nsteps
     hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, 0, nullptr);
     ED_HIP(hipGetLastError());
     int ip = 2, ic = 0, iw = 1;
+    HvBeta pend;
     for (int j = 0; j < M; ++j) {
+      if (basis_dev) ED_TRY(flush_beta(pend, s));  // the copy scales by 1/beta_j
       if (basis_dev) launch_compact(L, s, basis_dev + (int64_t)j * L.nu * L.nd, u[ic], 0, 1, c.scale + j, 0);
       ED_TRY(run_step(op, L, c, part, reinterpret_cast<double*>(base + L.part2_off), u[ip], u[ic], u[iw], j, s,
-                      nullptr, nullptr, 0.0, true));
+                      nullptr, nullptr, 0.0, true, pend));
       const int old_p = ip;
       ip = ic;
       ic = iw;
       iw = old_p;
     }
+    ED_TRY(flush_beta(pend, s));
   }
   std::vector<double> ha(M), hb(M + 1);
   double flag[4];

@@ -651,7 +651,7 @@ template <int RB, bool UNI, bool LZ>
 __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __restrict__ x, double* __restrict__ y,
                                                   HvEpilogue e, int nrg, int per_xcd, int64_t vstride) {
   extern __shared__ double rows[];  // [RB][nd]
-  __shared__ double red[16];
+  __shared__ double red[32];
   const int rg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
   if (rg >= nrg) {  // the whole block
     if (LZ && e.partial && threadIdx.x == 0) e.partial[blockIdx.x] = 0.0;
@@ -672,10 +672,16 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
   }
   zero_row_pads(y, r0, R, nd, ld);
   const double t = UNI ? a.hop[0] : 1.0;
-  const double sx = LZ && e.sx ? *e.sx : 1.0;
-  const double cp = LZ && e.cprev ? *e.cprev : 0.0;
+  double sx = 1.0, cp = 0.0, share = 0.0;
+  const bool forms = LZ && e.beta.j >= 0;
+  if (forms) {
+    // requested here, summed after the first chunk's up hops are in flight
+    share = beta_share(e.beta, threadIdx.x, nt);
+  } else if (LZ) {
+    if (e.sx) sx = *e.sx;
+    if (e.cprev) cp = *e.cprev;
+  }
   const double cs = LZ && e.cself ? *e.cself : 0.0;
-  const double ps = LZ ? e.psi_y * sx : 0.0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   constexpr int UP = RB == 4 ? 4 : 8;  // up hops of a row whose loads are in flight together
@@ -714,8 +720,20 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
 #pragma unroll
         for (int q = 0; q < UP; ++q) acc[r] = fma(v[r][q], g[r][q], acc[r]);
     }
-    if (first) __syncthreads();  // every wave passes here once
-    first = false;
+    if (first) {  // every wave passes here once
+      if (forms) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) share += __shfl_xor(share, off, 64);
+        if (lane == 0) red[wave] = share;
+      }
+      __syncthreads();
+      if (forms) {
+        double S = 0.0;
+        for (int w = 0; w < nt / 64; ++w) S += red[w];
+        sx = beta_scale(e.beta, S, blockIdx.x == 0 && threadIdx.x == 0, &cp);
+      }
+      first = false;
+    }
     const int w1 = a.dn_w - 1;
     uint32_t en[kTileDn];
     double vl[kTileDn];
@@ -756,7 +774,7 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
           double v = sx * (h - cs * xo);
           if (e.xprev) v -= cp * e.xprev[k];
           y[k] = v;
-          if (e.psi) e.psi[k] += ps * xo;
+          if (e.psi) e.psi[k] += e.psi_y * sx * xo;
           dot += v * xo;
         } else {
           y[k] = h;
@@ -767,11 +785,11 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
   if (LZ && e.partial) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) dot += __shfl_down(dot, off, 64);
-    if (lane == 0) red[wave] = dot;
+    if (lane == 0) red[16 + wave] = dot;
     __syncthreads();
     if (threadIdx.x == 0) {
       double s = 0.0;
-      for (int w = 0; w < nt / 64; ++w) s += red[w];
+      for (int w = 0; w < nt / 64; ++w) s += red[16 + w];
       e.partial[blockIdx.x] = s;
     }
   }
@@ -1544,9 +1562,9 @@ static TilePlan plan_tile(const ed_op* op) {
   p.threads = (int)waves * 64;
   p.rb = 4;
   for (; p.rb > 1; p.rb /= 2)
-    if (p.rb * op->num_dn * sizeof(double) <= kTileLds - 128 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
+    if (p.rb * op->num_dn * sizeof(double) <= kTileLds - 256 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
   p.lds_bytes = p.rb * op->num_dn * sizeof(double);
-  if (p.lds_bytes > kTileLds - 128) return p;  // the kernel has static LDS of its own
+  if (p.lds_bytes > kTileLds - 256) return p;  // the kernel has static LDS of its own
   p.nrg = (int)((op->num_up + p.rb - 1) / p.rb);
   p.per_xcd = (p.nrg + 7) / 8;
   p.ok = true;
@@ -1728,6 +1746,8 @@ int matvec_num_partials(const ed_op* op, int64_t ld) {
 
 bool matvec_is_fused(const ed_op* op, int64_t ld) { return !plan_two_pass(op, ld).ok; }
 
+bool matvec_forms_beta(const ed_op* op, int64_t ld) { return matvec_is_fused(op, ld) && plan_tile(op).ok; }
+
 int64_t vector_ld(const ed_op* op) {
   const int64_t nd = op->num_dn;
   const int64_t ld = (nd + 15) / 16 * 16;
@@ -1779,7 +1799,7 @@ int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const
                   int* num_partials) {
   const TwoPassPlan p = plan_two_pass(op, ld);
   if (p.ok) return launch_two_pass(op, p, x, y, ld, epi, s, num_partials);
-  const bool lz = epi.xprev || epi.sx || epi.cprev || epi.partial || epi.cself || epi.psi;
+  const bool lz = epi.xprev || epi.sx || epi.cprev || epi.partial || epi.cself || epi.psi || epi.beta.j >= 0;
   const TilePlan tp = plan_tile(op);
   if (tp.ok) {
     if (num_partials) *num_partials = tp.grid();

@@ -112,12 +112,11 @@ __device__ __forceinline__ double group_sum(double v, const ReorthLds& L, int lg
   return s;
 }
 
-// S subtiles of 64 states per block; npart: nn partials of |V_j|^2 (j > 0).
+// S subtiles of 64 states per block.
 __global__ __launch_bounds__(kReorthThreads) void k_reorth_hv(HvArgs a, int hops_up, int hops_dn,
                                                               const double* __restrict__ V, int D, int j, LzCoef c,
-                                                              const double* __restrict__ npart, int nn,
-                                                              double* __restrict__ w, double* __restrict__ part, int S,
-                                                              int lg) {
+                                                              HvBeta prev, double* __restrict__ w,
+                                                              double* __restrict__ part, int S, int lg) {
   extern __shared__ double tile[];
   __shared__ double red[kReorthThreads];
   __shared__ double tot[64];
@@ -127,24 +126,8 @@ __global__ __launch_bounds__(kReorthThreads) void k_reorth_hv(HvArgs a, int hops
   int k = (int)blockIdx.x * S * 64 + lane;
   double v[kPre];
   tile_request(v, V, D, k, wave, j);
-  double sx;
-  if (j > 0) {
-    double n2 = 0.0;
-    for (int i = lane; i < nn; i += 64) n2 += npart[i];
-    for (int off = 32; off > 0; off >>= 1) n2 += __shfl_xor(n2, off, 64);
-    bool bad;
-    const double b = lanczos_beta(n2, fabs(c.alpha[j - 1]) + (j > 1 ? c.beta[j - 1] : 0.0), c.scale[j - 1] == 0.0, &bad);
-    sx = b > 0.0 ? 1.0 / b : 0.0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      if (bad) c.misc[3] = 1.0;
-      if (b == 0.0) c.misc[0] = 1.0;
-      c.beta[j] = b;
-      c.scale[j] = sx;
-      c.cprev[j] = b * c.scale[j - 1];
-    }
-  } else {
-    sx = c.scale[0];
-  }
+  double cp;
+  const double sx = prev.j >= 0 ? form_beta(prev, blockIdx.x == 0, &cp) : c.scale[j];
   const double* __restrict__ u = V + (uint32_t)(j * D);
   const uint32_t nd = (uint32_t)a.num_dn;
   double acc = 0.0;
@@ -275,14 +258,14 @@ bool reorth_available() {
 }
 
 int launch_reorth_step(const ed_op* op, const double* V, int64_t D, int j, LzCoef c, double* part, double* part2,
-                       const double* npart, double* nout, hipStream_t s) {
+                       const HvBeta& prev, double* nout, hipStream_t s) {
   const ReorthGrid g = reorth_grid(D);
   double* w = const_cast<double*>(V) + (int64_t)(j + 1) * D;
   const dim3 grid((unsigned)g.blocks), block(kReorthThreads);
   const int lg = j < 64 ? 6 : (j < 128 ? 7 : 8);
   const size_t lds = sizeof(double) * 64 * (size_t)(j + 1);
   hipLaunchKernelGGL(k_reorth_hv, grid, block, lds, s, make_hv_args(op), op->max_hops_up, op->max_hops_dn, V, (int)D, j, c,
-                     npart, g.blocks, w, part, g.sub, lg);
+                     prev, w, part, g.sub, lg);
   hipLaunchKernelGGL(k_reorth_pass, grid, block, lds, s, V, (int)D, j, c, part, w, part2, g.sub, lg, 1);
   hipLaunchKernelGGL(k_reorth_pass, grid, block, lds, s, V, (int)D, j, c, part2, w, nout, g.sub, lg, 0);
   ED_HIP(hipGetLastError());
