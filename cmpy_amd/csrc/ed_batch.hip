@@ -111,6 +111,16 @@ struct Config {
 using lds_f64 = __attribute__((address_space(3))) double;
 using lds_u32 = __attribute__((address_space(3))) uint32_t;
 using lds_i32 = __attribute__((address_space(3))) int32_t;
+// Pointers to memory that reach a function of its own (not inlined) keep
+// their address space: through plain pointers every access there is a flat
+// one, which counts with the LDS accesses too, so that a wait for an LDS read
+// or a barrier also waited for the vector stores before it (400 states held on
+// chip: 3.5 us a step without, 6.6 with).
+using glb_f64 = __attribute__((address_space(1))) double;
+using glb_u32 = __attribute__((address_space(1))) uint32_t;
+using glb_i32 = __attribute__((address_space(1))) int32_t;
+__device__ __forceinline__ const glb_f64* glb(const double* p) { return (const glb_f64*)p; }
+__device__ __forceinline__ glb_f64* glb(double* p) { return (glb_f64*)p; }
 
 constexpr int kLdsChunks = 64;  // 64-state chunks of the dn sector the LDS cache covers
 // LDS sizes: staged rows (solve kernel: one row of at most 256 columns per
@@ -118,7 +128,9 @@ constexpr int kLdsChunks = 64;  // 64-state chunks of the dn sector the LDS cach
 // columns per wave or two buffers of R rows of at most 64 * 16 / R columns),
 // cached dn and up hop slots (12 bytes each) and up-state counts
 constexpr int kLdsRows = 2048;
-constexpr int kLdsRowsSolve = 4096;
+// (solve kernel: also the current vector of a sector held on chip, 4,900
+// states at 7 bath sites)
+constexpr int kLdsRowsSolve = 4904;
 constexpr int kLdsDnSolve = 4096;   // solve kernel: 48 KiB
 constexpr int kLdsUpSolve = 4096;   // 48 KiB
 constexpr int kLdsUpRowsSolve = 4096;
@@ -155,10 +167,58 @@ struct BlockLds {
   int ddn_cap = 0;
 };
 
+// Wave-uniform copy of a value every lane holds or reads from the same address.
+__device__ __forceinline__ int rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Sum over a wavefront, the same value on every lane: within rows of 16 lanes
+// by data-parallel-primitive moves, then the four rows' sums in order.
+#ifdef __HIP_DEVICE_COMPILE__
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+#endif
+__device__ __forceinline__ double readlane_d(double v, int l) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  v += dpp_move<0xB1>(v);   // lane ^ 1
+  v += dpp_move<0x4E>(v);   // lane ^ 2
+  v += dpp_move<0x141>(v);  // 7 - lane within 8: the other four
+  v += dpp_move<0x140>(v);  // 15 - lane within 16: the other eight
+#else
+  for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+#endif
+  return ((readlane_d(v, 0) + readlane_d(v, 16)) + readlane_d(v, 32)) + readlane_d(v, 48);
+}
+
+// The rank of a wavefront's first lane where hit holds, none if it holds
+// nowhere.
+__device__ __forceinline__ int first_lane(bool hit, int rank, int none) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const uint64_t bits = __ballot(hit);
+  return bits ? (rank & ~63) + __builtin_ctzll(bits) : none;
+#else
+  int v = hit ? rank : none;
+  for (int off = 32; off > 0; off >>= 1) {
+    const int w = __shfl_xor(v, off, 64);
+    v = w < v ? w : v;
+  }
+  return v;
+#endif
+}
+
 template <bool BLOCK>
 struct Group {
   int rank, size;
-  double* red;  // LDS: 2 * 16 doubles (block mode)
+  lds_f64* red;  // 2 * 16 doubles (block mode)
   BlockLds lds{};
   bool has_lds = false;
   bool wave_rows = false;  // block mode: wave-private row staging where the dn sector fits
@@ -172,15 +232,30 @@ struct Group {
   }
   // Sum over the group, the same value on every member, fixed order.
   __device__ double sum(double v) const {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (!BLOCK) return v;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) red[wid] = v;
+    if (!BLOCK) return wave_sum(v);
+    const double s = sum_half<0>(v, rfl(size >> 6));  // (a member read through a reference counts as divergent)
+    __syncthreads();
+    return s;
+  }
+  // Block mode: the sum over the first nw wavefronts (the others hold zeros)
+  // through one half of red, with one barrier.  The same half may be used
+  // again after another barrier (the other half's sum).
+  template <int HALF>
+  __device__ double sum_half(double v, int nw) const {
+    lds_f64* const r = red + 16 * HALF;
+    if (rfl(rank >> 6) < nw) {
+      v = wave_sum(v);
+      if ((rank & 63) == 0) r[rank >> 6] = v;
+    }
     __syncthreads();
     double s = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += red[w];
-    __syncthreads();
+    for (int w0 = 0; w0 < nw; w0 += 8) {  // eight reads in flight
+      double x[8];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) x[w] = r[w0 + w < nw ? w0 + w : 0];
+#pragma unroll
+      for (int w = 0; w < 8; ++w) s += w0 + w < nw ? x[w] : 0.0;
+    }
     return s;
   }
   __device__ double max(double v) const {
@@ -191,7 +266,8 @@ struct Group {
     if (lane == 0) red[wid] = v;
     __syncthreads();
     double s = red[0];
-    for (int w = 1; w < (int)(blockDim.x >> 6); ++w) s = fmax(s, red[w]);
+    const int nw = rfl(size >> 6);
+    for (int w = 1; w < nw; ++w) s = fmax(s, red[w]);
     __syncthreads();
     return s;
   }
@@ -205,11 +281,11 @@ struct Group {
 // keeps the solver's live register set small).
 // ---------------------------------------------------------------------------
 struct SpinList {
-  const uint32_t* st;
-  const double* dg;
-  const int32_t* cnt;
-  const int32_t* tgt;  // [n][kMaxBath] hop target | bond << 16 | sign << 31
-  const double* val;   // [n][kMaxBath] hop values sign * V_k
+  const glb_u32* st;
+  const glb_f64* dg;
+  const glb_i32* cnt;
+  const glb_i32* tgt;  // [n][kMaxBath] hop target | bond << 16 | sign << 31
+  const glb_f64* val;  // [n][kMaxBath] hop values sign * V_k
   int32_t n;
 };
 
@@ -251,7 +327,10 @@ struct SlotRef {
   // continued-fraction coefficients: 0 ap, 1 bp, 2 am, 3 bm
   __device__ double* cfc(int i) const { return (double*)(coef_base() + 4 * coef_bytes(miter) + i * coef_bytes(csteps)); }
   __device__ double* scal() const { return (double*)(coef_base() + 4 * coef_bytes(miter) + 4 * coef_bytes(csteps)); }
-  __device__ SpinList list(int l, int32_t n) const { return SpinList{st(l), dg(l), cnt(l), tgt(l), val(l), n}; }
+  __device__ SpinList list(int l, int32_t n) const { 
+    return SpinList{(const glb_u32*)st(l), glb((const double*)dg(l)), (const glb_i32*)cnt(l), (const glb_i32*)tgt(l),
+                    glb((const double*)val(l)), n};
+  }
 };
 
 __device__ __forceinline__ uint64_t mix64(uint64_t z) {
@@ -362,10 +441,8 @@ __device__ __forceinline__ bool up_cached(const Group<true>& g, const SpinList& 
          g.lds.umeta[3] == (int32_t)(uint32_t)(a >> 32);
 }
 
-// Wave-uniform copy of a value every lane reads from the same address (the
-// spin lists are written by this kernel, so they are read with vector loads,
-// not through the scalar cache).
-__device__ __forceinline__ int rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// rfl of a double (the spin lists are written by this kernel, so they are read
+// with vector loads, not through the scalar cache).
 __device__ __forceinline__ double rfl_d(double v) {
   const uint64_t b = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
@@ -374,13 +451,6 @@ __device__ __forceinline__ double rfl_d(double v) {
 }
 
 constexpr int kUpPre = 6;  // up hops whose loads start before the staging barrier
-
-__device__ __forceinline__ double readlane_d(double v, int l) {
-  const uint64_t b = __builtin_bit_cast(uint64_t, v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, l);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), l);
-  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
-}
 
 
 // Block-mode sweep 1 of lanczos_step with staged rows, for dn sectors of at
@@ -397,12 +467,12 @@ __device__ __forceinline__ double readlane_d(double v, int l) {
 // in slot order); the same arithmetic in the same order.
 template <bool LEAN>
 __device__ double hv_rows_block(const Group<true>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
-                                const double* __restrict__ u, const double* __restrict__ uprev,
-                                double* __restrict__ w, double sj, double sp, double bj) {
-  const int nd = Dn.n, nu = U.n;
+                                const glb_f64* __restrict__ u, const glb_f64* __restrict__ uprev,
+                                glb_f64* __restrict__ w, double sj, double sp, double bj) {
+  const int nd = rfl(Dn.n), nu = rfl(U.n);
   const int nch = (nd + 63) >> 6;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int R = (int)(blockDim.x >> 6) / nch;
+  const int R = rfl(g.size >> 6) / nch;
   const int rr = wave / nch;
   const int id = (wave - rr * nch) * 64 + (int)(threadIdx.x & 63);
   const bool act = id < nd;
@@ -412,7 +482,7 @@ __device__ double hv_rows_block(const Group<true>& g, const ModelParams& p, cons
   const double ddn = Dn.dg[idc];
   const uint32_t sdn = Dn.st[idc];
   const int cm = rfl(g.lds.meta[2 + (wave - rr * nch)]);
-  const int us = g.lds.umeta[1];  // up slots per state
+  const int us = rfl(g.lds.umeta[1]);  // up slots per state
   double dot = 0.0;
   int buf = 0;
   for (int r0 = 0; r0 < nu; r0 += R) {
@@ -525,16 +595,16 @@ __device__ double hv_rows_block(const Group<true>& g, const ModelParams& p, cons
 // barrier is taken: every wave streams its rows at its own pace.
 template <int C>
 __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
-                               const double* __restrict__ u, const double* __restrict__ uprev,
-                               double* __restrict__ w, double sj, double sp, double bj) {
+                               const glb_f64* __restrict__ u, const glb_f64* __restrict__ uprev,
+                               glb_f64* __restrict__ w, double sj, double sp, double bj) {
   constexpr int HB = C >= 4 ? 2 : 4;  // up hops whose loads (C columns each) are in flight together
-  const int nd = Dn.n, nu = U.n;
+  const int nd = rfl(Dn.n), nu = rfl(U.n);
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = (int)(threadIdx.x & 63);
-  const int nwv = (int)(blockDim.x >> 6);
+  const int nwv = rfl(g.size >> 6);
   lds_f64* const row = g.lds.rows + wave * (64 * C);
   const double bsp = bj * sp;
-  const int us = g.lds.umeta[1];      // up slots per state
+  const int us = rfl(g.lds.umeta[1]); // up slots per state
   const int ds = rfl(g.lds.meta[1]);  // dn slots per state
   int idc[C];
 #pragma unroll
@@ -542,7 +612,7 @@ __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const
   double dot = 0.0;
   for (int iu = wave; iu < nu; iu += nwv) {
     const int64_t ro = (int64_t)iu * nd;
-    const double* __restrict__ xr = u + ro;
+    const glb_f64* __restrict__ xr = u + ro;
     const int cu = rfl(g.lds.ucnt[iu]);
     const int lt = lane < cu ? (int)g.lds.utgt[iu * us + lane] : 0;
     const double lv = lane < cu ? g.lds.uval[iu * us + lane] : 0.0;
@@ -559,7 +629,7 @@ __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const
       for (int e = 0; e < HB; ++e) {
         const bool on = e0 + e < cu;  // uniform over the wave; an off hop re-reads hop e0 with value 0
         const int ee = on ? e0 + e : e0;
-        const double* __restrict__ src = u + (int64_t)__builtin_amdgcn_readlane(lt, ee) * nd;
+        const glb_f64* __restrict__ src = u + (int64_t)__builtin_amdgcn_readlane(lt, ee) * nd;
         hv[e] = on ? readlane_d(lv, ee) : 0.0;
 #pragma unroll
         for (int c = 0; c < C; ++c) gv[e][c] = src[idc[c]];
@@ -614,17 +684,19 @@ __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const
 // coefficient unknown) a = <w, v_j>; w -= a v_j; returns |w|^2 through *nrm2.
 // With known coefficients (regeneration passes) a_in is used as given.
 template <bool BLOCK, bool FAST = false, bool LEAN = false>
-__device__ void lanczos_step(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
-                             const double* __restrict__ u, const double* __restrict__ uprev, double* __restrict__ w,
-                             double sj, double sp, double bj, bool known, double a_in, double* a_out, double* nrm2) {
-  const int nd = Dn.n;
+__device__ __forceinline__ void lanczos_step(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U,
+                                             const SpinList& Dn, const glb_f64* __restrict__ u,
+                                             const glb_f64* __restrict__ uprev, glb_f64* __restrict__ w, double sj,
+                                             double sp, double bj, bool known, double a_in, double* a_out,
+                                             double* nrm2) {
+  const int nd = rfl(Dn.n);
   const int64_t D = (int64_t)U.n * nd;
   double dot = 0.0;
   // sweep 1: w = sj H u - bj sp uprev, dot <w, u>
   bool staged = false;
   if constexpr (BLOCK) {
     const int nch = (nd + 63) >> 6;
-    const int nwv = (int)(blockDim.x >> 6);
+    const int nwv = rfl(g.size >> 6);
     if (g.has_lds && g.lds.meta[0] == nd && nd > 0 && nch <= nwv && 2ll * (nwv / nch) * nd <= g.lds.rows_cap &&
         D < (1ll << 31)) {
       if (up_cached(g, U)) {
@@ -702,21 +774,45 @@ __device__ void lanczos_step(const Group<BLOCK>& g, const ModelParams& p, const 
 // than the 768-thread budget leaves beside the wave-private row sweep).
 template <bool BLOCK, bool FAST, bool LEAN>
 __device__ __noinline__ void lanczos_step_call(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U,
-                                               const SpinList& Dn, const double* __restrict__ u,
-                                               const double* __restrict__ uprev, double* __restrict__ w, double sj,
+                                               const SpinList& Dn, const glb_f64* __restrict__ u,
+                                               const glb_f64* __restrict__ uprev, glb_f64* __restrict__ w, double sj,
                                                double sp, double bj, bool known, double a_in, double* a_out,
                                                double* nrm2) {
   lanczos_step<BLOCK, FAST, LEAN>(g, p, U, Dn, u, uprev, w, sj, sp, bj, known, a_in, a_out, nrm2);
 }
 
+// 1 / d from the hardware estimate and two Newton steps (to rounding).
+__device__ __forceinline__ double recip(double d) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const double r0 = __builtin_amdgcn_rcp(d);
+  const double r1 = fma(r0, fma(-d, r0, 1.0), r0);
+  return fma(r1, fma(-d, r1, 1.0), r1);
+#else
+  return 1.0 / d;
+#endif
+}
+
 // Lowest eigenpair of the m x m tridiagonal (alpha, beta): multisection over
-// the group's lanes on the Sturm count, then inverse iteration at a shift just
-// below the eigenvalue (T - shift is positive definite there, so the Thomas
-// solve needs no pivoting).  Writes the unit eigenvector to sv (tc is scratch)
-// and returns theta and |last component| through theta / slast.
-template <bool BLOCK>
-__device__ __noinline__ void tri_lowest(const Group<BLOCK>& g, const double* alpha, const double* beta, int m, double* sv,
-                           double* tc, double* scal, double* theta, double* slast) {
+// the group's lanes, then inverse iteration at a shift just below the
+// eigenvalue (T - shift is positive definite there, so the Thomas solve needs
+// no pivoting).  Whether an eigenvalue lies below x is whether a leading minor
+// of T - x is not positive; the minors follow P_i = (a_i - x) P_{i-1} -
+// b_{i-1}^2 P_{i-2} without a division (the pivots' ratio form waits for one
+// every row), with T scaled by a power of two to a span of order one and the
+// minors brought back to order one every eight rows.  Every pass is a serial
+// chain over the rows: rows are read eight at a time, and one wavefront on each
+// SIMD tests shifts.  *theta: on entry an upper bound (the lowest eigenvalue
+// of a leading block, or 1e300), from which the first round's shifts step down
+// by powers of 2^(1/4), since the next check moves it by little.  Writes the
+// unit eigenvector to sv (tc and ti are scratch) and returns theta and |last
+// component| through theta / slast.  T: glb_f64, or lds_f64 for copies in LDS.
+// A check in block mode, 8 to 56 steps: 15 us (division form, serial rows: 74).
+template <bool BLOCK, class T>
+__device__ __noinline__ void tri_lowest(const Group<BLOCK>& gr, const T* alpha, const T* beta, int m, T* sv, T* tc,
+                                        T* ti, T* scal, double* theta, double* slast) {
+  const Group<BLOCK> g = gr;
+  constexpr double kEps = 2.220446049250313e-16;
+  m = rfl(m);  // arguments of a call of its own count as divergent
   double lo = 1e300, hi = -1e300;
   for (int i = g.rank; i < m; i += g.size) {
     const double r = (i > 0 ? fabs(beta[i - 1]) : 0.0) + (i < m - 1 ? fabs(beta[i]) : 0.0);
@@ -725,61 +821,170 @@ __device__ __noinline__ void tri_lowest(const Group<BLOCK>& g, const double* alp
   }
   lo = -g.max(-lo);
   hi = g.max(hi);
-  constexpr int P = 64;  // shifts tested per round, one per lane of the first wave
+  constexpr int P = BLOCK ? 255 : 63;  // shifts tested per round: 1 / (P + 1) is exact
+  constexpr int R = 8;                 // rows read at a time
+  double sc = 1.0;
+  {
+    int ex = 0;
+    if (hi - lo > 0.0) (void)frexp(hi - lo, &ex);
+    sc = ldexp(1.0, -ex);
+  }
+  for (int i = g.rank; i < m; i += g.size) {
+    const double b = i > 0 ? beta[i - 1] * sc : 0.0;
+    tc[i] = alpha[i] * sc;
+    ti[i] = -b * b;
+  }
+  const double top = *theta + 8.0 * kEps * fmax(fabs(lo), fabs(hi));
+  bool fine = top < hi;  // the next round's shifts crowd towards hi
+  if (fine) hi = top;
+  g.sync();
   for (int round = 0; round < 64; ++round) {
-    if (hi - lo <= 4.0 * 2.220446049250313e-16 * fmax(fabs(lo), fabs(hi)) + 1e-300) break;
-    // lane r < P tests x_r = lo + (hi - lo) (r + 1) / (P + 1): is an eigenvalue below it?
-    bool below = false;
-    if (g.rank < P) {
-      const double xr = lo + (hi - lo) * (double)(g.rank + 1) / (double)(P + 1);
-      double q = alpha[0] - xr;
-      int c = q < 0.0 ? 1 : 0;
-      for (int i = 1; i < m; ++i) {
-        const double qq = q != 0.0 ? q : 1e-300;
-        q = alpha[i] - xr - beta[i - 1] * beta[i - 1] / qq;
-        c += q < 0.0 ? 1 : 0;
+    if (hi - lo <= 4.0 * kEps * fmax(fabs(lo), fabs(hi)) + 1e-300) break;
+    // shift r < P, increasing with r: is an eigenvalue below it?
+    const auto shift_at = [=](int r) {
+      if (fine) {
+        const int q = r & 3;
+        const double c = q == 0 ? 1.0 : q == 1 ? 0.8408964152537145 : q == 2 ? 0.7071067811865476 : 0.5946035575013605;
+        return hi - (hi - lo) * ldexp(c, -(r >> 2));
       }
-      below = c >= 1;
+      return lo + (hi - lo) * ((double)(r + 1) * (1.0 / (P + 1)));
+    };
+    bool below = false;
+    if (rfl(g.rank & ~63) < P) {
+      const double xr = shift_at(g.rank) * sc;
+      double p1 = 0.0, p0 = 1.0, least = 1.0;  // P_{i-2}, P_{i-1}, the least minor so far (by sign)
+      const auto row = [&](double av, double cv) {
+        const double pn = fma(av - xr, p0, cv * p1);
+        p1 = p0;
+        p0 = pn;
+        least = fmin(least, pn);
+      };
+      int i0 = 0;
+      for (; i0 + R <= m; i0 += R) {
+        double av[R], cv[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          av[q] = tc[i0 + q];
+          cv[q] = ti[i0 + q];
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) row(av[q], cv[q]);
+        int ex = 0;
+        (void)frexp(fmax(fabs(p0), fabs(p1)), &ex);
+        p0 = ldexp(p0, -ex);
+        p1 = ldexp(p1, -ex);
+      }
+#pragma unroll 1
+      for (; i0 < m; ++i0) row(tc[i0], ti[i0]);
+      below = !(least > 0.0) || !(p0 > 0.0);
     }
     // r1 = first shift with an eigenvalue below it (P if none): the lowest
     // eigenvalue lies in [x_{r1-1}, x_{r1}] with x_{-1} = lo, x_P = hi
-    const int r1 = (int)(-g.max(below ? -(double)g.rank : -(double)P));
-    const double nlo = lo + (hi - lo) * (double)r1 / (double)(P + 1);
-    const double nhi = r1 >= P ? hi : lo + (hi - lo) * (double)(r1 + 1) / (double)(P + 1);
+    int r1 = P;
+    {
+      const int mine = first_lane(below && g.rank < P, g.rank, P);
+      if constexpr (BLOCK) {
+        lds_f64* const r = g.red + 16 * (round & 1);  // the other half's barrier lies between two uses
+        if (g.rank < 256 && (g.rank & 63) == 0) r[g.rank >> 6] = (double)mine;
+        __syncthreads();
+        const double r0 = r[0], ra = r[1], rb = r[2], rc = r[3];
+        r1 = rfl((int)fmin(fmin(r0, ra), fmin(rb, rc)));
+      } else {
+        r1 = mine;
+      }
+    }
+    const double nlo = r1 > 0 ? shift_at(r1 - 1) : lo;
+    const double nhi = r1 >= P ? hi : shift_at(r1);
     lo = nlo;
     hi = nhi;
+    fine = false;
   }
   const double th = 0.5 * (lo + hi);
-  if (g.rank == 0) {
+  g.sync();
+  if (rfl(g.rank & ~63) == 0) {
+    // Thomas algorithm on (T - shift) x = sv, factored once (ti = 1 / pivot,
+    // tc = upper coefficient), from x = 1: the factorisation runs with the
+    // first forward elimination; then back substitution, and once more from
+    // the unit vector.  The whole wavefront runs it (the same values in every
+    // lane), so that no branch depends on the lane.
     const double shift = th - fmax(1e-10 * fabs(th), 1e-12);
-    for (int i = 0; i < m; ++i) sv[i] = 1.0;
-    for (int it = 0; it < 2; ++it) {
-      // Thomas algorithm on (T - shift) x = sv: forward elimination, then back substitution
-      double c_prev = 0.0, d_prev = 0.0;
-      for (int i = 0; i < m; ++i) {
-        const double bl = i > 0 ? beta[i - 1] : 0.0;
-        const double den = (alpha[i] - shift) - bl * c_prev;
-        const double ci = i < m - 1 ? beta[i] / den : 0.0;
-        const double di = (sv[i] - bl * d_prev) / den;
-        tc[i] = ci;
-        sv[i] = di;
-        c_prev = ci;
-        d_prev = di;
+    double c_prev = 0.0, d_prev = 0.0, bl = 0.0, nrm = 1.0;
+    const auto factor = [&](int i, double av, double bv) {
+      const double inv = recip((av - shift) - bl * c_prev);
+      d_prev = (1.0 - bl * d_prev) * inv;
+      c_prev = bv * inv;
+      ti[i] = inv;
+      tc[i] = c_prev;
+      sv[i] = d_prev;
+      bl = bv;
+    };
+    int i0 = 0;
+    for (; i0 + R < m; i0 += R) {
+      double av[R], bv[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        av[q] = alpha[i0 + q];
+        bv[q] = beta[i0 + q];
       }
-      for (int i = m - 2; i >= 0; --i) sv[i] -= tc[i] * sv[i + 1];
-      double nrm = 0.0;
-      for (int i = 0; i < m; ++i) nrm += sv[i] * sv[i];
-      nrm = 1.0 / sqrt(nrm);
-      for (int i = 0; i < m; ++i) sv[i] *= nrm;
+#pragma unroll
+      for (int q = 0; q < R; ++q) factor(i0 + q, av[q], bv[q]);
     }
-    if (sv[0] < 0.0)
-      for (int i = 0; i < m; ++i) sv[i] = -sv[i];
-    scal[0] = th;
-    scal[1] = fabs(sv[m - 1]);
+#pragma unroll 1
+    for (; i0 < m; ++i0) factor(i0, alpha[i0], i0 < m - 1 ? (double)beta[i0] : 0.0);
+    for (int it = 0; it < 2; ++it) {
+      if (it > 0) {
+        const auto forward = [&](int i, double xv, double bv, double iv) {
+          d_prev = (nrm * xv - bl * d_prev) * iv;
+          sv[i] = d_prev;
+          bl = bv;
+        };
+        d_prev = 0.0;
+        bl = 0.0;
+        i0 = 0;
+        for (; i0 + R < m; i0 += R) {
+          double xv[R], bv[R], iv[R];
+#pragma unroll
+          for (int q = 0; q < R; ++q) {
+            xv[q] = sv[i0 + q];
+            bv[q] = beta[i0 + q];
+            iv[q] = ti[i0 + q];
+          }
+#pragma unroll
+          for (int q = 0; q < R; ++q) forward(i0 + q, xv[q], bv[q], iv[q]);
+        }
+#pragma unroll 1
+        for (; i0 < m; ++i0) forward(i0, sv[i0], i0 < m - 1 ? (double)beta[i0] : 0.0, ti[i0]);
+      }
+      double n2 = d_prev * d_prev;
+      const auto back = [&](int i, double xv, double cv) {
+        d_prev = xv - cv * d_prev;
+        sv[i] = d_prev;
+        n2 = fma(d_prev, d_prev, n2);
+      };
+      i0 = m - 2;
+      for (; i0 >= R - 1; i0 -= R) {
+        double xv[R], cv[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          xv[q] = sv[i0 - q];
+          cv[q] = tc[i0 - q];
+        }
+#pragma unroll
+        for (int q = 0; q < R; ++q) back(i0 - q, xv[q], cv[q]);
+      }
+#pragma unroll 1
+      for (; i0 >= 0; --i0) back(i0, sv[i0], tc[i0]);
+      nrm = 1.0 / sqrt(n2);
+    }
+    if (d_prev < 0.0) nrm = -nrm;  // first component positive
+    scal[0] = nrm;
   }
   g.sync();
-  *theta = scal[0];
-  *slast = scal[1];
+  const double nrm = scal[0];
+  *theta = th;
+  *slast = fabs(nrm * sv[m - 1]);
+  g.sync();
+  for (int i = g.rank; i < m; i += g.size) sv[i] = nrm * sv[i];
   g.sync();
 }
 
@@ -818,77 +1023,358 @@ __device__ cplx cf_value(const double* a, const double* b, int m, double norm2, 
   return r;
 }
 
+// ---------------------------------------------------------------------------
+// Sectors held on chip (block mode): u_j in LDS, each thread its own up to S
+// states of u_j and u_{j-1} in registers, so a Lanczos step reads nothing from
+// memory: its hops are LDS gathers through the cached lists, and the
+// orthogonalisation against u_j and the norm stay in registers.  A step is
+// then two reductions over the workgroup and the gathers (ground state, 400
+// states: 2.2 us a step against 14 through the L2, where a step is six round
+// trips; 4,900 states: 6 us against 29, LDS reads).  Hops kept in registers as
+// packed LDS offsets, bond by bond, measured the same step at 400 states and a
+// longer one at 4,900 (a bond without a hop still costs its read).
+// ---------------------------------------------------------------------------
+constexpr int kResGround = 5;  // states per thread: 1024 * 5 >= kLdsRowsSolve
+constexpr int kResFrac = 7;    // 768 * 7
+constexpr int kResHops = 4;    // hops in flight (a half-filled spin sector of 6 or 8 sites has 3 or 4 slots)
+static_assert(kBlockGround * kResGround >= kLdsRowsSolve && kBlockFrac * kResFrac >= kLdsRowsSolve, "resident states");
+
+template <int S>
+struct Resident {
+  double u[S], up[S], dg[S];
+  uint32_t at[S];  // row << 16 | column
+};
+
+// Both lists cached (cache_dn and cache_up of this sector) and the sector's
+// vector within the row buffer.
+__device__ __forceinline__ bool resident_fits(const Group<true>& g, const SpinList& U, const SpinList& Dn) {
+  const int64_t D = (int64_t)U.n * Dn.n;
+  return g.has_lds && g.wave_rows && D > 0 && D <= g.lds.rows_cap && g.lds.meta[0] == Dn.n && up_cached(g, U);
+}
+
+// u_j and u_{j-1} (null: zero) from global memory (element k written by this
+// very thread, or before a barrier).
+template <int S>
+__device__ __forceinline__ void resident_load(const Group<true>& g, const ModelParams& p, const SpinList& U,
+                                              const SpinList& Dn, const glb_f64* u0, const glb_f64* up0,
+                                              Resident<S>& r) {
+  const int nd = Dn.n, D = U.n * nd;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int k = g.rank + s * g.size;
+    const bool act = k < D;
+    const int kc = act ? k : 0;
+    const int iu = kc / nd, id = kc - iu * nd;
+    r.at[s] = (uint32_t)iu << 16 | (uint32_t)id;
+    r.dg[s] = U.dg[iu] + Dn.dg[id] + ((U.st[iu] & Dn.st[id] & 1u) ? p.u : 0.0);
+    r.u[s] = act ? u0[kc] : 0.0;
+    r.up[s] = act && up0 ? up0[kc] : 0.0;
+    if (act) g.lds.rows[k] = r.u[s];
+  }
+  __syncthreads();
+}
+
+// One step, as lanczos_step on a sector of D states and nd columns: u_{j+1} =
+// w in place of u_j (LDS and registers), alpha_j and |w|^2 returned.
+template <int S>
+__device__ __forceinline__ void resident_step(const Group<true>& g, Resident<S>& r, int D, int nd, double sj, double sp,
+                                              double bj, double* a_out, double* nrm2) {
+  const BlockLds L = g.lds;
+  const int us = rfl(L.umeta[1]), ds = rfl(L.meta[1]);
+  const int first = rfl(g.rank & ~63);  // the wave's first state
+  const int nw = (D < g.size ? D + 63 : g.size) >> 6;  // wavefronts with a state
+  double dot = 0.0;
+  const double bsp = bj * sp;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {  // w takes the place of u_{j-1}
+    if (first + s * g.size < D) {  // uniform over the wave
+      const int iu = (int)(r.at[s] >> 16), id = (int)(r.at[s] & 0xffffu);
+      double acc = r.dg[s] * r.u[s];
+      // four hops at a time: their entries, then their states
+#pragma unroll 1
+      for (int e0 = 0; e0 < us; e0 += kResHops) {
+        double hv[kResHops], x[kResHops];
+        int t[kResHops];
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q) {
+          const int e = iu * us + (e0 + q < us ? e0 + q : 0);
+          t[q] = (int)L.utgt[e];
+          hv[q] = L.uval[e];
+        }
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q) x[q] = L.rows[t[q] * nd + id];
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q)
+          if (e0 + q < us) acc = fma(hv[q], x[q], acc);
+      }
+#pragma unroll 1
+      for (int e0 = 0; e0 < ds; e0 += kResHops) {
+        double hv[kResHops], x[kResHops];
+        int t[kResHops];
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q) {
+          const int e = (e0 + q < ds ? e0 + q : 0) * nd + id;
+          t[q] = (int)L.tgt[e];
+          hv[q] = L.val[e];
+        }
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q) x[q] = L.rows[iu * nd + t[q]];
+#pragma unroll
+        for (int q = 0; q < kResHops; ++q)
+          if (e0 + q < ds) acc = fma(hv[q], x[q], acc);
+      }
+      const double v = sj * acc - bsp * r.up[s];
+      r.up[s] = g.rank + s * g.size < D ? v : 0.0;
+      dot = fma(r.up[s], r.u[s], dot);
+    }
+  }
+  const double a = sj * g.template sum_half<0>(dot, nw);
+  const double as = a * sj;
+  double n2 = 0.0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const double us = r.u[s];
+    r.u[s] = r.up[s] - as * us;
+    r.up[s] = us;
+    n2 = fma(r.u[s], r.u[s], n2);
+    const int k = g.rank + s * g.size;
+    if (k < D) L.rows[k] = r.u[s];  // every gather from u_j lies before the sum's barrier
+  }
+  *a_out = a;
+  *nrm2 = g.template sum_half<1>(n2, nw);  // and its barrier makes u_{j+1} visible
+}
+
+// Ground-state tridiagonal check on LDS copies at st (5 m + 8 doubles), the
+// eigenvector copied to sv.
+__device__ __noinline__ void tri_lowest_lds(const Group<true>& g, lds_f64* st, const glb_f64* alpha,
+                                            const glb_f64* beta, int m, glb_f64* sv, double* theta, double* slast) {
+  for (int i = g.rank; i < m; i += g.size) {
+    st[i] = alpha[i];
+    st[m + i] = beta[i];
+  }
+  g.sync();
+  tri_lowest<true, lds_f64>(g, st, st + m, m, st + 2 * m, st + 3 * m, st + 4 * m, st + 5 * m, theta, slast);
+  for (int i = g.rank; i < m; i += g.size) sv[i] = st[2 * m + i];
+  g.sync();
+}
+
+// Steps j0 .. j1 - 1 of solve_ground's Lanczos on a resident sector, every u_j
+// written to V, fewer on breakdown (returned: the step after the last).  A
+// call of its own between two convergence checks, so neither's registers are
+// live in the other.
+__device__ __noinline__ int ground_resident(const Group<true>& gr, const ModelParams& p, const SpinList& U,
+                                            const SpinList& Dn, glb_f64* V, glb_f64* alpha, glb_f64* beta, int j0, int j1,
+                                            double s0) {
+  Group<true> g = gr;  // in registers
+  g.size = rfl(gr.size);
+  const int nd = rfl(Dn.n), D = rfl(U.n) * nd;
+  Resident<kResGround> r;
+  resident_load(g, p, U, Dn, V + (int64_t)j0 * D, j0 > 0 ? V + (int64_t)(j0 - 1) * D : nullptr, r);
+  j0 = rfl(j0);
+  j1 = rfl(j1);
+  double bj = j0 > 0 ? beta[j0 - 1] : 0.0;
+  double sj = j0 > 0 ? 1.0 / bj : s0;
+  double sp = j0 > 1 ? 1.0 / beta[j0 - 2] : (j0 > 0 ? s0 : 0.0);
+  for (int j = j0; j < j1; ++j) {
+    double aj, nn;
+    resident_step(g, r, D, nd, sj, sp, bj, &aj, &nn);
+    glb_f64* const Vn = V + (int64_t)(j + 1) * D;
+#pragma unroll
+    for (int s = 0; s < kResGround; ++s) {
+      const int k = g.rank + s * g.size;
+      if (k < D) Vn[k] = r.u[s];
+    }
+    const double bn = sqrt(nn);
+    if (g.rank == 0) {
+      alpha[j] = aj;
+      beta[j] = bn;
+    }
+    if (!(bn > 1e-12 * (fabs(aj) + bj))) {
+      j1 = j + 1;
+      break;
+    }
+    sp = sj;
+    sj = 1.0 / bn;
+    bj = bn;
+  }
+  g.sync();
+  return j1;
+}
+
+// solve_ground's Lanczos loop: the step count, with the Ritz value and its
+// residual.
+template <bool BLOCK, bool FAST>
+__device__ __forceinline__ int ground_loop(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U,
+                                           const SpinList& Dn, const SlotRef& sl, double* V, int check_every, int cap,
+                                           double tol, double s0, double* theta, double* ritz) {
+  const int64_t D = (int64_t)U.n * Dn.n;
+  double* const alpha = sl.alpha();
+  double* const beta = sl.beta();
+  double sj = s0, sp = 0.0, bj = 0.0;
+  for (int m = 0;;) {
+    const int next = (m / check_every + 1) * check_every < cap ? (m / check_every + 1) * check_every : cap;
+    bool done = false;
+    if constexpr (BLOCK && FAST) {
+      if (resident_fits(g, U, Dn)) {
+        m = ground_resident(g, p, U, Dn, glb(V), glb(alpha), glb(beta), m, next, s0);
+        done = true;
+      }
+    }
+    while (!done) {
+      double aj, nn;
+      const glb_f64* u = glb(V + (int64_t)m * D);
+      lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, u, m > 0 ? u - D : u, glb(V + (int64_t)(m + 1) * D), sj, sp, bj,
+                                           false, 0.0, &aj, &nn);
+      const double bn = sqrt(nn);
+      if (g.rank == 0) {
+        alpha[m] = aj;
+        beta[m] = bn;
+      }
+      g.sync();
+      const bool breakdown = !(bn > 1e-12 * (fabs(aj) + bj));
+      sp = sj;
+      sj = 1.0 / bn;
+      bj = bn;
+      ++m;
+      done = breakdown || m == next;
+    }
+    const double bn = beta[m - 1];
+    const bool breakdown = !(bn > 1e-12 * (fabs(alpha[m - 1]) + (m > 1 ? beta[m - 2] : 0.0)));
+    double slast;
+    // block mode: the tridiagonal solve runs on copies in the LDS row buffer
+    // (idle between sweeps); the eigenvector goes back to sv
+    bool lds = false;
+    if constexpr (BLOCK) lds = g.has_lds && 5 * m + 8 <= g.lds.rows_cap;
+    if constexpr (BLOCK) {
+      if (lds) tri_lowest_lds(g, g.lds.rows, glb(alpha), glb(beta), m, glb(sl.sv()), theta, &slast);
+    }
+    if (!lds)
+      tri_lowest<BLOCK, glb_f64>(g, glb(alpha), glb(beta), m, glb(sl.sv()), glb(sl.tc()), glb(sl.vec(3)), glb(sl.scal()),
+                                 theta, &slast);
+    *ritz = breakdown ? 0.0 : bn * slast;
+    if (*ritz <= tol || breakdown || m == cap) return m;
+  }
+}
+
+// Convergence of a continued fraction, step by step.  Continuants of the
+// fraction at z = i wmin: y_m = d_0 - b_0^2 / (d_1 - b_1^2 / (... d_{m-1})) =
+// A_m / B_m with d_k = (e0 - a_k) + i sgn wmin, A_n = d_n A_{n-1} - b_{n-1}^2
+// A_{n-2} (A_{-1} = 1, A_0 = d_0; B_{-1} = 0, B_0 = 1), and f_m = sgn n2 B_m /
+// A_m is the value cf_value(a, b, m, n2, e0, sgn, wmin) takes.  Every member
+// holds the same values (rescaled by the size of A_m when that leaves
+// 10^+-60), so a check costs O(1) and no barrier.
+struct CfTrack {
+  cplx A{1.0, 0.0}, Ap{0.0, 0.0}, B{0.0, 0.0}, Bp{1.0, 0.0}, prev{0.0, 0.0};
+  int calm = 0;
+
+  // Step j with coefficient aj (bj: the previous off-diagonal); true when the
+  // fraction has changed by at most cf_tol * max(|f|, n2) over each of the
+  // last two 8-step checks (against the part's spectral weight n2 as well, so
+  // a small |G(i wmin)| does not make the test unreachable).
+  __device__ __forceinline__ bool step(int j, double aj, double bj, double n2, double e0, double sgn, double wmin,
+                                       double cf_tol) {
+    const cplx d = {e0 - aj, sgn * wmin};
+    const double c = -bj * bj;  // -b_{j-1}^2 (unused at j = 0)
+    cplx An, Bn;
+    if (j == 0) {
+      An = d;
+      Bn = {1.0, 0.0};
+      Ap = {1.0, 0.0};
+      Bp = {0.0, 0.0};
+    } else {
+      An = {d.re * A.re - d.im * A.im + c * Ap.re, d.re * A.im + d.im * A.re + c * Ap.im};
+      Bn = {d.re * B.re - d.im * B.im + c * Bp.re, d.re * B.im + d.im * B.re + c * Bp.im};
+      Ap = A;
+      Bp = B;
+    }
+    A = An;
+    B = Bn;
+    const double sz = fmax(fabs(A.re), fabs(A.im));
+    if (sz > 1e60 || (sz < 1e-60 && sz > 0.0)) {
+      const double r = 1.0 / sz;
+      A = {A.re * r, A.im * r};
+      B = {B.re * r, B.im * r};
+      Ap = {Ap.re * r, Ap.im * r};
+      Bp = {Bp.re * r, Bp.im * r};
+    }
+    if ((j + 1) % 8 != 0) return false;
+    const cplx f = cdiv({sgn * n2 * B.re, sgn * n2 * B.im}, A);
+    const double dd = hypot(f.re - prev.re, f.im - prev.im);
+    calm = dd <= cf_tol * fmax(hypot(f.re, f.im), n2) ? calm + 1 : 0;
+    prev = f;
+    return calm >= 2;
+  }
+};
+
+// cf_coeffs on a resident sector.
+__device__ __noinline__ int cf_resident(const Group<true>& gr, const ModelParams& p, const SpinList& U,
+                                        const SpinList& Dn, const glb_f64* u0, double n2, int cap, double e0,
+                                        double sgn, double wmin, double cf_tol, glb_f64* a, glb_f64* b, glb_f64* qt,
+                                        int kcap) {
+  Group<true> g = gr;  // in registers
+  g.size = rfl(gr.size);
+  const int nd = rfl(Dn.n), D = rfl(U.n) * nd;
+  Resident<kResFrac> r;
+  resident_load(g, p, U, Dn, u0, nullptr, r);
+  CfTrack track;
+  cap = rfl(cap);
+  double sj = 1.0 / sqrt(n2), sp = 0.0, bj = 0.0;
+  for (int j = 0;; ++j) {
+    if (qt) {
+#pragma unroll
+      for (int s = 0; s < kResFrac; ++s) {
+        const int k = g.rank + s * g.size;
+        if (k < D) qt[(int64_t)k * kcap + j] = sj * r.u[s];
+      }
+    }
+    double aj, nn;
+    resident_step(g, r, D, nd, sj, sp, bj, &aj, &nn);
+    const double bn = sqrt(nn);
+    const bool last = j == cap - 1 || !(bn > 1e-12 * (fabs(aj) + bj));
+    if (g.rank == 0) {
+      a[j] = aj;
+      if (!last) b[j] = bn;
+    }
+    if (last) return j + 1;
+    if (track.step(j, aj, bj, n2, e0, sgn, wmin, cf_tol)) return j + 1;
+    sp = sj;
+    sj = 1.0 / bn;
+    bj = bn;
+  }
+}
+
 // Lanczos coefficients of the sector (U, Dn) from the start vector in vec(1)
 // (unnormalised, |u|^2 = n2), stopping at breakdown, at cap steps, or when the
-// continued fraction s n2 / (s z + e0 - a0 - ...) at z = i wmin has changed by
-// at most cf_tol * max(|G|, n2) over each of the last two 8-step checks (the
-// fraction converges last at the frequency closest to the real axis).
-// Returns the step count.
+// continued fraction s n2 / (s z + e0 - a0 - ...) at z = i wmin has converged
+// (CfTrack; the fraction converges last at the frequency closest to the real
+// axis).  Returns the step count.
 template <bool BLOCK, bool FAST>
 __device__ int cf_coeffs(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
                          const SlotRef& sl, double n2, int cap, double e0, double sgn, double wmin, double cf_tol,
                          double* a, double* b, double* qt, int kcap) {
   double* u = sl.vec(1);
+  if constexpr (BLOCK && FAST) {
+    if (resident_fits(g, U, Dn))
+      return cf_resident(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap);
+  }
   double* up = sl.vec(0);
   double* w = sl.vec(2);
   double sj = 1.0 / sqrt(n2), sp = 0.0, bj = 0.0;
-  int m = 0, calm = 0;
-  cplx prev = {0.0, 0.0};
-  // Continuants of the fraction at z = i wmin, carried step by step:
-  // y_m = d_0 - b_0^2 / (d_1 - b_1^2 / (... d_{m-1})) = A_m / B_m with
-  // d_k = (e0 - a_k) + i sgn wmin, A_n = d_n A_{n-1} - b_{n-1}^2 A_{n-2}
-  // (A_{-1} = 1, A_0 = d_0; B_{-1} = 0, B_0 = 1), and f_m = sgn n2 B_m / A_m
-  // is the value cf_value(a, b, m, n2, e0, sgn, wmin) takes.  Every member
-  // holds the same values (rescaled by the size of A_m each step), so a check
-  // costs O(1) and no barrier.
-  cplx A = {1.0, 0.0}, Ap = {0.0, 0.0}, B = {0.0, 0.0}, Bp = {1.0, 0.0};
+  int m = 0;
+  CfTrack track;
   const int64_t D = (int64_t)U.n * Dn.n;
   for (int j = 0; j < cap; ++j) {
     double aj, nn;
     if (qt)  // keep the normalised Krylov vector v_j = sj u, state-major
       for (int64_t k = g.rank; k < D; k += g.size) qt[k * kcap + j] = sj * u[k];
-    lanczos_step<BLOCK, FAST, true>(g, p, U, Dn, u, up, w, sj, sp, bj, false, 0.0, &aj, &nn);
+    lanczos_step<BLOCK, FAST, true>(g, p, U, Dn, glb(u), glb(up), glb(w), sj, sp, bj, false, 0.0, &aj, &nn);
     a[j] = aj;
     m = j + 1;
     const double bn = sqrt(nn);
     if (j == cap - 1) break;
     if (!(bn > 1e-12 * (fabs(aj) + bj))) break;  // invariant subspace
     b[j] = bn;
-    {
-      const cplx d = {e0 - aj, sgn * wmin};
-      const double c = -bj * bj;  // -b_{j-1}^2 (unused at j = 0)
-      cplx An, Bn;
-      if (j == 0) {
-        An = d;
-        Bn = {1.0, 0.0};
-        Ap = {1.0, 0.0};
-        Bp = {0.0, 0.0};
-      } else {
-        An = {d.re * A.re - d.im * A.im + c * Ap.re, d.re * A.im + d.im * A.re + c * Ap.im};
-        Bn = {d.re * B.re - d.im * B.im + c * Bp.re, d.re * B.im + d.im * B.re + c * Bp.im};
-        Ap = A;
-        Bp = B;
-      }
-      A = An;
-      B = Bn;
-      const double sz = fmax(fabs(A.re), fabs(A.im));
-      if (sz > 0.0) {
-        const double r = 1.0 / sz;
-        A = {A.re * r, A.im * r};
-        B = {B.re * r, B.im * r};
-        Ap = {Ap.re * r, Ap.im * r};
-        Bp = {Bp.re * r, Bp.im * r};
-      }
-    }
-    if (m % 8 == 0) {
-      const cplx f = cdiv({sgn * n2 * B.re, sgn * n2 * B.im}, A);
-      // change measured against the part's spectral weight n2 as well, so a
-      // small |G(i wmin)| does not make the test unreachable
-      const double dd = hypot(f.re - prev.re, f.im - prev.im);
-      calm = dd <= cf_tol * fmax(hypot(f.re, f.im), n2) ? calm + 1 : 0;
-      prev = f;
-      if (calm >= 2) break;
-    }
+    if (track.step(j, aj, bj, n2, e0, sgn, wmin, cf_tol)) break;
     double* t = up;
     up = u;
     u = w;
@@ -913,7 +1399,7 @@ __device__ __forceinline__ double start_value(uint64_t seed, int64_t k) {
 // loads in flight at a time, summed in step order.  A call of its own, so its
 // registers are allocated apart from the ground-state loop's.
 template <bool BLOCK>
-__device__ __noinline__ void combine_psi(const Group<BLOCK>& g, double* V, const double* c, int m, int64_t D) {
+__device__ __noinline__ void combine_psi(const Group<BLOCK>& g, glb_f64* V, const glb_f64* c, int m, int64_t D) {
   for (int64_t k = g.rank; k < D; k += g.size) {
     double acc = 0.0;
     int j = 0;
@@ -933,7 +1419,7 @@ __device__ __noinline__ void combine_psi(const Group<BLOCK>& g, double* V, const
 }
 
 template <bool BLOCK, bool FAST>
-__device__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, const SlotRef& sl) {
+__device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, const SlotRef& sl) {
   const ModelParams& p = cf.params[mi];
   const int ns = p.nb + 1;
   const int n_0 = build_list<BLOCK>(g, p, ns, p.n_up, cf.sign_width, sl, 1);
@@ -948,8 +1434,6 @@ __device__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, co
     }
   }
   const int64_t D = (int64_t)n_0 * nd;
-  double* const alpha = sl.alpha();
-  double* const beta = sl.beta();
 
   // ---- Lanczos with every vector kept (u_j = V_j, v_j = s_j u_j) ----
   const uint64_t seed = cf.seed ^ (0xA0761D6478BD642Full * (uint64_t)(mi + 1));
@@ -963,57 +1447,17 @@ __device__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, co
   n2 = g.sum(n2);
   g.sync();
   const double s0 = 1.0 / sqrt(n2);
-  double sj = s0, sp = 0.0, bj = 0.0;
-  int m = 0;
-  double theta = 0.0, slast = 0.0, ritz = 1e300;
+  double theta = 1e300, ritz = 1e300;
   const int cap = (int)((int64_t)cf.max_iter < D ? (int64_t)cf.max_iter : D);
-  for (int j = 0; j < cap; ++j) {
-    double aj, nn;
-    const double* u = V + (int64_t)j * D;
-    lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, u, j > 0 ? u - D : u, V + (int64_t)(j + 1) * D, sj, sp, bj, false, 0.0, &aj, &nn);
-    m = j + 1;
-    const double bn = sqrt(nn);
-    if (g.rank == 0) {
-      alpha[j] = aj;
-      beta[j] = bn;
-    }
-    g.sync();
-    const bool breakdown = !(bn > 1e-12 * (fabs(aj) + bj));
-    const bool check = breakdown || m == cap || (m >= cf.check_every && m % cf.check_every == 0);
-    if (check) {
-      bool done = false;
-      if constexpr (BLOCK) {
-        // block mode: the tridiagonal solve runs on copies in the LDS row
-        // buffer (idle between sweeps); the eigenvector goes back to sv
-        if (g.has_lds && 4 * m + 8 <= g.lds.rows_cap) {
-          double* const st = (double*)g.lds.rows;
-          for (int i = g.rank; i < m; i += g.size) {
-            st[i] = alpha[i];
-            st[m + i] = beta[i];
-          }
-          g.sync();
-          tri_lowest<BLOCK>(g, st, st + m, m, st + 2 * m, st + 3 * m, st + 4 * m, &theta, &slast);
-          for (int i = g.rank; i < m; i += g.size) sl.sv()[i] = st[2 * m + i];
-          g.sync();
-          done = true;
-        }
-      }
-      if (!done) tri_lowest<BLOCK>(g, alpha, beta, m, sl.sv(), sl.tc(), sl.scal(), &theta, &slast);
-      ritz = breakdown ? 0.0 : bn * slast;
-      if (ritz <= cf.tol || breakdown) break;
-    }
-    sp = sj;
-    sj = 1.0 / bn;
-    bj = bn;
-  }
+  const int m = ground_loop<BLOCK, FAST>(g, p, U, Dn, sl, V, cf.check_every, cap, cf.tol, s0, &theta, &ritz);
   // psi = sum_j sv_j s_j V_j in step order, over V_0: each state's entries of
   // every V_j are read by the one member that then overwrites V_0 there
   double* const psi = V;
   {
     double* const c = sl.tc();
-    for (int j = g.rank; j < m; j += g.size) c[j] = sl.sv()[j] * (j == 0 ? s0 : 1.0 / beta[j - 1]);
+    for (int j = g.rank; j < m; j += g.size) c[j] = sl.sv()[j] * (j == 0 ? s0 : 1.0 / sl.beta()[j - 1]);
     g.sync();
-    combine_psi<BLOCK>(g, V, c, m, D);
+    combine_psi<BLOCK>(g, glb(V), glb(c), m, D);
   }
   g.sync();
   // normalise psi and take the explicit residual |H psi - theta psi|
@@ -1031,7 +1475,7 @@ __device__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, co
     double aj, nn;
     // w = H psi - theta psi (unit scale, no previous vector, known coefficient)
     double* wr = sl.vec(2);
-    lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, psi, sl.vec(0), wr, 1.0, 0.0, 0.0, true, theta, &aj, &nn);
+    lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, glb(psi), glb(sl.vec(0)), glb(wr), 1.0, 0.0, 0.0, true, theta, &aj, &nn);
     double r2 = 0.0;
     for (int64_t k = g.rank; k < D; k += g.size) r2 += wr[k] * wr[k];
     res2 = g.sum(r2);
@@ -1100,7 +1544,7 @@ __device__ void solve_fraction(const Group<BLOCK>& g, const Config& cf, int mi, 
     m = cf_coeffs<BLOCK, FAST>(g, p, T, Dn, sl, nn, cf.cf_steps, theta, part == 0 ? 1.0 : -1.0, cf.wmin, cf.cf_tol, a, b,
                          qt, kc);
   }
-  // coefficient arrays were written by every member with the same values
+  // coefficient arrays were written by one member, or by every one with the same values
   g.sync();
   for (int j = g.rank; j < kc; j += g.size) {
     if (j >= m) a[j] = 0.0;
@@ -1151,7 +1595,7 @@ __global__ __launch_bounds__(PHASE ? kBlockFrac : kBlockGround) void k_batch_sol
     __shared__ int32_t s_umeta[4];
     __shared__ double s_ddn[kLdsDiagSolve];
     __shared__ uint32_t s_sdn[kLdsDiagSolve];
-    Group<true> g{(int)threadIdx.x, (int)blockDim.x, red};
+    Group<true> g{(int)threadIdx.x, (int)blockDim.x, (lds_f64*)red};
     g.lds = BlockLds{(lds_f64*)s_rows, kLdsRowsSolve,     (lds_u32*)s_tgt,  (lds_f64*)s_val,
                      kLdsDnSolve,      (lds_i32*)s_meta,  (lds_u32*)s_utgt, (lds_f64*)s_uval,
                      (lds_i32*)s_ucnt, kLdsUpSolve,       kLdsUpRowsSolve,  (lds_i32*)s_umeta,
@@ -1759,7 +2203,7 @@ __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi
   int it = 0;
   for (; it < bc.cg_max && rho > bc.cg_tol * bc.cg_tol * rho0 && rho > 0.0; ++it) {
     double aj, nn;
-    lanczos_step<true>(g, p, U0, Dn, pv, bs.vec(8), qv, 1.0, 0.0, 0.0, true, e0, &aj, &nn);  // q = (H - E0) p
+    lanczos_step<true>(g, p, U0, Dn, glb(pv), glb(bs.vec(8)), glb(qv), 1.0, 0.0, 0.0, true, e0, &aj, &nn);  // q = (H - E0) p
     double qp = 0.0, qpsi = 0.0;
     for (int64_t k = g.rank; k < D; k += g.size) {
       qp += qv[k] * pv[k];
@@ -1822,7 +2266,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_backward(BwdConfig bc) {
   __shared__ double s_uval[kLdsUpBwd];
   __shared__ int32_t s_ucnt[kLdsUpRowsBwd];
   __shared__ int32_t s_umeta[4];
-  Group<true> g{(int)threadIdx.x, (int)blockDim.x, red};
+  Group<true> g{(int)threadIdx.x, (int)blockDim.x, (lds_f64*)red};
   g.lds = BlockLds{(lds_f64*)s_rows, kLdsRows,          (lds_u32*)s_tgt,  (lds_f64*)s_val,
                    kLdsDnBwd,        (lds_i32*)s_meta,  (lds_u32*)s_utgt, (lds_f64*)s_uval,
                    (lds_i32*)s_ucnt, kLdsUpBwd,         kLdsUpRowsBwd,    (lds_i32*)s_umeta};
