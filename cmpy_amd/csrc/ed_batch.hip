@@ -46,12 +46,11 @@ constexpr int kMaxSites = kMaxBath + 1;
 constexpr int kBlock = 1024;      // threads per workgroup of the backward kernel
 // Solve kernels, per phase (ground-state tasks, continued-fraction tasks):
 // threads per workgroup (the VGPR budget is 512 / waves per SIMD) and whether
-// block-mode sweeps take the wave-private row path.  Measured on the
-// 512-model batch (bath sizes 5..9): the ground-state phase is fastest with
-// 16 waves and workgroup rows (the wave-private path needs more than the 128
-// VGPRs of 16 waves: 27-30 ms against 32-40 ms on 8 waves), the fraction phase
-// with 12 waves and wave-private rows (54-57 ms against 70 ms).
-constexpr int kBlockGround = 1024;
+// block-mode sweeps take the wave-private row path, which needs more than the
+// 128 VGPRs of 16 waves: with 12 waves a ground-state step of 63,504 states
+// takes 103 us against 135 on 16, one of 400 states held on chip 2.0 us against
+// 2.2; the 512-model batch (bath sizes 5..9) 62.8 ms against 69.6.
+constexpr int kBlockGround = 768;
 constexpr bool kFastGround = true;
 constexpr int kBlockFrac = 768;
 constexpr bool kFastFrac = true;
@@ -450,6 +449,16 @@ __device__ __forceinline__ double rfl_d(double v) {
   return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
 }
 
+// p, as a value the compiler knows nothing about (so that what is derived from
+// it in a loop is not computed ahead of the loop and kept in registers).
+template <class T>
+__device__ __forceinline__ T* opaque_uniform(T* p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+s"(p));
+#endif
+  return p;
+}
+
 constexpr int kUpPre = 6;  // up hops whose loads start before the staging barrier
 
 
@@ -592,7 +601,10 @@ __device__ double hv_rows_block(const Group<true>& g, const ModelParams& p, cons
 // wave-uniform row base) are loaded together, the row is staged in the
 // wave's own LDS buffer, and the dn hops are gathered slot by slot with the C
 // columns' table reads and gathers in flight together.  No workgroup
-// barrier is taken: every wave streams its rows at its own pace.
+// barrier is taken: every wave streams its rows at its own pace.  What bounds
+// it is the bytes a compute unit takes from the L2 (11 vectors a step with the
+// second sweep, 75 us at 52,920 states): more hop loads in flight, or the dn
+// tables in registers, measured the same.
 template <int C>
 __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
                                const glb_f64* __restrict__ u, const glb_f64* __restrict__ uprev,
@@ -602,72 +614,85 @@ __device__ double hv_rows_wave(const Group<true>& g, const ModelParams& p, const
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = (int)(threadIdx.x & 63);
   const int nwv = rfl(g.size >> 6);
+  // members once, by value: a store through w could alias the callers' copies
   lds_f64* const row = g.lds.rows + wave * (64 * C);
+  lds_i32* const ucnt = g.lds.ucnt;
+  lds_u32* const utgt = g.lds.utgt;
+  lds_f64* const uval = g.lds.uval;
+  lds_u32* const dtgt = g.lds.tgt;
+  lds_f64* const dval = g.lds.val;
+  const glb_f64* const udg = U.dg;
+  const glb_u32* const ust = U.st;
+  const double pu = p.u;
   const double bsp = bj * sp;
-  const int us = rfl(g.lds.umeta[1]); // up slots per state
-  const int ds = rfl(g.lds.meta[1]);  // dn slots per state
+  const int us = rfl(g.lds.umeta[1]);  // up slots per state
+  const int ds = rfl(g.lds.meta[1]);   // dn slots per state
   int idc[C];
 #pragma unroll
   for (int c = 0; c < C; ++c) idc[c] = lane + 64 * c < nd ? lane + 64 * c : nd - 1;
+  const bool dl = nd <= g.lds.ddn_cap;  // the dn diagonal and states cached in LDS
+  double ddn[C];
+  uint32_t occ = 0;  // the impurity's dn occupation, one bit a column
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    ddn[c] = dl ? (double)g.lds.ddn[idc[c]] : (double)Dn.dg[idc[c]];
+    occ |= ((dl ? (uint32_t)g.lds.sdn[idc[c]] : (uint32_t)Dn.st[idc[c]]) & 1u) << c;
+  }
   double dot = 0.0;
   for (int iu = wave; iu < nu; iu += nwv) {
     const int64_t ro = (int64_t)iu * nd;
     const glb_f64* __restrict__ xr = u + ro;
-    const int cu = rfl(g.lds.ucnt[iu]);
-    const int lt = lane < cu ? (int)g.lds.utgt[iu * us + lane] : 0;
-    const double lv = lane < cu ? g.lds.uval[iu * us + lane] : 0.0;
-    double x[C], acc[C];
+    const int cu = rfl(ucnt[iu]);
+    const int lt = lane < cu ? (int)utgt[iu * us + lane] : 0;
+    const double lv = lane < cu ? (double)uval[iu * us + lane] : 0.0;
+    // everything the row needs from memory but its hops, ahead of them
+    double x[C], acc[C], xp[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
       x[c] = xr[idc[c]];
       acc[c] = 0.0;
+      xp[c] = bsp != 0.0 ? uprev[ro + idc[c]] : 0.0;
     }
+    const double dgu = udg[iu];
+    const uint32_t stv = ust[iu];
     for (int e0 = 0; e0 < cu; e0 += HB) {
       double gv[HB][C];
-      double hv[HB];
-#pragma unroll
-      for (int e = 0; e < HB; ++e) {
-        const bool on = e0 + e < cu;  // uniform over the wave; an off hop re-reads hop e0 with value 0
-        const int ee = on ? e0 + e : e0;
-        const glb_f64* __restrict__ src = u + (int64_t)__builtin_amdgcn_readlane(lt, ee) * nd;
-        hv[e] = on ? readlane_d(lv, ee) : 0.0;
-#pragma unroll
-        for (int c = 0; c < C; ++c) gv[e][c] = src[idc[c]];
-      }
 #pragma unroll
       for (int e = 0; e < HB; ++e)
+        if (e0 + e < cu) {  // uniform over the wave
+          const glb_f64* __restrict__ src = u + (int64_t)__builtin_amdgcn_readlane(lt, e0 + e) * nd;
 #pragma unroll
-        for (int c = 0; c < C; ++c) acc[c] = fma(hv[e], gv[e][c], acc[c]);
+          for (int c = 0; c < C; ++c) gv[e][c] = src[idc[c]];
+        }
+#pragma unroll
+      for (int e = 0; e < HB; ++e)
+        if (e0 + e < cu) {
+          const double hv = readlane_d(lv, e0 + e);
+#pragma unroll
+          for (int c = 0; c < C; ++c) acc[c] = fma(hv, gv[e][c], acc[c]);
+        }
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) row[idc[c]] = x[c];
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    double xp[C];
-#pragma unroll
-    for (int c = 0; c < C; ++c) xp[c] = bsp != 0.0 ? uprev[ro + idc[c]] : 0.0;
     // dn hops slot by slot (slots past a state's count hold target 0 and value 0)
     for (int e = 0; e < ds; ++e) {
       uint32_t tg[C];
       double vl[C], gr[C];
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        tg[c] = g.lds.tgt[e * nd + idc[c]];
-        vl[c] = g.lds.val[e * nd + idc[c]];
+        tg[c] = dtgt[e * nd + idc[c]];
+        vl[c] = dval[e * nd + idc[c]];
       }
 #pragma unroll
       for (int c = 0; c < C; ++c) gr[c] = row[tg[c]];
 #pragma unroll
       for (int c = 0; c < C; ++c) acc[c] = fma(vl[c], gr[c], acc[c]);
     }
-    const double dgu = U.dg[iu];
-    const uint32_t stu = (uint32_t)rfl((int)U.st[iu]);
-    const bool dl = nd <= g.lds.ddn_cap;  // the dn diagonal and states cached in LDS
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-      const double ddn = dl ? (double)g.lds.ddn[idc[c]] : Dn.dg[idc[c]];
-      const uint32_t sdn = dl ? (uint32_t)g.lds.sdn[idc[c]] : Dn.st[idc[c]];
-      const double a = fma(ddn + dgu + ((stu & sdn & 1u) ? p.u : 0.0), x[c], acc[c]);
+      const double a = fma(ddn[c] + dgu + ((stv & occ >> c & 1u) ? pu : 0.0), x[c], acc[c]);
       const double wk = sj * a - bsp * xp[c];
       w[ro + idc[c]] = wk;
       if (lane + 64 * c < nd) dot += wk * x[c];
@@ -1029,13 +1054,13 @@ __device__ cplx cf_value(const double* a, const double* b, int m, double norm2, 
 // memory: its hops are LDS gathers through the cached lists, and the
 // orthogonalisation against u_j and the norm stay in registers.  A step is
 // then two reductions over the workgroup and the gathers (ground state, 400
-// states: 2.2 us a step against 14 through the L2, where a step is six round
+// states: 2.0 us a step against 14 through the L2, where a step is six round
 // trips; 4,900 states: 6 us against 29, LDS reads).  Hops kept in registers as
 // packed LDS offsets, bond by bond, measured the same step at 400 states and a
 // longer one at 4,900 (a bond without a hop still costs its read).
 // ---------------------------------------------------------------------------
-constexpr int kResGround = 5;  // states per thread: 1024 * 5 >= kLdsRowsSolve
-constexpr int kResFrac = 7;    // 768 * 7
+constexpr int kResGround = 7;  // states per thread: 768 * 7 >= kLdsRowsSolve
+constexpr int kResFrac = 7;
 constexpr int kResHops = 4;    // hops in flight (a half-filled spin sector of 6 or 8 sites has 3 or 4 slots)
 static_assert(kBlockGround * kResGround >= kLdsRowsSolve && kBlockFrac * kResFrac >= kLdsRowsSolve, "resident states");
 
@@ -1419,7 +1444,8 @@ __device__ __noinline__ void combine_psi(const Group<BLOCK>& g, glb_f64* V, cons
 }
 
 template <bool BLOCK, bool FAST>
-__device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, const SlotRef& sl) {
+__device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, SlotRef sl) {
+  sl.base = opaque_uniform(sl.base);  // its pointers are not computed ahead of the task loop and kept
   const ModelParams& p = cf.params[mi];
   const int ns = p.nb + 1;
   const int n_0 = build_list<BLOCK>(g, p, ns, p.n_up, cf.sign_width, sl, 1);
