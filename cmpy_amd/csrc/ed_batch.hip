@@ -1016,6 +1016,9 @@ __device__ __noinline__ void tri_lowest(const Group<BLOCK>& gr, const T* alpha, 
 struct cplx {
   double re, im;
 };
+struct alignas(16) cplx16 {  // one access of 16 bytes
+  double x, y;
+};
 __device__ __forceinline__ cplx cdiv(cplx a, cplx b) {
   // Smith's algorithm
   if (fabs(b.re) >= fabs(b.im)) {
@@ -1099,6 +1102,45 @@ __device__ __forceinline__ void resident_load(const Group<true>& g, const ModelP
   __syncthreads();
 }
 
+// acc plus the hops of state (iu, id) from the vector x in LDS, kResHops at a
+// time: their cached entries, then their states (us, ds: slots per state).
+__device__ __forceinline__ double resident_hops(const BlockLds& L, const lds_f64* x, int iu, int id, int nd, int us,
+                                                int ds, double acc) {
+#pragma unroll 1
+  for (int e0 = 0; e0 < us; e0 += kResHops) {
+    double hv[kResHops], xv[kResHops];
+    int t[kResHops];
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q) {
+      const int e = iu * us + (e0 + q < us ? e0 + q : 0);
+      t[q] = (int)L.utgt[e];
+      hv[q] = L.uval[e];
+    }
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q) xv[q] = x[t[q] * nd + id];
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q)
+      if (e0 + q < us) acc = fma(hv[q], xv[q], acc);
+  }
+#pragma unroll 1
+  for (int e0 = 0; e0 < ds; e0 += kResHops) {
+    double hv[kResHops], xv[kResHops];
+    int t[kResHops];
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q) {
+      const int e = (e0 + q < ds ? e0 + q : 0) * nd + id;
+      t[q] = (int)L.tgt[e];
+      hv[q] = L.val[e];
+    }
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q) xv[q] = x[iu * nd + t[q]];
+#pragma unroll
+    for (int q = 0; q < kResHops; ++q)
+      if (e0 + q < ds) acc = fma(hv[q], xv[q], acc);
+  }
+  return acc;
+}
+
 // One step, as lanczos_step on a sector of D states and nd columns: u_{j+1} =
 // w in place of u_j (LDS and registers), alpha_j and |w|^2 returned.
 template <int S>
@@ -1115,39 +1157,7 @@ __device__ __forceinline__ void resident_step(const Group<true>& g, Resident<S>&
     if (first + s * g.size < D) {  // uniform over the wave
       const int iu = (int)(r.at[s] >> 16), id = (int)(r.at[s] & 0xffffu);
       double acc = r.dg[s] * r.u[s];
-      // four hops at a time: their entries, then their states
-#pragma unroll 1
-      for (int e0 = 0; e0 < us; e0 += kResHops) {
-        double hv[kResHops], x[kResHops];
-        int t[kResHops];
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q) {
-          const int e = iu * us + (e0 + q < us ? e0 + q : 0);
-          t[q] = (int)L.utgt[e];
-          hv[q] = L.uval[e];
-        }
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q) x[q] = L.rows[t[q] * nd + id];
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q)
-          if (e0 + q < us) acc = fma(hv[q], x[q], acc);
-      }
-#pragma unroll 1
-      for (int e0 = 0; e0 < ds; e0 += kResHops) {
-        double hv[kResHops], x[kResHops];
-        int t[kResHops];
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q) {
-          const int e = (e0 + q < ds ? e0 + q : 0) * nd + id;
-          t[q] = (int)L.tgt[e];
-          hv[q] = L.val[e];
-        }
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q) x[q] = L.rows[iu * nd + t[q]];
-#pragma unroll
-        for (int q = 0; q < kResHops; ++q)
-          if (e0 + q < ds) acc = fma(hv[q], x[q], acc);
-      }
+      acc = resident_hops(L, L.rows, iu, id, nd, us, ds, acc);
       const double v = sj * acc - bsp * r.up[s];
       r.up[s] = g.rank + s * g.size < D ? v : 0.0;
       dot = fma(r.up[s], r.u[s], dot);
@@ -1803,57 +1813,271 @@ __device__ __forceinline__ double bond_hops(const SpinList& U, const SpinList& D
 constexpr int kPc = 16;             // W columns per LDS chunk in the backward
 constexpr int kBwdLds = 512 * kPc;  // doubles of the backward's LDS staging buffer (64 KiB)
 constexpr int kBwdMaxSteps = 1024;  // continued-fraction steps a kept basis may hold
-constexpr int kBwdSplitM = 96;      // parts with this many steps run their K products device-wide
+// Parts run their K products device-wide (backward ms, device-wide against one
+// workgroup a model for parts below 96 steps: 4 models x 7 baths 1.8 / 6.4, 64 x
+// 5 1.3 / 1.7, 512 x 5 3.5 / 3.9, 300 x 7 11.9 / 14.2, 16 x 9 54 / 194); those
+// below kBwdSplitM only while the job store leaves half of the free memory.
+constexpr int kBwdSplitM = 96;
 
-// sum_j x[j] y[j] over j < n in order, eight entries' loads in flight at a
-// time (the same sum as one term at a time).
-__device__ __forceinline__ double row_dot(const double* __restrict__ x, const double* __restrict__ y, int n) {
-  double acc = 0.0;
-  int j = 0;
-  for (; j + 8 <= n; j += 8) {
-    double a[8], b[8];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      a[r] = x[j + r];
-      b[r] = y[j + r];
-    }
-#pragma unroll
-    for (int r = 0; r < 8; ++r) acc += a[r] * b[r];
+// u_n = sigma |phi| (sigma z_n + e0 - T)^-1 e1 by a complex Thomas solve, one
+// thread per frequency, into Uc (Ur holds the eliminated right-hand sides).
+// Both are stored frequency-fastest ([i][n], complex), so a step's accesses are
+// whole lines.  The denominators are O(|z| + |T|), far from overflow, so 1/den
+// is taken as conj(den) / |den|^2 (one division per step).  T's coefficients
+// come from LDS (lc, 2 m doubles), and the back substitution reads eight rows
+// at a time: row by row each step waited for its own load (7 baths, two parts,
+// 512 frequencies: 0.09 ms against 0.55).
+__device__ __noinline__ void fraction_columns(const Group<true>& gr, const glb_f64* a, const glb_f64* b, int m, int nw,
+                                              double e0, double sigma, double nphi, const glb_f64* wn, lds_f64* lc,
+                                              glb_f64* Uc, glb_f64* Ur) {
+  typedef __attribute__((address_space(1))) cplx16 glb_c16;
+  const Group<true> g = gr;
+  m = rfl(m);
+  nw = rfl(nw);
+  for (int i = g.rank; i < m; i += g.size) {
+    lc[i] = a[i];
+    lc[m + i] = i < m - 1 ? (double)b[i] : 0.0;
   }
-  for (; j < n; ++j) acc += x[j] * y[j];
-  return acc;
+  __syncthreads();
+  const double sn = sigma * nphi;
+  for (int n = g.rank; n < nw; n += g.size) {
+    glb_c16* const uc = (glb_c16*)Uc + n;
+    glb_c16* const ur = (glb_c16*)Ur + n;
+    const cplx zs = {e0, sigma * wn[n]};
+    cplx cp = {0.0, 0.0}, rp = {0.0, 0.0};
+    double offl = 0.0;
+    for (int i = 0; i < m; ++i) {
+      const double bi = lc[m + i];
+      const cplx den = {zs.re - lc[i] - offl * cp.re, zs.im - offl * cp.im};
+      const double s2 = 1.0 / (den.re * den.re + den.im * den.im);
+      const cplx inv = {den.re * s2, -den.im * s2};
+      const cplx ci = {-bi * inv.re, -bi * inv.im};
+      const cplx ri = cmul({(i == 0 ? 1.0 : 0.0) - offl * rp.re, -offl * rp.im}, inv);
+      uc[(int64_t)i * nw].x = ci.re;
+      uc[(int64_t)i * nw].y = ci.im;
+      ur[(int64_t)i * nw].x = ri.re;
+      ur[(int64_t)i * nw].y = ri.im;
+      cp = ci;
+      rp = ri;
+      offl = -bi;
+    }
+    cplx x = rp;
+    uc[(int64_t)(m - 1) * nw].x = sn * x.re;
+    uc[(int64_t)(m - 1) * nw].y = sn * x.im;
+    for (int i0 = m - 2; i0 >= 0; i0 -= 8) {
+      cplx cv[8], rv[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const int64_t at = (int64_t)(i0 - q >= 0 ? i0 - q : 0) * nw;
+        cv[q] = {uc[at].x, uc[at].y};
+        rv[q] = {ur[at].x, ur[at].y};
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (i0 - q >= 0) {
+          const cplx t = cmul(cv[q], x);
+          x = {rv[q].re - t.re, rv[q].im - t.im};
+          uc[(int64_t)(i0 - q) * nw].x = sn * x.re;
+          uc[(int64_t)(i0 - q) * nw].y = sn * x.im;
+        }
+    }
+  }
+  g.sync();
 }
 
-// <p, y1> and <p, y2> (y2 may be null: its sum stays 0) in order, p's loads
-// shared, eight entries of each in flight at a time.
-__device__ __forceinline__ void row_dot2(const double* __restrict__ x, const double* __restrict__ y1,
-                                         const double* __restrict__ y2, int n, double* s1, double* s2) {
-  double a1 = 0.0, a2 = 0.0;
-  int j = 0;
-  if (y2) {
-    for (; j + 8 <= n; j += 8) {
-      double xv[8], v1[8], v2[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        xv[r] = x[j + r];
-        v1[r] = y1[j + r];
-        v2[r] = y2[j + r];
+// Sums over rows r of a part's K = P Qt^T: tr K, S_eps[k] = sum occ_k(r) K_rr and
+// S_V[k] = sum of sign * K_{r, t(r)} over the hops r -> t of bond k.  Only sums
+// over the rows are wanted, so a wavefront takes a row at a time, a Krylov
+// index a lane (whole lines of P and Qt, and no reduction per product), and
+// every lane keeps its own sums over its rows to the end.  A row's hops come
+// from its index, bond k's up hop on lane k and its dn hop on lane 32 + k.
+constexpr int kBondsPerPass = 8;
+struct BondSums {
+  double tr = 0.0, se[kBondsPerPass] = {}, sv[kBondsPerPass] = {};
+};
+struct PartRows {  // the part's sector and stores
+  int ns, n_up, n_dn, nd, nb, width, m, ldp, ldq;
+};
+__device__ __forceinline__ void bond_rows(const PartRows& w, const glb_f64* P, const glb_f64* Q, int r0, int r1,
+                                          int step, int k0, BondSums& b) {
+  const int lane = (int)(threadIdx.x & 63), bond = lane & 31;
+  for (int j0 = 0; j0 < w.m; j0 += 64) {
+    const bool on = j0 + lane < w.m;
+    const int j = on ? j0 + lane : w.m - 1;
+    for (int r = r0; r < r1; r += step) {
+      const int iu = r / w.nd, id = r - iu * w.nd;
+      const double pl = P[(int64_t)r * w.ldp + j], ql = Q[(int64_t)r * w.ldq + j];
+      const uint32_t su = comb_unrank(iu, w.ns, w.n_up), sd = comb_unrank(id, w.ns, w.n_dn);
+      int hop = -1;  // 2 target + (sign < 0)
+      {
+        const uint32_t s = lane < 32 ? su : sd, mask = 1u | (2u << bond), at = s & mask;
+        if (bond < w.nb && at != 0 && at != mask) {
+          const int t = (int)comb_rank(s ^ mask);
+          hop = 2 * (lane < 32 ? t * w.nd + id : iu * w.nd + t) + (hop_sign(s, w.width, 0, bond + 1) < 0 ? 1 : 0);
+        }
       }
+      int hu[kBondsPerPass], hd[kBondsPerPass];
+      double xu[kBondsPerPass], xd[kBondsPerPass];
 #pragma unroll
-      for (int r = 0; r < 8; ++r) {
-        a1 += xv[r] * v1[r];
-        a2 += xv[r] * v2[r];
+      for (int k = 0; k < kBondsPerPass; ++k) {  // no hop (and k0 + k >= nb): -1
+        hu[k] = __builtin_amdgcn_readlane(hop, k0 + k);
+        hd[k] = __builtin_amdgcn_readlane(hop, 32 + k0 + k);
+        xu[k] = xd[k] = 0.0;
+        if (hu[k] >= 0) xu[k] = Q[(int64_t)(hu[k] >> 1) * w.ldq + j];
+        if (hd[k] >= 0) xd[k] = Q[(int64_t)(hd[k] >> 1) * w.ldq + j];
+      }
+      const double pv = on ? pl : 0.0, pq = pv * ql;
+      b.tr += pq;
+#pragma unroll
+      for (int k = 0; k < kBondsPerPass; ++k) {
+        b.sv[k] = fma(pv, (hu[k] & 1 ? -xu[k] : xu[k]) + (hd[k] & 1 ? -xd[k] : xd[k]), b.sv[k]);
+        b.se[k] = fma(occ_k(su, sd, k0 + k), pq, b.se[k]);
       }
     }
-    for (; j < n; ++j) {
-      a1 += x[j] * y1[j];
-      a2 += x[j] * y2[j];
-    }
-  } else {
-    a1 = row_dot(x, y1, n);
   }
-  *s1 = a1;
-  *s2 = a2;
+}
+
+// A whole part by one workgroup, to out[0], out[1 + k] and out[1 + kMaxBath + k].
+__device__ __noinline__ void bond_sums(const Group<true>& gr, const PartRows& part, const glb_f64* P, const glb_f64* Q,
+                                       int rows, glb_f64* out) {
+  const Group<true> g = gr;
+  const PartRows w = {rfl(part.ns), rfl(part.n_up), rfl(part.n_dn), rfl(part.nd), rfl(part.nb),
+                      rfl(part.width), rfl(part.m), rfl(part.ldp), rfl(part.ldq)};
+  rows = rfl(rows);
+  for (int k0 = 0; k0 < w.nb; k0 += kBondsPerPass) {
+    BondSums b;
+    bond_rows(w, P, Q, rfl(g.rank >> 6), rows, rfl(g.size >> 6), k0, b);
+    if (k0 == 0) {
+      const double s = g.sum(b.tr);
+      if (g.rank == 0) out[0] = s;
+    }
+#pragma unroll
+    for (int k = 0; k < kBondsPerPass; ++k) {
+      if (k0 + k < w.nb) {
+        const double s1 = g.sum(b.se[k]), s2 = g.sum(b.sv[k]);
+        if (g.rank == 0) {
+          out[1 + k0 + k] = s1;
+          out[1 + kMaxBath + k0 + k] = s2;
+        }
+      }
+    }
+  }
+  g.sync();
+}
+
+// The projected conjugate gradients of backward_model on a sector held on chip:
+// p in LDS (buf), each thread its states' p, residual, solution and psi in
+// registers, q = (H - E0) p by LDS gathers; four barriers an iteration (4,900
+// states: 7 us against 31 through the L2).  zeta is written at the end; the
+// iteration count is returned.
+constexpr int kResBwd = 5;  // states per thread
+__device__ __noinline__ int cg_resident(const Group<true>& gr, const ModelParams& p, const SpinList& U,
+                                        const SpinList& Dn, lds_f64* buf, double e0, const glb_f64* psi,
+                                        const glb_f64* res, glb_f64* zeta, int cg_max, double cg_tol, double rho) {
+  Group<true> g = gr;
+  g.size = rfl(gr.size);
+  const BlockLds L = g.lds;
+  const int nd = rfl(Dn.n), D = rfl(U.n) * nd;
+  const int us = rfl(L.umeta[1]), ds = rfl(L.meta[1]);
+  const int first = rfl(g.rank & ~63);
+  const int nw = (D < g.size ? D + 63 : g.size) >> 6;
+  double pv[kResBwd], rv[kResBwd], zv[kResBwd], ps[kResBwd], dg[kResBwd], qv[kResBwd];
+  uint32_t at[kResBwd];
+#pragma unroll
+  for (int s = 0; s < kResBwd; ++s) {
+    const int k = g.rank + s * g.size;
+    const bool act = k < D;
+    const int kc = act ? k : 0;
+    const int iu = kc / nd, id = kc - iu * nd;
+    at[s] = (uint32_t)iu << 16 | (uint32_t)id;
+    dg[s] = U.dg[iu] + Dn.dg[id] + ((U.st[iu] & Dn.st[id] & 1u) ? p.u : 0.0) - e0;
+    pv[s] = rv[s] = act ? (double)res[kc] : 0.0;
+    ps[s] = act ? (double)psi[kc] : 0.0;
+    zv[s] = 0.0;
+    if (act) buf[k] = pv[s];
+  }
+  __syncthreads();
+  const double rho0 = rho;
+  int it = 0;
+  for (; it < cg_max && rho > cg_tol * cg_tol * rho0 && rho > 0.0; ++it) {
+    double qp = 0.0, qpsi = 0.0;
+#pragma unroll
+    for (int s = 0; s < kResBwd; ++s) {
+      qv[s] = 0.0;
+      if (first + s * g.size < D) {  // uniform over the wave
+        const double v = resident_hops(L, buf, (int)(at[s] >> 16), (int)(at[s] & 0xffffu), nd, us, ds, dg[s] * pv[s]);
+        qv[s] = g.rank + s * g.size < D ? v : 0.0;
+        qp = fma(qv[s], pv[s], qp);
+        qpsi = fma(qv[s], ps[s], qpsi);
+      }
+    }
+    qp = g.template sum_half<0>(qp, nw);
+    qpsi = g.template sum_half<1>(qpsi, nw);
+    const double alpha = rho / qp;
+    double rn = 0.0;
+#pragma unroll
+    for (int s = 0; s < kResBwd; ++s) {
+      const double q = qv[s] - qpsi * ps[s];
+      zv[s] = fma(alpha, pv[s], zv[s]);
+      rv[s] = rv[s] - alpha * q;
+      rn = fma(rv[s], rv[s], rn);
+    }
+    rn = g.template sum_half<0>(rn, nw);  // (the second sum's barrier lies between)
+    const double beta = rn / rho;
+    rho = rn;
+#pragma unroll
+    for (int s = 0; s < kResBwd; ++s) {
+      const int k = g.rank + s * g.size;
+      pv[s] = rv[s] + beta * pv[s];
+      if (k < D) buf[k] = pv[s];  // every gather from p lies before the sums' barriers
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int s = 0; s < kResBwd; ++s) {
+    const int k = g.rank + s * g.size;
+    if (k < D) zeta[k] = zv[s];
+  }
+  g.sync();
+  return it;
+}
+
+// The same through memory.  up: a vector's room that the step may name (its
+// factor is zero).
+__device__ __noinline__ int cg_memory(const Group<true>& g, const ModelParams& p, const SpinList& U,
+                                      const SpinList& Dn, double e0, const glb_f64* psi, glb_f64* res, glb_f64* zeta,
+                                      glb_f64* pv, glb_f64* qv, const glb_f64* up, int cg_max, double cg_tol,
+                                      double rho) {
+  const int64_t D = (int64_t)U.n * Dn.n;
+  const double rho0 = rho;
+  int it = 0;
+  for (; it < cg_max && rho > cg_tol * cg_tol * rho0 && rho > 0.0; ++it) {
+    double aj, nn;
+    lanczos_step<true>(g, p, U, Dn, pv, up, qv, 1.0, 0.0, 0.0, true, e0, &aj, &nn);  // q = (H - E0) p
+    double qp = 0.0, qpsi = 0.0;
+    for (int64_t k = g.rank; k < D; k += g.size) {
+      qp += qv[k] * pv[k];
+      qpsi += qv[k] * psi[k];
+    }
+    qp = g.sum(qp);
+    qpsi = g.sum(qpsi);
+    const double alpha = rho / qp;
+    double rn = 0.0;
+    for (int64_t k = g.rank; k < D; k += g.size) {
+      const double q = qv[k] - qpsi * psi[k];
+      zeta[k] += alpha * pv[k];
+      const double r = res[k] - alpha * q;
+      res[k] = r;
+      rn += r * r;
+    }
+    rn = g.sum(rn);
+    g.sync();
+    const double beta = rn / rho;
+    rho = rn;
+    for (int64_t k = g.rank; k < D; k += g.size) pv[k] = res[k] + beta * pv[k];
+    g.sync();
+  }
+  return it;
 }
 
 __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi, const BwdSlot& bs, double* wl) {
@@ -1893,42 +2117,9 @@ __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi
     const double* qt = bc.store_q + bc.off_q[2 * mi + part];
     double* Uc = bs.U(0, nw);   // c' then x
     double* Ur = bs.U(1, nw);   // rhs'
-    // (a) u_n = sigma |phi| (sigma z_n + e0 - T)^-1 e1, complex Thomas, one
-    // thread per frequency; U is stored frequency-fastest ([i][n], complex),
-    // so a step's stores and loads are coalesced over the frequencies.  The
-    // denominators are O(|z| + |T|), far from overflow, so 1/den is taken as
-    // conj(den) / |den|^2 (one division per step)
+    // (a) u_n = sigma |phi| (sigma z_n + e0 - T)^-1 e1
     auto ux = [&](int n, int i) { return 2 * ((int64_t)i * nw + n); };
-    for (int n = g.rank; n < nw; n += g.size) {
-      const cplx zs = {e0, sigma * bc.wn[n]};
-      cplx cp = {0.0, 0.0}, rp = {0.0, 0.0};
-      for (int i = 0; i < m; ++i) {
-        const double offl = i > 0 ? -b[i - 1] : 0.0;
-        const cplx den = {zs.re - a[i] - offl * cp.re, zs.im - offl * cp.im};
-        const double s2 = 1.0 / (den.re * den.re + den.im * den.im);
-        const cplx inv = {den.re * s2, -den.im * s2};
-        const cplx ci = i < m - 1 ? cplx{-b[i] * inv.re, -b[i] * inv.im} : cplx{0.0, 0.0};
-        const cplx ri = cmul({(i == 0 ? 1.0 : 0.0) - offl * rp.re, -offl * rp.im}, inv);
-        Uc[ux(n, i)] = ci.re;
-        Uc[ux(n, i) + 1] = ci.im;
-        Ur[ux(n, i)] = ri.re;
-        Ur[ux(n, i) + 1] = ri.im;
-        cp = ci;
-        rp = ri;
-      }
-      cplx x = rp;
-      Uc[ux(n, m - 1)] = sigma * nphi * x.re;
-      Uc[ux(n, m - 1) + 1] = sigma * nphi * x.im;
-      for (int i = m - 2; i >= 0; --i) {
-        const cplx ci = {Uc[ux(n, i)], Uc[ux(n, i) + 1]};
-        const cplx ri = {Ur[ux(n, i)], Ur[ux(n, i) + 1]};
-        const cplx t = cmul(ci, x);
-        x = {ri.re - t.re, ri.im - t.im};
-        Uc[ux(n, i)] = sigma * nphi * x.re;
-        Uc[ux(n, i) + 1] = sigma * nphi * x.im;
-      }
-    }
-    g.sync();
+    fraction_columns(g, glb(a), glb(b), m, nw, e0, sigma, nphi, glb(bc.wn), (lds_f64*)wl, glb(Uc), glb(Ur));
     // (b) Re W = Re(U diag(gre - i gim) U^T), upper triangle in 4 x 4 tiles
     // (one per thread and pass), frequencies staged through LDS nc at a
     // time as v_in = (gre_n - i gim_n) u_in and u_jn; then ubar
@@ -2140,59 +2331,9 @@ __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi
       __syncthreads();
     }
     g.sync();
-    // (d) diag of K, its trace, and the per-bond sums
-    double* dg = bs.vec(8);
-    double tr = 0.0;
-    for (int64_t r = g.rank; r < Dt; r += g.size) {
-      const double acc = row_dot(P + r * kcap, qt + r * kcap, m);
-      dg[r] = acc;
-      tr += acc;
-    }
-    tr = g.sum(tr);
-    if (g.rank == 0) rec[part * kRecPart] = tr;
-    g.sync();
-    for (int k = 0; k < nb; ++k) {
-      double se = 0.0, sv = 0.0;
-      for (int64_t r = g.rank; r < Dt; r += g.size) {
-        const int iu = (int)(r / nd), id = (int)(r - (int64_t)iu * nd);
-        se += occ_k(T.st[iu], Dn.st[id], k) * dg[r];
-        // the bond's up hop and dn hop from r (at most one each), their dots
-        // with P's row r together; summed as one hop after the other
-        int64_t t0 = -1, t1 = -1;
-        double g0 = 0.0, g1 = 0.0;
-        for (int e = 0; e < T.cnt[iu]; ++e) {
-          const uint32_t t = (uint32_t)T.tgt[iu * kMaxBath + e];
-          if ((int)((t >> 16) & 0xff) != k) continue;
-          g0 = (t & 0x80000000u) ? -1.0 : 1.0;
-          t0 = (int64_t)(t & 0xffff) * nd + id;
-        }
-        for (int e = 0; e < Dn.cnt[id]; ++e) {
-          const uint32_t t = (uint32_t)Dn.tgt[id * kMaxBath + e];
-          if ((int)((t >> 16) & 0xff) != k) continue;
-          g1 = (t & 0x80000000u) ? -1.0 : 1.0;
-          t1 = (int64_t)iu * nd + (t & 0xffff);
-        }
-        if (t0 < 0) {  // dn hop only: it takes the first slot
-          t0 = t1;
-          g0 = g1;
-          t1 = -1;
-        }
-        if (t0 >= 0) {
-          double d0, d1;
-          row_dot2(P + r * kcap, qt + t0 * kcap, t1 >= 0 ? qt + t1 * kcap : nullptr, m, &d0, &d1);
-          double sb = g0 * d0;
-          if (t1 >= 0) sb += g1 * d1;
-          sv += sb;
-        }
-      }
-      se = g.sum(se);
-      sv = g.sum(sv);
-      if (g.rank == 0) {
-        rec[part * kRecPart + 1 + k] = se;
-        rec[part * kRecPart + 1 + kMaxBath + k] = sv;
-      }
-      g.sync();
-    }
+    // (d) trace and per-bond sums of K = P Qt^T
+    const PartRows rows{ns, part == 0 ? p.n_up + 1 : p.n_up - 1, p.n_dn, nd, nb, bc.sign_width, m, kcap, kcap};
+    bond_sums(g, rows, glb(P), glb(qt), (int)Dt, glb(rec + part * kRecPart));
   }
   // (f) r = Re(c X + c+ Y) in the N sector, projected off psi
   double* zeta = bs.vec(0);
@@ -2225,34 +2366,14 @@ __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi
   rho = g.sum(rho);
   g.sync();
   // (g) projected conjugate gradients on (H - E0) over the complement of psi
-  const double rho0 = rho;
-  int it = 0;
-  for (; it < bc.cg_max && rho > bc.cg_tol * bc.cg_tol * rho0 && rho > 0.0; ++it) {
-    double aj, nn;
-    lanczos_step<true>(g, p, U0, Dn, glb(pv), glb(bs.vec(8)), glb(qv), 1.0, 0.0, 0.0, true, e0, &aj, &nn);  // q = (H - E0) p
-    double qp = 0.0, qpsi = 0.0;
-    for (int64_t k = g.rank; k < D; k += g.size) {
-      qp += qv[k] * pv[k];
-      qpsi += qv[k] * psi[k];
-    }
-    qp = g.sum(qp);
-    qpsi = g.sum(qpsi);
-    const double alpha = rho / qp;
-    double rn = 0.0;
-    for (int64_t k = g.rank; k < D; k += g.size) {
-      const double q = qv[k] - qpsi * psi[k];
-      zeta[k] += alpha * pv[k];
-      const double r = res[k] - alpha * q;
-      res[k] = r;
-      rn += r * r;
-    }
-    rn = g.sum(rn);
-    g.sync();
-    const double beta = rn / rho;
-    rho = rn;
-    for (int64_t k = g.rank; k < D; k += g.size) pv[k] = res[k] + beta * pv[k];
-    g.sync();
-  }
+  const bool resident = g.has_lds && g.wave_rows && D <= (int64_t)kResBwd * g.size && D <= kBwdLds &&
+                        g.lds.meta[0] == nd && up_cached(g, U0);
+  int it;
+  if (resident)
+    it = cg_resident(g, p, U0, Dn, (lds_f64*)wl, e0, glb(psi), glb(res), glb(zeta), bc.cg_max, bc.cg_tol, rho);
+  else
+    it = cg_memory(g, p, U0, Dn, e0, glb(psi), glb(res), glb(zeta), glb(pv), glb(qv), glb(bs.vec(8)), bc.cg_max,
+                   bc.cg_tol, rho);
   // (h) dE0/dtheta and psi^T dH zeta, (i) the gradient
   for (int k = 0; k < nb; ++k) {
     double de = 0.0, te = 0.0, dv = 0.0, tv = 0.0;
@@ -2370,63 +2491,34 @@ __global__ __launch_bounds__(256) void k_bwd_gemm(const BwdGemm* __restrict__ ge
       }
 }
 
-// <x, y> over n entries, lanes striding the entries, the same value on every
-// lane (fixed order).
-__device__ __forceinline__ double wave_dot(const double* __restrict__ x, const double* __restrict__ y, int n) {
-  double s = 0.0;
-  for (int j = (int)(threadIdx.x & 63); j < n; j += 64) s += x[j] * y[j];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  return s;
-}
-
-// diag(K) = rows of P . rows of Qt, its trace, S_eps[k] = sum occ_k diag(K)
-// and S_v[k] = sum over the hops of bond k of K[a, t] (with the hop signs)
-// over one 64-row block of one job: a wave per row in turn, states and hops
-// regenerated from the row index (the same hops as the spin lists hold);
-// the block's sums, wave by wave in order, go to its partial record.
+// The same over one 64-row block of one job, four waves; the block's sums, wave
+// by wave in order, go to its partial record.  128 parts of 7-bath models take
+// 0.84 ms (with a wave-wide reduction per product 2.5 ms more).
 __global__ __launch_bounds__(256) void k_bwd_sums(BwdConfig bc) {
   __shared__ double red[4][kRecPart];
   const BwdBlock bl = bc.blocks[blockIdx.x];
   const BwdJob jb = bc.jobs[bl.job];
   const ModelParams& p = bc.params[jb.model];
   const int ns = p.nb + 1, nb = p.nb;
-  const int n_t = p.n_up + (jb.part == 0 ? 1 : -1);
-  const int nd = (int)binom_u(ns, p.n_dn);
-  const int m = jb.m, kcap = bc.kcap;
-  const double* __restrict__ P = bc.jstore + jb.p_off;
-  const double* __restrict__ Q = bc.store_q + jb.q_off;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  double acc[kRecPart];  // uniform over the wave
+  const PartRows w{ns, p.n_up + (jb.part == 0 ? 1 : -1), p.n_dn, (int)binom_u(ns, p.n_dn), nb, bc.sign_width,
+                   jb.m, jb.m, bc.kcap};
+  const int wave = rfl((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+  const int r1 = jb.dt < bl.r0 + 64 ? jb.dt : bl.r0 + 64;
+  if (lane < kRecPart) red[wave][lane] = 0.0;
+  for (int k0 = 0; k0 < nb; k0 += kBondsPerPass) {
+    BondSums b;
+    bond_rows(w, glb((const double*)(bc.jstore + jb.p_off)), glb(bc.store_q + jb.q_off), bl.r0 + wave, r1, 4, k0, b);
+    const double tr = wave_sum(b.tr);
+    if (lane == 0 && k0 == 0) red[wave][0] = tr;
 #pragma unroll
-  for (int t = 0; t < kRecPart; ++t) acc[t] = 0.0;
-  for (int rr = wave; rr < 64; rr += 4) {
-    const int64_t r = (int64_t)bl.r0 + rr;
-    if (r >= jb.dt) break;
-    const int it = (int)(r / nd), id = (int)(r - (int64_t)it * nd);
-    const uint32_t st = comb_unrank(it, ns, n_t), sd = comb_unrank(id, ns, p.n_dn);
-    const double* pr = P + r * m;
-    const double dg = wave_dot(pr, Q + r * kcap, m);
-    acc[0] += dg;
-    for (int k = 0; k < nb; ++k) {
-      acc[1 + k] += occ_k(st, sd, k) * dg;
-      const uint32_t mk = 1u | (2u << k);
-      double sv = 0.0;
-      const uint32_t bu = st & mk;
-      if (bu != 0 && bu != mk) {
-        const double sg = hop_sign(st, bc.sign_width, 0, k + 1) < 0 ? -1.0 : 1.0;
-        sv += sg * wave_dot(pr, Q + ((int64_t)comb_rank(st ^ mk) * nd + id) * kcap, m);
+    for (int k = 0; k < kBondsPerPass; ++k) {
+      const double se = wave_sum(b.se[k]), sv = wave_sum(b.sv[k]);
+      if (lane == 0 && k0 + k < nb) {
+        red[wave][1 + k0 + k] = se;
+        red[wave][1 + kMaxBath + k0 + k] = sv;
       }
-      const uint32_t bd = sd & mk;
-      if (bd != 0 && bd != mk) {
-        const double sg = hop_sign(sd, bc.sign_width, 0, k + 1) < 0 ? -1.0 : 1.0;
-        sv += sg * wave_dot(pr, Q + ((int64_t)it * nd + comb_rank(sd ^ mk)) * kcap, m);
-      }
-      acc[1 + kMaxBath + k] += sv;
     }
   }
-  if (lane == 0)
-    for (int t = 0; t < kRecPart; ++t) red[wave][t] = acc[t];
   __syncthreads();
   for (int t = threadIdx.x; t < kRecPart; t += blockDim.x)
     bc.partial[(int64_t)blockIdx.x * kRecPart + t] = ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
@@ -2436,49 +2528,43 @@ __global__ __launch_bounds__(256) void k_bwd_sums(BwdConfig bc) {
 // the blocks' partial sums (in block order):
 //   dL/deps_k = sum_parts s_part S_eps[k] + (trK_hole - trK_particle) dE0/deps_k - 2 psi dH/deps_k zeta,
 // the same for v_k with S_v.
-__global__ void k_bwd_combine(BwdConfig bc) {
-  const int mi = blockIdx.x * blockDim.x + threadIdx.x;
-  if (mi >= bc.num_models) return;
+// A wavefront a model, one record entry a lane, eight blocks' loads in flight
+// (a thread a model: 0.26 ms at 62 blocks a part).
+__global__ __launch_bounds__(64) void k_bwd_combine(BwdConfig bc) {
+  __shared__ double sums[2][kRecPart];
+  const int mi = blockIdx.x, lane = threadIdx.x;
   const ModelParams& p = bc.params[mi];
   const double* rec = bc.rec + (int64_t)mi * kRec;
   const double* rt = rec + 2 * kRecPart;
   const double* co = bc.store_coef + (int64_t)mi * (4 * bc.kcap + 8);
-  double tr[2] = {0.0, 0.0};
   for (int part = 0; part < 2; ++part) {
-    if ((int)co[4 * bc.kcap + 3 + part] <= 0) continue;
-    const int job = bc.job_of[2 * mi + part];
-    if (job < 0) {
-      tr[part] = rec[part * kRecPart];
-    } else {
-      const BwdJob jb = bc.jobs[job];
-      double t = 0.0;
-      for (int b = 0; b < jb.nblk; ++b) t += bc.partial[(int64_t)(jb.blk0 + b) * kRecPart];
-      tr[part] = t;
-    }
-  }
-  for (int k = 0; k < p.nb; ++k) {
-    double se = 0.0, sv = 0.0;
-    for (int part = 0; part < 2; ++part) {
-      if ((int)co[4 * bc.kcap + 3 + part] <= 0) continue;
-      const double sigma = part == 0 ? 1.0 : -1.0;
+    if (lane >= kRecPart) continue;
+    double t = 0.0;
+    if ((int)co[4 * bc.kcap + 3 + part] > 0) {
       const int job = bc.job_of[2 * mi + part];
-      double e, v;
       if (job < 0) {
-        e = rec[part * kRecPart + 1 + k];
-        v = rec[part * kRecPart + 1 + kMaxBath + k];
+        t = rec[part * kRecPart + lane];
       } else {
         const BwdJob jb = bc.jobs[job];
-        e = 0.0;
-        v = 0.0;
-        for (int b = 0; b < jb.nblk; ++b) {
-          e += bc.partial[(int64_t)(jb.blk0 + b) * kRecPart + 1 + k];
-          v += bc.partial[(int64_t)(jb.blk0 + b) * kRecPart + 1 + kMaxBath + k];
+        const double* x = bc.partial + (int64_t)jb.blk0 * kRecPart + lane;
+        for (int b0 = 0; b0 < jb.nblk; b0 += 8) {
+          double v[8];
+#pragma unroll
+          for (int q = 0; q < 8; ++q) v[q] = x[(int64_t)(b0 + q < jb.nblk ? b0 + q : b0) * kRecPart];
+#pragma unroll
+          for (int q = 0; q < 8; ++q)
+            if (b0 + q < jb.nblk) t += v[q];
         }
       }
-      se += sigma * e;
-      sv += sigma * v;
     }
-    const double ba = tr[1] - tr[0];
+    sums[part][lane] = t;
+  }
+  __syncthreads();
+  const double ba = sums[1][0] - sums[0][0];
+  if (lane < p.nb) {
+    const int k = lane;
+    const double se = sums[0][1 + k] - sums[1][1 + k];
+    const double sv = sums[0][1 + kMaxBath + k] - sums[1][1 + kMaxBath + k];
     bc.grad_eps[(int64_t)mi * bc.max_bath + k] = se + ba * rt[k] - 2.0 * rt[kMaxBath + k];
     bc.grad_v[(int64_t)mi * bc.max_bath + k] = sv + ba * rt[2 * kMaxBath + k] - 2.0 * rt[3 * kMaxBath + k];
   }
@@ -2871,7 +2957,7 @@ extern "C" int ed_batch_create(ed_batch** out, const ed_batch_desc* d, void* str
   if ((rc = balloc(&b->d_params, d->num_models)) != ED_OK || (rc = balloc(&b->d_queues, d->num_models)) != ED_OK ||
       (rc = balloc(&b->d_counters, 4)) != ED_OK || (rc = balloc(&b->d_e0, d->num_models)) != ED_OK ||
       (rc = balloc(&b->d_iters, 3 * d->num_models)) != ED_OK || (rc = balloc(&b->d_resid, 2 * d->num_models)) != ED_OK ||
-      (rc = balloc(&b->d_store_coef, d->num_models * (4 * (int64_t)d->cf_steps + 8))) != ED_OK) {
+      (rc = balloc(&b->d_store_coef, d->num_models * (4 * (int64_t)b->kcap + 8))) != ED_OK) {
     free_batch(b);
     return rc;
   }
@@ -3128,10 +3214,9 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   }
   ED_HIP(hipMemcpyAsync(b->d_gre, dl_dre, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
   ED_HIP(hipMemcpyAsync(b->d_gim, dl_dim, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
-  // parts with at least split_m continued-fraction steps run their K
-  // products device-wide (CMPY_AMD_BWD_SPLIT_M; the per-model workgroup
-  // would spend O(D m^2) on them alone)
-  const int split_m = env_flag("CMPY_AMD_BWD_SPLIT_M", kBwdSplitM);
+  // parts with at least split_m continued-fraction steps run their K products
+  // device-wide (CMPY_AMD_BWD_SPLIT_M)
+  const int split_m = env_flag("CMPY_AMD_BWD_SPLIT_M", 1);
   std::vector<int32_t> iters(3 * M);
   ED_HIP(hipMemcpy(iters.data(), b->d_iters, sizeof(int32_t) * 3 * M, hipMemcpyDeviceToHost));
   std::vector<int32_t> job_of(2 * M, -1);
@@ -3140,6 +3225,8 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   std::vector<BwdTile> tiles_w, tiles;        // their tiles
   std::vector<BwdBlock> blocks;
   int64_t jst = 0;
+  int64_t room = b->cap_jstore;  // doubles a short part may fill the job store to
+  bool asked = false;
   for (int64_t i = 0; i < M; ++i) {
     const ModelParams& p = b->params[i];
     const int ns = p.nb + 1;
@@ -3152,6 +3239,14 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
       jb.part = part;
       jb.m = m;
       jb.dt = (int32_t)sector_dim(ns, n_t, p.n_dn);
+      const int64_t need = 4ll * m * nw + (int64_t)m * m + (int64_t)jb.dt * m;
+      if (m < kBwdSplitM && jst + need > room) {
+        size_t free_b = 0, total_b = 0;
+        if (!asked && hipMemGetInfo(&free_b, &total_b) == hipSuccess)
+          room = b->cap_jstore + (int64_t)(free_b / (2 * sizeof(double)));
+        asked = true;
+        if (jst + need > room) continue;
+      }
       jb.q_off = b->h_off_q[2 * i + part];
       jb.a_off = jst;
       jst += 2ll * m * nw;
@@ -3256,7 +3351,7 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
                        (const BwdTile*)(b->d_tiles + tiles_w.size()), (const double*)b->d_store_q, b->d_jstore);
     hipLaunchKernelGGL(k_bwd_sums, dim3((unsigned)blocks.size()), dim3(256), 0, s, bc);
   }
-  hipLaunchKernelGGL(k_bwd_combine, dim3((unsigned)((M + 63) / 64)), dim3(64), 0, s, bc);
+  hipLaunchKernelGGL(k_bwd_combine, dim3((unsigned)M), dim3(64), 0, s, bc);
   const hipError_t el = hipGetLastError();
   (void)hipEventRecord(e1, s);
   const hipError_t es = hipEventSynchronize(e1);
