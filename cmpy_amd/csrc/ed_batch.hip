@@ -1342,6 +1342,12 @@ struct CfTrack {
 };
 
 // cf_coeffs on a resident sector.
+// KEEP: the basis goes to qt, a row a state, kHeld steps at a time: a step's
+// entries lie in as many lines as there are states, which left the L2 before
+// the next step came to them (64 models x 7 baths: 1.57 ms against 1.95; more
+// steps do not fit the registers).
+constexpr int kHeld = 2;
+template <bool KEEP>
 __device__ __noinline__ int cf_resident(const Group<true>& gr, const ModelParams& p, const SpinList& U,
                                         const SpinList& Dn, const glb_f64* u0, double n2, int cap, double e0,
                                         double sgn, double wmin, double cf_tol, glb_f64* a, glb_f64* b, glb_f64* qt,
@@ -1354,13 +1360,28 @@ __device__ __noinline__ int cf_resident(const Group<true>& gr, const ModelParams
   CfTrack track;
   cap = rfl(cap);
   double sj = 1.0 / sqrt(n2), sp = 0.0, bj = 0.0;
+  double held[kResFrac][kHeld - 1];  // (the last of them is u_j itself)
   for (int j = 0;; ++j) {
-    if (qt) {
+    const int h = j % kHeld;
+    if (KEEP) {
+      if (h == kHeld - 1) {
 #pragma unroll
-      for (int s = 0; s < kResFrac; ++s) {
-        const int k = g.rank + s * g.size;
-        if (k < D) qt[(int64_t)k * kcap + j] = sj * r.u[s];
+        for (int s = 0; s < kResFrac; ++s) {
+          const int k = g.rank + s * g.size;
+          if (k < D) {
+            glb_f64* const q = qt + (int64_t)k * kcap + (j - (kHeld - 1));
+#pragma unroll
+            for (int t = 0; t < kHeld - 1; ++t) q[t] = held[s][t];
+            q[kHeld - 1] = sj * r.u[s];
+          }
+        }
       }
+#pragma unroll
+      for (int t = 0; t < kHeld - 1; ++t)
+        if (h == t) {
+#pragma unroll
+          for (int s = 0; s < kResFrac; ++s) held[s][t] = sj * r.u[s];
+        }
     }
     double aj, nn;
     resident_step(g, r, D, nd, sj, sp, bj, &aj, &nn);
@@ -1370,8 +1391,18 @@ __device__ __noinline__ int cf_resident(const Group<true>& gr, const ModelParams
       a[j] = aj;
       if (!last) b[j] = bn;
     }
-    if (last) return j + 1;
-    if (track.step(j, aj, bj, n2, e0, sgn, wmin, cf_tol)) return j + 1;
+    if (last || track.step(j, aj, bj, n2, e0, sgn, wmin, cf_tol)) {
+      if (KEEP && h < kHeld - 1) {  // the steps still held
+#pragma unroll
+        for (int s = 0; s < kResFrac; ++s) {
+          const int k = g.rank + s * g.size;
+#pragma unroll
+          for (int t = 0; t < kHeld - 1; ++t)
+            if (k < D && t <= h) qt[(int64_t)k * kcap + (j - h + t)] = held[s][t];
+        }
+      }
+      return j + 1;
+    }
     sp = sj;
     sj = 1.0 / bn;
     bj = bn;
@@ -1390,7 +1421,8 @@ __device__ int cf_coeffs(const Group<BLOCK>& g, const ModelParams& p, const Spin
   double* u = sl.vec(1);
   if constexpr (BLOCK && FAST) {
     if (resident_fits(g, U, Dn))
-      return cf_resident(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap);
+      return qt ? cf_resident<true>(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap)
+                : cf_resident<false>(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap);
   }
   double* up = sl.vec(0);
   double* w = sl.vec(2);
