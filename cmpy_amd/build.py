@@ -37,8 +37,8 @@ CFLAGS = [
 LDFLAGS = ["-shared", f"-L{ROCM}/lib", "-lrocsolver", "-lrocblas"]
 
 # Largest private (scratch) size per lane a kernel may compile to.  The
-# persistent batch kernels (1024-thread workgroups, one per CU slot) run at
-# 240-304 bytes/lane; two builds that spilled to ~1.37 KB/lane (164-166
+# persistent batch kernels (768- and 1024-thread workgroups, one per CU slot) run at
+# 456-492 bytes/lane, mostly call frames; two builds that spilled to ~1.37 KB/lane (164-166
 # spilled VGPRs) faulted on MI355X with a memory-aperture violation, while the
 # same code run on the CPU under AddressSanitizer (tests/cpu_kernels) stays in
 # bounds.  A build past this limit is refused rather than shipped.

@@ -22,8 +22,9 @@
 // the ground-state tasks (one per model), then the continued-fraction tasks
 // (particle and hole of each model, two tasks), so a model's two fractions
 // run on two groups at once; a last small kernel sums G from each model's
-// coefficient record.  All vectors and spin tables of a group live in its slot
-// of a global workspace (L1/L2-resident for these sizes); Lanczos scalars are
+// coefficient record.  The spin tables of a group live in its slot of a global
+// workspace, and so do its vectors (L2-resident for these sizes) unless block
+// mode holds the sector on chip (up to 4,904 states); Lanczos scalars are
 // reduced in a fixed order, so results are deterministic for a given
 // configuration.  The ground-state Lanczos vectors of every model are kept
 // in a store of their own ((max_iter + 1) D doubles per model), so psi is
