@@ -639,25 +639,30 @@ __global__ __launch_bounds__(kRowThreads) void k_hv_rows_held(Hv2Args a, int row
 // Single fused pass on staged rows: a block stages RB rows of x in LDS and
 // each of its waves takes 64-column chunks of them.  Up hops are read from x
 // itself (one list per row, wave-uniform: scalar loads; every hop a contiguous
-// 64-column piece of another row, eight in flight), dn hops are LDS gathers
-// through the packed column-major table, whose entries serve all RB rows.
-// Blocks go to XCDs in contiguous runs of rows, whose hop sources lie mostly
-// near them.  blockIdx.y picks the vector.  Every wave has a chunk (at most
-// nch waves a block).
+// 64-column piece of another row, UP of them in flight a row), dn hops are LDS
+// gathers through the packed column-major table, whose entries serve all RB
+// rows.  Slots past a state's count take nothing from x, so that an infinity
+// reaches only the entries that H couples to it: an up slot is branched over (a
+// row's count is uniform; another hop's address in its place also cost its
+// load, as much as half of a star's, whose rows have 3 and 13 hops: 13-site
+// impurity (4,5) 24.0 us, 16.5 without), a dn slot gathers the zero past its
+// row.  Blocks go to XCDs in contiguous runs of rows, whose hop sources lie
+// mostly near them.  blockIdx.y picks the vector.  Every wave has a chunk (at
+// most nch waves a block).
 // ---------------------------------------------------------------------------
 constexpr int kTileDn = 4;  // dn slots per step; the next step's entries are loaded ahead
 
 template <int RB, bool UNI, bool LZ>
 __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __restrict__ x, double* __restrict__ y,
                                                   HvEpilogue e, int nrg, int per_xcd, int64_t vstride) {
-  extern __shared__ double rows[];  // [RB][nd]
+  extern __shared__ double rows[];  // [RB][nd + 1], a zero past each row
   __shared__ double red[32];
   const int rg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
   if (rg >= nrg) {  // the whole block
     if (LZ && e.partial && threadIdx.x == 0) e.partial[blockIdx.x] = 0.0;
     return;
   }
-  const int nd = (int)a.nd, nt = (int)blockDim.x;
+  const int nd = (int)a.nd, nt = (int)blockDim.x, rs = nd + 1;
   const int64_t ld = a.ld;
   const int r0 = rg * RB;
   const int R = (int)a.nu - r0 < RB ? (int)a.nu - r0 : RB;
@@ -668,8 +673,9 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
 #pragma unroll
     for (int r = 0; r < RB; ++r) v[r] = x[(int64_t)(r0 + (r < R ? r : 0)) * ld + k];
 #pragma unroll
-    for (int r = 0; r < RB; ++r) rows[r * nd + k] = v[r];
+    for (int r = 0; r < RB; ++r) rows[r * rs + k] = v[r];
   }
+  if (threadIdx.x < RB) rows[threadIdx.x * rs + nd] = 0.0;
   zero_row_pads(y, r0, R, nd, ld);
   const double t = UNI ? a.hop[0] : 1.0;
   double sx = 1.0, cp = 0.0, share = 0.0;
@@ -684,7 +690,9 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
   const double cs = LZ && e.cself ? *e.cself : 0.0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  constexpr int UP = RB == 4 ? 4 : 8;  // up hops of a row whose loads are in flight together
+  // up hops of a row whose loads are in flight together (more of them, with
+  // four rows or two, take registers that a second block of the CU needs)
+  constexpr int UP = 8 / RB;
   int cu[RB], cmax = 0;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -708,17 +716,18 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
 #pragma unroll
       for (int r = 0; r < RB; ++r)
 #pragma unroll
-        for (int q = 0; q < UP; ++q) {
-          const int64_t k = (int64_t)(r0 + (r < R ? r : 0)) * a.up_w + (e0 + q < cu[r] ? e0 + q : 0);
-          const uint32_t en = uniform_load(a.up_pk + k);
-          const double h = UNI ? ((en & 0x80000000u) ? -1.0 : 1.0) : uniform_load(a.up_val + k);
-          v[r][q] = e0 + q < cu[r] ? h : 0.0;
-          g[r][q] = (x + (int64_t)hop_target(en) * ld)[ids];
-        }
+        for (int q = 0; q < UP; ++q)
+          if (e0 + q < cu[r]) {  // uniform over the block
+            const int64_t k = (int64_t)(r0 + r) * a.up_w + e0 + q;
+            const uint32_t en = uniform_load(a.up_pk + k);
+            v[r][q] = UNI ? ((en & 0x80000000u) ? -1.0 : 1.0) : uniform_load(a.up_val + k);
+            g[r][q] = (x + (int64_t)hop_target(en) * ld)[ids];
+          }
 #pragma unroll
       for (int r = 0; r < RB; ++r)
 #pragma unroll
-        for (int q = 0; q < UP; ++q) acc[r] = fma(v[r][q], g[r][q], acc[r]);
+        for (int q = 0; q < UP; ++q)
+          if (e0 + q < cu[r]) acc[r] = fma(v[r][q], g[r][q], acc[r]);
     }
     if (first) {  // every wave passes here once
       if (forms) {
@@ -744,31 +753,28 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
       if (!UNI) vl[q] = a.dn_val[k];
     }
     for (int e0 = 0; __ballot(e0 < cnt); e0 += kTileDn) {
-      uint32_t cur[kTileDn];
+      int tg[kTileDn];
       double v[kTileDn];
 #pragma unroll
       for (int q = 0; q < kTileDn; ++q) {
-        cur[q] = en[q];
-        const double h = UNI ? ((en[q] & 0x80000000u) ? -1.0 : 1.0) : vl[q];
-        v[q] = e0 + q < cnt ? h : 0.0;
+        tg[q] = e0 + q < cnt ? hop_target(en[q]) : nd;
+        v[q] = UNI ? ((en[q] & 0x80000000u) ? -1.0 : 1.0) : vl[q];
         const int n = e0 + kTileDn + q;
         const int64_t k = (int64_t)(n < w1 ? n : w1) * nd + ids;
         en[q] = a.dn_pk[k];
         if (!UNI) vl[q] = a.dn_val[k];
       }
 #pragma unroll
-      for (int q = 0; q < kTileDn; ++q) {
-        const int tg = hop_target(cur[q]);
+      for (int q = 0; q < kTileDn; ++q)
 #pragma unroll
-        for (int r = 0; r < RB; ++r) acc[r] = fma(v[q], rows[r * nd + tg], acc[r]);
-      }
+        for (int r = 0; r < RB; ++r) acc[r] = fma(v[q], rows[r * rs + tg[q]], acc[r]);
     }
 #pragma unroll
     for (int r = 0; r < RB; ++r) {
       if (r < R && act) {
         const int iu = r0 + r;
         const int64_t k = (int64_t)iu * ld + id;
-        const double xo = rows[r * nd + id];
+        const double xo = rows[r * rs + id];
         const double h = (a.d_up[iu] + ddn + u_term2(a, a.st_up[iu] & sdn)) * xo + t * acc[r];
         if (LZ) {
           double v = sx * (h - cs * xo);
@@ -1549,10 +1555,12 @@ constexpr int64_t kTileWaves = 2048;    // waves that keep the chip busy (2 per 
 constexpr size_t kTileLds = 64 * 1024;  // granted without an attribute, and two blocks fit a CU
 constexpr int kTileMaxThreads = 1024;
 
-// Rows per block: as many as keep kTileWaves waves in flight, up to four (the
-// dn table's entries are read once for all of a block's rows; 12-site chain:
-// 14.1 us with four rows, 15.2 with two, 16.7 with one).
-
+// Rows per block: as many as keep kTileWaves waves in flight, up to four where
+// a block has 14 waves or more and two below (the dn table's entries are read
+// once for all of a block's rows, but four rows leave registers for 20 waves a
+// CU, so that a block of 11 or 12 is alone on it: 13-site chain (6,5) 33.6 us
+// with four, 30.7 with two, (5,4) 17.1 and 12.6; 4x4 (4,4), 15 waves, 56.4 and
+// 59.9; 12-site chain (6,6), 15 waves, 13.0 and 13.2).
 static TilePlan plan_tile(const ed_op* op) {
   TilePlan p{};
   if (!op->packed || op->size == 0) return p;
@@ -1560,10 +1568,10 @@ static TilePlan plan_tile(const ed_op* op) {
   const int64_t iters = (nch + kTileMaxThreads / 64 - 1) / (kTileMaxThreads / 64);
   const int64_t waves = (nch + iters - 1) / iters;
   p.threads = (int)waves * 64;
-  p.rb = 4;
+  p.rb = waves >= 14 ? 4 : 2;
   for (; p.rb > 1; p.rb /= 2)
-    if (p.rb * op->num_dn * sizeof(double) <= kTileLds - 256 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
-  p.lds_bytes = p.rb * op->num_dn * sizeof(double);
+    if (p.rb * (op->num_dn + 1) * sizeof(double) <= kTileLds - 256 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
+  p.lds_bytes = p.rb * (op->num_dn + 1) * sizeof(double);
   if (p.lds_bytes > kTileLds - 256) return p;  // the kernel has static LDS of its own
   p.nrg = (int)((op->num_up + p.rb - 1) / p.rb);
   p.per_xcd = (p.nrg + 7) / 8;

@@ -39,3 +39,30 @@ def test_fused_rows_vs_oracle(gpu, ns, nu, nd, uniform):
     yp = yp.cpu().numpy()
     assert np.all(yp[:, :, op.num_dn:] == 0.0)
     assert np.abs(yp[:, :, :op.num_dn].reshape(nvec, -1) - want).max() <= tol
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ns,nu,nd", [(6, 3, 2), (8, 4, 4), (13, 5, 3), (12, 6, 6)])
+def test_infinities_reach_only_coupled_entries(gpu, ns, nu, nd, uniform):
+    """One infinite entry of x, at the first state of a row (what an unused hop slot names), a hop's source and
+    elsewhere: y is infinite, with the oracle's sign, exactly where H has an element to it, and finite where it has none."""
+    from cmpy_amd import SectorHamiltonOperator
+
+    rng = np.random.default_rng(ns * 10 + nd)
+    bonds = [(0, k) for k in range(1, ns)]  # rows of very different length
+    hops = np.full(len(bonds), -0.7) if uniform else rng.uniform(0.2, 1, len(bonds))
+    eps, u = rng.uniform(-1, 1, ns), rng.uniform(0, 4, ns)
+    op = SectorHamiltonOperator(ns, nu, nd, bonds, hops, eps, u, ns)
+    ref = O.SectorOperator(ns, nu, nd, bonds, hops, eps, u, ns)
+    x = rng.standard_normal(ref.size)
+    tol = 1e-13 * np.abs(ref.matvec(x)).max()
+    row = int(ref.t_up.indices[ref.t_up.indptr[ref.num_up // 2]])
+    for iu, idn in [(0, 0), (row, 0), (ref.num_up - 1, 0), (row, ref.num_dn // 2), (ref.num_up // 2, ref.num_dn - 1)]:
+        xi = x.copy()
+        xi[iu * ref.num_dn + idn] = np.inf
+        want = ref.matvec(xi)
+        got = op.matvec(xi)
+        assert not np.isnan(want).any() and np.isinf(want).any()
+        inf = np.isinf(want)
+        assert np.array_equal(got[inf], want[inf])
+        assert np.abs(got[~inf] - want[~inf]).max() <= tol
