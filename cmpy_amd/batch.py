@@ -107,6 +107,7 @@ class AndersonBatch:
                            float(cf_tol))
         self.keep_basis = bool(keep_basis)
         self.cf_steps_cap = int(cf_steps)
+        self._num_freq = None  # of the last solve
         h = C.c_void_p()
         _lib.call("ed_batch_create", C.byref(h), C.byref(d), _lib.stream_ptr())
         self._h = h
@@ -151,6 +152,7 @@ class AndersonBatch:
         _lib.call("ed_batch_solve", self._h, _ptr(wn, C.c_double), nw, _ptr(e0, C.c_double),
                   _ptr(g, C.c_double), _ptr(it, C.c_int32), _ptr(res, C.c_double), C.byref(ms),
                   _lib.stream_ptr())
+        self._num_freq = nw
         steps = it[:, 1:].copy()
         capped = steps >= self.cf_steps_cap
         if capped.any():
@@ -181,6 +183,9 @@ class AndersonBatch:
         gr = np.ascontiguousarray(dl_dre, dtype=np.float64)
         gi = np.ascontiguousarray(dl_dim, dtype=np.float64)
         M, mb = self.eps_bath.shape
+        if self._num_freq is not None and not gr.size == gi.size == M * self._num_freq:
+            raise ValueError(f"the gradient must have the shape of the last solve's G, ({M}, {self._num_freq}); "
+                             f"got {gr.shape} and {gi.shape}")
         ge = np.zeros((M, mb))
         gv = np.zeros((M, mb))
         cg = np.empty(M, dtype=np.int32)

@@ -2670,7 +2670,7 @@ struct ed_batch {
   BwdTile* d_tiles = nullptr;
   BwdBlock* d_blocks = nullptr;
   double *d_jstore = nullptr, *d_rec = nullptr, *d_partial = nullptr;
-  int64_t cap_jobs = 0, cap_gemms = 0, cap_tiles = 0, cap_blocks = 0, cap_jstore = 0;
+  int64_t cap_jobs = 0, cap_gemms = 0, cap_tiles = 0, cap_blocks = 0, cap_jstore = 0, cap_grad = 0;
   char* d_bws = nullptr;
   int64_t bws_bytes = 0;
   int32_t solved_nw = -1;  // frequencies of the last solve (the backward uses them)
@@ -2717,6 +2717,22 @@ static int balloc(T** p, int64_t n) {
     return set_error(ED_ERR_NOMEM, "hipMalloc of %lld bytes failed: %s", (long long)(sizeof(T) * n),
                      hipGetErrorString(e));
   }
+  return ED_OK;
+}
+
+// Two buffers that grow together, of n and n * per entries; the capacity counts
+// only once both are there.
+template <typename T, typename U>
+static int grow_pair(T** p, U** q, int64_t per, int64_t* cap, int64_t n) {
+  if (n <= *cap) return ED_OK;
+  *cap = 0;
+  if (*p) (void)hipFree(*p);
+  if (*q) (void)hipFree(*q);
+  *p = nullptr;
+  *q = nullptr;
+  ED_TRY(balloc(p, n));
+  ED_TRY(balloc(q, n * per));
+  *cap = n;
   return ED_OK;
 }
 
@@ -3229,10 +3245,7 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   hipStream_t s = as_stream(stream);
   const int64_t M = b->num_models;
   const int32_t nw = b->solved_nw;
-  if (!b->d_gre) {
-    ED_TRY(balloc(&b->d_gre, M * nw));
-    ED_TRY(balloc(&b->d_gim, M * nw));
-  }
+  ED_TRY(grow_pair(&b->d_gre, &b->d_gim, 1, &b->cap_grad, M * nw));
   int dev = 0, cus = 256;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
@@ -3332,12 +3345,7 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   ED_TRY(grow(&b->d_jobs, &b->cap_jobs, (int64_t)jobs.size()));
   ED_TRY(grow(&b->d_gemms, &b->cap_gemms, (int64_t)gemms.size()));
   ED_TRY(grow(&b->d_tiles, &b->cap_tiles, (int64_t)(tiles_w.size() + tiles.size())));
-  if ((int64_t)blocks.size() > b->cap_blocks) {
-    if (b->d_partial) (void)hipFree(b->d_partial);
-    b->d_partial = nullptr;
-    ED_TRY(grow(&b->d_blocks, &b->cap_blocks, (int64_t)blocks.size()));
-    ED_TRY(balloc(&b->d_partial, b->cap_blocks * kRecPart));
-  }
+  ED_TRY(grow_pair(&b->d_blocks, &b->d_partial, kRecPart, &b->cap_blocks, (int64_t)blocks.size()));
   ED_TRY(grow(&b->d_jstore, &b->cap_jstore, jst));
   ED_HIP(hipMemcpy(b->d_job_of, job_of.data(), sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice));
   if (!jobs.empty()) {

@@ -1,0 +1,48 @@
+"""The batch buffers that grow with the number of frequencies, on the CPU under AddressSanitizer and UBSan
+(tests/cpu_kernels/regrow_check.cpp): one batch solved and differentiated at a few frequencies, at more of them and at
+a few again, against a fresh batch for each; the same with an allocation that fails on the way."""
+
+import subprocess
+
+import numpy as np
+import pytest
+
+from test_cpu_batch_kernel import CLANG, HERE, _build_harness
+
+pytestmark = pytest.mark.skipif(not CLANG.exists(), reason="host clang++ with sanitizer runtimes not found")
+
+
+@pytest.fixture(scope="module")
+def run():
+    bh = _build_harness()
+    bh.TARGETS["regrow"] = (HERE / "cpu_kernels/regrow_check.cpp", "ed_batch")
+    exe = bh.build(name="regrow_check", target="regrow")
+
+    def steps(*script):
+        r = subprocess.run([str(exe), *script], capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stderr[-4000:]
+        assert "AddressSanitizer" not in r.stderr and "runtime error" not in r.stderr, r.stderr[-4000:]
+        return [(t[0], int(t[1]), np.array(t[2:], dtype=float)) for t in map(str.split, r.stdout.splitlines())]
+
+    return steps
+
+
+@pytest.fixture(scope="module")
+def fresh(run):
+    """The gradients of a fresh batch at n frequencies."""
+    return {n: run("s%d" % n, "b")[-1][2] for n in (4, 48)}
+
+
+def test_more_and_fewer_frequencies_on_one_batch(run, fresh):
+    got = [r for r in run("s4", "b", "s48", "b", "s4", "b") if r[0] == "grad"]
+    for (_, rc, g), n in zip(got, (4, 48, 4)):
+        assert rc == 0 and np.isfinite(g).all() and np.array_equal(g, fresh[n])
+
+
+@pytest.mark.parametrize("before", [(), ("s4", "b")])
+@pytest.mark.parametrize("fail", range(9))
+def test_failed_allocation_of_a_backward(run, fresh, before, fail):
+    """One of the allocations of a backward, the batch's first or one that grows, fails: that call is refused, the next
+    one is right."""
+    out = run(*before, "s48", "f%d" % fail, "b", "b")
+    assert out[-1][1] == 0 and np.array_equal(out[-1][2], fresh[48])

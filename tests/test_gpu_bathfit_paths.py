@@ -60,3 +60,31 @@ def test_backward_routes_agree(gpu, monkeypatch, nb, n_up, n_dn):
         for i in range(M):
             _, de, dv = O.bathfit_grad_dense(3.0, -1.5, eb[i], v[i], 0.0, n_up, n_dn, wn, target[i], 0)
             _check(got[i:i + 1], np.concatenate([de, dv])[None], "dense")
+
+
+def test_number_of_frequencies_changes_on_one_batch(gpu):
+    """One batch solved and differentiated at 16, 300 and 16 frequencies: the gradients of fresh batches, and gradients
+    of another size than the last solve's G are refused."""
+    from cmpy_amd.batch import AndersonBatch, matsubara
+
+    rng = np.random.default_rng(31)
+    M, nb = 3, 4
+    kw = dict(u=np.full(M, 3.0), eps_imp=-1.5, eps_bath=list(rng.uniform(-3, 3, (M, nb))),
+              v=list(rng.uniform(0.1, 1.2, (M, nb))), mu=0.0, keep_basis=True)
+
+    def grads(b, n):
+        wn = matsubara(50.0, n)
+        _, gr, gi, _ = _loss_grads(b, wn, 1.0 / (1j * wn - np.linspace(-1, 1, M)[:, None]))
+        return gr, gi, np.concatenate(b.backward(gr, gi)[:2], axis=1)
+
+    b = AndersonBatch(**kw)
+    b.config(-1, 4, 0)
+    for n in (16, 300, 16):
+        f = AndersonBatch(**kw)
+        f.config(-1, 4, 0)
+        gr, gi, got = grads(b, n)
+        assert np.array_equal(got, grads(f, n)[2])
+        with pytest.raises(ValueError, match="last solve"):
+            b.backward(gr[:, 1:], gi[:, 1:])
+        with pytest.raises(ValueError, match="last solve"):
+            b.backward(gr, gi[:, 1:])
