@@ -2675,7 +2675,7 @@ struct ed_batch {
   int64_t bws_bytes = 0;
   int32_t solved_nw = -1;  // frequencies of the last solve (the backward uses them)
   int64_t ws_bytes = 0;
-  int32_t nw_cap = 0;
+  int64_t nw_cap = 0;
   // launch configuration
   int64_t wave_max_dim = -1;  // models with dim <= this run in wave mode (-1: not chosen)
   int32_t grid = 0, wave_blocks = 0;
@@ -3127,24 +3127,18 @@ extern "C" int ed_batch_solve(ed_batch* b, const double* wn, int32_t nw, double*
   ED_REQUIRE(b, "NULL batch");
   ED_REQUIRE(nw >= 0 && (nw == 0 || wn), "bad frequency list");
   hipStream_t s = as_stream(stream);
-  if (nw > b->nw_cap) {
-    if (b->d_g) (void)hipFree(b->d_g);
-    if (b->d_wn) (void)hipFree(b->d_wn);
-    b->d_g = nullptr;
-    b->d_wn = nullptr;
-    b->nw_cap = 0;
-    ED_TRY(balloc(&b->d_g, 2 * b->num_models * (int64_t)nw));
-    ED_TRY(balloc(&b->d_wn, nw));
-    b->nw_cap = nw;
-    if (b->graph) {
-      (void)hipGraphExecDestroy(b->graph);
-      b->graph = nullptr;
-    }
-  }
   double wmin = 1.0;
   for (int32_t k = 0; k < nw; ++k) {
     ED_REQUIRE(std::isfinite(wn[k]) && wn[k] != 0.0, "frequencies must be finite and non-zero");
     wmin = k == 0 ? fabs(wn[k]) : std::min(wmin, fabs(wn[k]));
+  }
+  b->solved_nw = -1;  // from here on the last solve's frequencies and coefficients are overwritten
+  if (nw > b->nw_cap) {
+    if (b->graph) {
+      (void)hipGraphExecDestroy(b->graph);
+      b->graph = nullptr;
+    }
+    ED_TRY(grow_pair(&b->d_wn, &b->d_g, 2 * b->num_models, &b->nw_cap, nw));
   }
   if (nw > 0) ED_HIP(hipMemcpyAsync(b->d_wn, wn, sizeof(double) * nw, hipMemcpyHostToDevice, s));
   if (!b->tuned) {

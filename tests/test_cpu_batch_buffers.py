@@ -30,7 +30,7 @@ def run():
 @pytest.fixture(scope="module")
 def fresh(run):
     """The gradients of a fresh batch at n frequencies."""
-    return {n: run("s%d" % n, "b")[-1][2] for n in (4, 48)}
+    return {n: run("s%d" % n, "b")[-1][2] for n in (2, 4, 48)}
 
 
 def test_more_and_fewer_frequencies_on_one_batch(run, fresh):
@@ -46,3 +46,18 @@ def test_failed_allocation_of_a_backward(run, fresh, before, fail):
     one is right."""
     out = run(*before, "s48", "f%d" % fail, "b", "b")
     assert out[-1][1] == 0 and np.array_equal(out[-1][2], fresh[48])
+
+
+def test_refused_frequencies_leave_the_last_solve(run, fresh):
+    """A solve refused for a zero frequency, at more of them than the batch had, does not touch what a backward of the
+    solve before it reads."""
+    out = run("s2", "z", "b")
+    assert out[1][1] != 0 and out[2][1] == 0 and np.array_equal(out[2][2], fresh[2])
+
+
+@pytest.mark.parametrize("fail", range(2))
+def test_failed_allocation_of_a_solve(run, fresh, fail):
+    """Nor is a backward of a solve that did not come about taken for one."""
+    out = run("s4", "f%d" % fail, "s48", "b", "s48", "b")
+    assert out[1][1] != 0 and out[2][1] != 0
+    assert out[4][1] == 0 and np.array_equal(out[4][2], fresh[48])
