@@ -95,18 +95,19 @@ static __constant__ FourierSeries kFourierSeries = make_fourier_series();
 // t_0 < ... < t_{nt-1}: per interval of length h, with a = i z and x = a h,
 //   e^{a t_k} h [g_k E1(x) + (g_{k+1} - g_k) E2(x)],
 //   E1 = (e^x - 1)/x = sum_n x^n/(n+1)!,  E2 = (x e^x - e^x + 1)/x^2 = sum_n (n+1) x^n/(n+2)!,
-// the series (12 terms) for |x| < 0.1.  A block per frequency, its threads over
-// the intervals, their sums added in thread order within a wave's halves and
-// then over the waves.  One thread per frequency left 16 waves to walk 1000
-// intervals each: 1,045 us for 1000 x 1000, 14 us now (FP64 exponentials).
+// the series (12 terms) for |x| < 0.1.  T threads a frequency, the intervals
+// dealt over them; their sums are added in thread order within a wave's halves
+// and then over the waves.
+template <int T>
 __global__ __launch_bounds__(256) void k_fourier_t2z(const double* __restrict__ t, const double* __restrict__ g,
-                                                     int64_t nt, const double* __restrict__ z,
+                                                     int64_t nt, const double* __restrict__ z, int64_t nz,
                                                      double* __restrict__ out) {
   __shared__ double sh[2][4];
-  const int64_t j = blockIdx.x;
+  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) / T;
+  const int64_t j = at < nz ? at : nz - 1;
   const c64 a = {-z[2 * j + 1], z[2 * j]};  // i z
   c64 acc = {0.0, 0.0};
-  for (int64_t k = threadIdx.x; k + 1 < nt; k += blockDim.x) {
+  for (int64_t k = threadIdx.x % T; k + 1 < nt; k += T) {
     const double h = t[k + 1] - t[k];
     const c64 x = {a.re * h, a.im * h};
     c64 e1, e2;
@@ -135,18 +136,21 @@ __global__ __launch_bounds__(256) void k_fourier_t2z(const double* __restrict__ 
     acc.im += term.im;
   }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
+  for (int off = (T < 64 ? T : 64) / 2; off > 0; off >>= 1) {
     acc.re += __shfl_down(acc.re, off, 64);
     acc.im += __shfl_down(acc.im, off, 64);
   }
-  if ((threadIdx.x & 63) == 0) {
-    sh[0][threadIdx.x >> 6] = acc.re;
-    sh[1][threadIdx.x >> 6] = acc.im;
+  if constexpr (T == 256) {
+    if ((threadIdx.x & 63) == 0) {
+      sh[0][threadIdx.x >> 6] = acc.re;
+      sh[1][threadIdx.x >> 6] = acc.im;
+    }
+    __syncthreads();
+    acc = {(sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]), (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3])};
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    out[2 * j] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
-    out[2 * j + 1] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+  if (threadIdx.x % T == 0 && at < nz) {
+    out[2 * j] = acc.re;
+    out[2 * j + 1] = acc.im;
   }
 }
 
@@ -161,10 +165,23 @@ extern "C" int ed_fourier_t2z(const double* t_dev, const double* g_dev, int64_t 
   ED_REQUIRE(nz == 0 || (z_dev && out_dev), "NULL buffer");
   ED_REQUIRE(nt == 0 || (t_dev && g_dev), "NULL buffer");
   if (nz == 0) return ED_OK;
-  // at most 2^30 frequencies a launch
-  for (int64_t j = 0; j < nz; j += int64_t(1) << 30)
-    hipLaunchKernelGGL(k_fourier_t2z, dim3((unsigned)std::min<int64_t>(nz - j, int64_t(1) << 30)), dim3(256), 0,
-                       as_stream(stream), t_dev, g_dev, nt, z_dev + 2 * j, out_dev + 2 * j);
+  // Threads a frequency: as many as fill the chip (2^19 threads) and have an
+  // interval each.  1000 times x 1000 frequencies take 12 us at 256 (1,041 at
+  // one), 8 x 10^5 take 12 at 4 (152 at 256), 100 x 10^6 take 906 at one (1,929 at
+  // 256: reductions of single terms), 1000 x 10^5 take 777 at 16 (1,561 at one, 805
+  // at 256).
+  constexpr int64_t kFill = int64_t(1) << 19;
+  int T = 1;
+  while (T < 256 && 4 * T < nt && nz * T < kFill) T *= 4;
+  const auto kernel = T == 1 ? k_fourier_t2z<1> : T == 4 ? k_fourier_t2z<4> : T == 16 ? k_fourier_t2z<16>
+                    : T == 64 ? k_fourier_t2z<64> : k_fourier_t2z<256>;
+  // a launch has fewer than 2^32 threads
+  constexpr int64_t kPer = int64_t(1) << 30;
+  for (int64_t j = 0; j < nz; j += kPer) {
+    const int64_t n = std::min(nz - j, kPer);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((n * T + 255) / 256)), dim3(256), 0, as_stream(stream), t_dev, g_dev,
+                       nt, z_dev + 2 * j, n, out_dev + 2 * j);
+  }
   ED_HIP(hipGetLastError());
   return ED_OK;
 }

@@ -51,3 +51,29 @@ def test_fourier_t2z(gpu, nt, nz):
     want = O.fourier_t2z(t, g, w, eta=0.05)
     want = want[1] if isinstance(want, tuple) else want
     assert np.abs(got - want).max() <= 1e-12 * max(np.abs(want).max(), 1.0)
+
+
+@pytest.mark.parametrize("nt,nz", [(3, (1 << 24) + 5), (5, 1 << 18), (9, (1 << 18) - 1), (70, 65537), (300, 16385),
+                                   (17, 16383), (400, 4095), (3, 1000)])
+def test_fourier_t2z_many_frequencies(gpu, nt, nz):
+    """One, 4, 16, 64 and 256 threads a frequency, and more frequencies than a launch has room for at 256: the first,
+    the last and those around a block's edge against the oracle, as above."""
+    from cmpy_amd import _lib as L
+
+    rng = np.random.default_rng(nt)
+    t = np.cumsum(rng.uniform(0.01, 0.4, nt))
+    g = rng.standard_normal(nt) + 1j * rng.standard_normal(nt)
+    at = np.unique([k % nz for k in (0, 1, 3, 4, 63, 64, 255, 256, nz // 2, (1 << 24) - 1, 1 << 24, -257, -2, -1)])
+    z = torch.zeros((nz, 2), dtype=torch.float64, device="cuda")
+    z[:, 0] = torch.linspace(-4, 4, nz, dtype=torch.float64, device="cuda")
+    z[:, 1] = 0.05
+    out = torch.full((nz, 2), float("nan"), dtype=torch.float64, device="cuda")
+    td = torch.from_numpy(t).cuda()
+    gd = torch.from_numpy(np.stack([g.real, g.imag], axis=1).copy()).cuda()
+    L.call("ed_fourier_t2z", L.dptr(td), L.dptr(gd), nt, L.dptr(z), nz, L.dptr(out), L.stream_ptr())
+    assert not torch.isnan(out).any()
+    idx = torch.from_numpy(at).cuda()
+    got = out[idx].cpu().numpy()
+    want = O.fourier_t2z(t, g, z[idx, 0].cpu().numpy(), eta=0.05)
+    want = want[1] if isinstance(want, tuple) else want
+    assert np.abs(got[:, 0] + 1j * got[:, 1] - want).max() <= 1e-12 * max(np.abs(want).max(), 1.0)
