@@ -244,7 +244,8 @@ __global__ __launch_bounds__(256) void k_tevo_sum(const double* __restrict__ the
 // Moments: one block, thread i holds entries i, i + blockDim, ... of the two
 // last vectors T_k e1 in LDS.
 constexpr int kChebEntries = 2;      // entries per thread: m <= 2048
-constexpr int kChebMaxTerms = 3584; // in LDS beside the two vectors; one block forms them in order
+constexpr int kChebMaxTerms = 3584;  // in LDS beside the two vectors; one block forms them in order
+constexpr int kChebMinTerms = 40;
 __global__ __launch_bounds__(1024) void k_cheb_moments(const double* __restrict__ a, const double* __restrict__ b,
                                                        int m, double c, double rinv, int terms,
                                                        double* __restrict__ mu) {
@@ -284,6 +285,23 @@ __global__ __launch_bounds__(1024) void k_cheb_moments(const double* __restrict_
     __syncthreads();
   }
   for (int k = threadIdx.x; k < terms; k += nt) mu[k] = ms[k];
+}
+
+// max |t| of each block's share; infinity where one is not finite.
+constexpr int kSpanBlocks = 64;
+__global__ __launch_bounds__(256) void k_time_span(const double* __restrict__ t, int64_t nt,
+                                                   double* __restrict__ span) {
+  __shared__ double sh[4];
+  double v = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nt; i += (int64_t)gridDim.x * 256) {
+    const double a = fabs(t[i]);
+    v = fmax(v, isfinite(a) ? a : (double)INFINITY);
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) span[blockIdx.x] = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
 }
 
 // One time per thread: J_k(z), z = r |t|, by downward recurrence from k = terms
@@ -620,6 +638,48 @@ static int get_handle(rocblas_handle* h, hipStream_t s) {
   return ED_OK;
 }
 
+// Interval [c - r, c + r] that holds the spectrum of a Lanczos tridiagonal; r is
+// infinite where a coefficient is not finite.
+struct Interval {
+  double c, r;
+};
+static Interval gershgorin(const double* alpha, const double* beta, int m) {
+  double lo = alpha[0], hi = alpha[0];
+  for (int j = 0; j < m; ++j) {
+    const double w = (j > 0 ? fabs(beta[j - 1]) : 0.0) + (j + 1 < m ? fabs(beta[j]) : 0.0);
+    if (!std::isfinite(alpha[j]) || !std::isfinite(w)) return {0.0, (double)INFINITY};
+    lo = std::min(lo, alpha[j] - w);
+    hi = std::max(hi, alpha[j] + w);
+  }
+  const double c = 0.5 * lo + 0.5 * hi;
+  return {c, std::max(0.5 * (hi - lo) * (1.0 + 1e-12), 1e-12 * std::max(fabs(c), 1.0))};
+}
+
+// max |t| (infinite where a time is not finite), the call's work before s waited
+// for: up to kSpanHost times are read as they are, more by their blocks' maxima.
+constexpr int kSpanHost = 4096;
+static int time_span(const double* t_dev, int64_t nt, double* tmax, hipStream_t s) {
+  double h[kSpanHost];
+  int n = (int)nt;
+  *tmax = 0.0;
+  if (nt <= kSpanHost) {
+    ED_HIP(hipMemcpyAsync(h, t_dev, sizeof(double) * nt, hipMemcpyDeviceToHost, s));
+    ED_HIP(hipStreamSynchronize(s));
+  } else {
+    double* d = nullptr;
+    n = kSpanBlocks;
+    ED_HIP(hipMallocAsync((void**)&d, sizeof(double) * n, s));
+    hipLaunchKernelGGL(k_time_span, dim3(kSpanBlocks), dim3(256), 0, s, t_dev, nt, d);
+    hipError_t e = hipMemcpyAsync(h, d, sizeof(double) * n, hipMemcpyDeviceToHost, s);
+    (void)hipFreeAsync(d, s);
+    const hipError_t es = hipStreamSynchronize(s);
+    if (e == hipSuccess) e = es;
+    if (e != hipSuccess) return set_error(ED_ERR_HIP, "reading the times failed: %s", hipGetErrorString(e));
+  }
+  for (int i = 0; i < n; ++i) *tmax = std::isfinite(h[i]) ? std::max(*tmax, fabs(h[i])) : (double)INFINITY;
+  return ED_OK;
+}
+
 }  // namespace ed
 
 using namespace ed;
@@ -691,23 +751,15 @@ int ed_tevo_eval(const double* alpha, const double* beta, int32_t m, double norm
   for (int j = 0; j < m; ++j) hd[j] = alpha[j];
   for (int j = 0; j + 1 < m; ++j) hd[m + j] = beta[j];
   int rc = ED_OK;
-  // The Chebyshev sum where its terms fit: they number about r max |t|, which
-  // the host needs to know.
-  if (m <= 2048) {
-    double lo = alpha[0], hi = alpha[0];
-    for (int j = 0; j < m; ++j) {
-      const double w = (j > 0 ? fabs(beta[j - 1]) : 0.0) + (j + 1 < m ? fabs(beta[j]) : 0.0);
-      lo = std::min(lo, alpha[j] - w);
-      hi = std::max(hi, alpha[j] + w);
-    }
-    const double c = 0.5 * (lo + hi), r = std::max(0.5 * (hi - lo) * (1.0 + 1e-12), 1e-12 * std::max(fabs(c), 1.0));
-    std::vector<double> ht((size_t)nt);
-    ED_HIP(hipMemcpyAsync(ht.data(), t_dev, sizeof(double) * nt, hipMemcpyDeviceToHost, s));
-    ED_HIP(hipStreamSynchronize(s));
-    double z = 0.0;
-    for (double t : ht) z = std::isfinite(t) ? std::max(z, r * fabs(t)) : (double)INFINITY;
-    const double terms = z + 12.0 * cbrt(z) + 40.0;
-    if (terms <= (double)kChebMaxTerms) {
+  // The Chebyshev sum where its terms fit: they number about r max |t|, which the
+  // host needs to know.
+  const Interval span = gershgorin(alpha, beta, m);
+  if (m <= kChebEntries * 1024 && std::isfinite(span.r)) {
+    double tmax;
+    ED_TRY(time_span(t_dev, nt, &tmax, s));
+    const double z = span.r * tmax;
+    const double terms = z + 12.0 * cbrt(z) + kChebMinTerms;
+    if (terms <= kChebMaxTerms) {
       const int n = (int)terms;
       double* d = nullptr;
       ED_HIP(hipMallocAsync((void**)&d, sizeof(double) * (2 * (size_t)m + n), s));
@@ -715,10 +767,10 @@ int ed_tevo_eval(const double* alpha, const double* beta, int32_t m, double norm
         rc = set_error(ED_ERR_HIP, "copying Lanczos coefficients failed");
       } else {
         const unsigned bt = (unsigned)std::min(1024, ((m + 1) / 2 + 63) / 64 * 64);
-        hipLaunchKernelGGL(k_cheb_moments, dim3(1), dim3(bt), sizeof(double) * n, s, d, d + m, m, c, 1.0 / r, n,
-                           d + 2 * (size_t)m);
+        hipLaunchKernelGGL(k_cheb_moments, dim3(1), dim3(bt), sizeof(double) * n, s, d, d + m, m, span.c,
+                           1.0 / span.r, n, d + 2 * (size_t)m);
         hipLaunchKernelGGL(k_cheb_sum, dim3((unsigned)((nt + 63) / 64)), dim3(64), sizeof(double) * n, s,
-                           d + 2 * (size_t)m, n, c, r, norm2, e0, sign, t_dev, nt, g_dev, accumulate);
+                           d + 2 * (size_t)m, n, span.c, span.r, norm2, e0, sign, t_dev, nt, g_dev, accumulate);
         if (hipGetLastError() != hipSuccess) rc = set_error(ED_ERR_HIP, "time-sum launch failed");
       }
       (void)hipFreeAsync(d, s);

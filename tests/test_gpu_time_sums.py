@@ -39,6 +39,37 @@ def test_tevo_eval(gpu, m, tmax, sign):
         assert np.abs(got - want).max() <= 2e-12 * norm2
 
 
+def _tevo(a, b, norm2, e0, sign, t):
+    from cmpy_amd import _lib as L
+
+    dp = C.POINTER(C.c_double)
+    td = torch.from_numpy(t).cuda()
+    g = torch.full((2 * len(t),), float("nan"), dtype=torch.float64, device="cuda")
+    L.call("ed_tevo_eval", a.ctypes.data_as(dp), b.ctypes.data_as(dp), len(a), norm2, e0, sign, L.dptr(td), len(t),
+           L.dptr(g), 0, L.stream_ptr())
+    g = g.cpu().numpy()
+    return g[::2] + 1j * g[1::2]
+
+
+# the largest number of times the host reads, one more (maxima of blocks), and many; the largest |t| last, first, inside
+@pytest.mark.parametrize("nt", [4096, 4097, 300001])
+@pytest.mark.parametrize("at", [0, -1, 0.5])
+def test_tevo_eval_many_times(gpu, nt, at):
+    """The number of terms follows from the largest |t|, wherever it stands.  Bound as above."""
+    rng = np.random.default_rng(nt)
+    m = 40
+    a, b = rng.uniform(-2, 2, m), rng.uniform(0.1, 1.0, m - 1)
+    t = rng.uniform(-1, 1, nt)
+    k = int(at * nt) if at == 0.5 else at
+    t[k] = -90.0
+    got = _tevo(a, b, 0.7, -1.3, 1, t)
+    assert np.isfinite(got).all()
+    pick = np.unique(np.concatenate([[k % nt, 0, nt - 1], rng.integers(0, nt, 50)]))
+    w, v = np.linalg.eigh(np.diag(a) + np.diag(b, 1) + np.diag(b, -1))
+    want = -0.7j * (np.exp(-1j * (w[None, :] + 1.3) * t[pick, None]) @ v[0] ** 2)
+    assert np.abs(got[pick] - want).max() <= 2e-12 * 0.7
+
+
 @pytest.mark.parametrize("nt,nz", [(1, 2), (2, 1), (64, 3), (257, 5), (258, 2), (1300, 7)])
 def test_fourier_t2z(gpu, nt, nz):
     from cmpy_amd import fourier_t2z
