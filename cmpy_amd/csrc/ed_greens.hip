@@ -241,6 +241,8 @@ __global__ __launch_bounds__(256) void k_tevo_sum(const double* __restrict__ the
 // (moments, a chain of barriers) and 45 us (1000 times, a chain of fused
 // multiply-adds) here.
 //
+// Which of the two a call takes: chebyshev_us and eigenpairs_us.
+//
 // Moments: one block, thread i holds entries i, i + blockDim, ... of the two
 // last vectors T_k e1 in LDS.
 constexpr int kChebEntries = 2;      // entries per thread: m <= 2048
@@ -655,6 +657,16 @@ static Interval gershgorin(const double* alpha, const double* beta, int m) {
   return {c, std::max(0.5 * (hi - lo) * (1.0 + 1e-12), 1e-12 * std::max(fabs(c), 1.0))};
 }
 
+// Microseconds of the two sums over nt times, by `terms` terms and by the
+// eigenpairs of m nodes, fitted to both at m = 1 .. 2048, 40 .. 3519 terms and 1 ..
+// 10^6 times: the moments and the sum are chains over the terms; the
+// eigensolver's launches grow with m.  (2 nodes, |r t| = 3300, 1000 times: 915 us
+// by terms, 53 by eigenpairs; 340 nodes, |r t| = 200: 131 and 1,224.)
+static double chebyshev_us(double terms, int64_t nt) { return 65.0 + 0.245 * terms + 1e-6 * terms * (double)nt; }
+static double eigenpairs_us(int m, int64_t nt) {
+  return std::min(40.0 + 5.0 * m + 0.8 * m * m, 73.0 * sqrt((double)m)) + 2e-6 * m * (double)nt;
+}
+
 // max |t| (infinite where a time is not finite), the call's work before s waited
 // for: up to kSpanHost times are read as they are, more by their blocks' maxima.
 constexpr int kSpanHost = 4096;
@@ -751,15 +763,16 @@ int ed_tevo_eval(const double* alpha, const double* beta, int32_t m, double norm
   for (int j = 0; j < m; ++j) hd[j] = alpha[j];
   for (int j = 0; j + 1 < m; ++j) hd[m + j] = beta[j];
   int rc = ED_OK;
-  // The Chebyshev sum where its terms fit: they number about r max |t|, which the
-  // host needs to know.
+  // The Chebyshev sum where its terms fit and it is the cheaper one.  They number
+  // about r max |t|, which the host asks for (scan_us) where it can be.
   const Interval span = gershgorin(alpha, beta, m);
-  if (m <= kChebEntries * 1024 && std::isfinite(span.r)) {
+  const double eigen_us = eigenpairs_us(m, nt), scan_us = nt <= kSpanHost ? 25.0 : 100.0;
+  if (m <= kChebEntries * 1024 && std::isfinite(span.r) && chebyshev_us(kChebMinTerms, nt) + scan_us < eigen_us) {
     double tmax;
     ED_TRY(time_span(t_dev, nt, &tmax, s));
     const double z = span.r * tmax;
     const double terms = z + 12.0 * cbrt(z) + kChebMinTerms;
-    if (terms <= kChebMaxTerms) {
+    if (terms <= kChebMaxTerms && chebyshev_us(terms, nt) < eigen_us) {
       const int n = (int)terms;
       double* d = nullptr;
       ED_HIP(hipMallocAsync((void**)&d, sizeof(double) * (2 * (size_t)m + n), s));

@@ -70,6 +70,20 @@ def test_tevo_eval_many_times(gpu, nt, at):
     assert np.abs(got[pick] - want).max() <= 2e-12 * 0.7
 
 
+@pytest.mark.parametrize("m", [1, 3, 4, 6, 7, 8, 12, 20, 50, 120])
+@pytest.mark.parametrize("phase", [1.0, 60.0, 250.0, 1000.0, 3300.0])
+def test_tevo_eval_either_side_of_the_rule(gpu, m, phase):
+    """Few nodes or long times go to the eigenpairs, many nodes to the terms; both within the bound above."""
+    rng = np.random.default_rng(m)
+    a, b = rng.uniform(-2, 2, m), rng.uniform(0.1, 1.0, max(m - 1, 1))
+    h = np.diag(a) + (np.diag(b[:m - 1], 1) + np.diag(b[:m - 1], -1) if m > 1 else 0.0)
+    t = np.append(rng.uniform(-1, 1, 70), 1.0) * phase / max(np.abs(h).sum(axis=1).max(), 1.0)
+    got = _tevo(a, b, 0.7, -1.3, -1, t)
+    w, v = np.linalg.eigh(h)
+    want = 0.7j * (np.exp(1j * (w[None, :] + 1.3) * t[:, None]) @ v[0] ** 2)
+    assert np.abs(got - want).max() <= 2e-12 * 0.7
+
+
 @pytest.mark.parametrize("nt,nz", [(1, 2), (2, 1), (64, 3), (257, 5), (258, 2), (1300, 7)])
 def test_fourier_t2z(gpu, nt, nz):
     from cmpy_amd import fourier_t2z
