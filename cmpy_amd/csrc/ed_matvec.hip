@@ -643,9 +643,9 @@ __global__ __launch_bounds__(kRowThreads) void k_hv_rows_held(Hv2Args a, int row
 // gathers through the packed column-major table, whose entries serve all RB
 // rows.  Slots past a state's count take nothing from x, so that an infinity
 // reaches only the entries that H couples to it: an up slot is branched over (a
-// row's count is uniform; another hop's address in its place also cost its
-// load, as much as half of a star's, whose rows have 3 and 13 hops: 13-site
-// impurity (4,5) 24.0 us, 16.5 without), a dn slot gathers the zero past its
+// row's count is uniform; a load in its place costs as much as half of a star's
+// hops, whose rows have 3 and 13 of them: 13-site impurity (4,5) 24.0 us, 16.5
+// without), a dn slot gathers the zero past its
 // row.  Blocks go to XCDs in contiguous runs of rows, whose hop sources lie
 // mostly near them.  blockIdx.y picks the vector.  Every wave has a chunk (at
 // most nch waves a block).
@@ -690,9 +690,11 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
   const double cs = LZ && e.cself ? *e.cself : 0.0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  // up hops of a row whose loads are in flight together (more of them, with
-  // four rows or two, take registers that a second block of the CU needs)
-  constexpr int UP = 8 / RB;
+  // up hops of a row whose loads are in flight together: more, or the branches
+  // over four rows' unused slots where rows are of nearly one length (lattices,
+  // of uniform hopping), take registers that a second block of the CU needs
+  constexpr bool EVEN = RB == 4 && UNI;
+  constexpr int UP = RB == 1 ? 8 : EVEN || (RB == 2 && !LZ) ? 4 : 2;
   int cu[RB], cmax = 0;
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -717,8 +719,8 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
       for (int r = 0; r < RB; ++r)
 #pragma unroll
         for (int q = 0; q < UP; ++q)
-          if (e0 + q < cu[r]) {  // uniform over the block
-            const int64_t k = (int64_t)(r0 + r) * a.up_w + e0 + q;
+          if (EVEN || e0 + q < cu[r]) {  // uniform over the block
+            const int64_t k = (int64_t)(r0 + (r < R ? r : 0)) * a.up_w + (e0 + q < cu[r] ? e0 + q : 0);
             const uint32_t en = uniform_load(a.up_pk + k);
             v[r][q] = UNI ? ((en & 0x80000000u) ? -1.0 : 1.0) : uniform_load(a.up_val + k);
             g[r][q] = (x + (int64_t)hop_target(en) * ld)[ids];
@@ -1551,16 +1553,15 @@ static TileKernel tile_kernel(int rb, bool uni, bool lz) {
   return rb == 4 ? tile_kernel_rb<4>(uni, lz) : rb == 2 ? tile_kernel_rb<2>(uni, lz) : tile_kernel_rb<1>(uni, lz);
 }
 
+constexpr int64_t kTileFourRows = 192;  // blocks, 3/4 of one a CU
 constexpr int64_t kTileWaves = 2048;    // waves that keep the chip busy (2 per SIMD)
 constexpr size_t kTileLds = 64 * 1024;  // granted without an attribute, and two blocks fit a CU
 constexpr int kTileMaxThreads = 1024;
 
-// Rows per block: as many as keep kTileWaves waves in flight, up to four where
-// a block has 14 waves or more and two below (the dn table's entries are read
-// once for all of a block's rows, but four rows leave registers for 20 waves a
-// CU, so that a block of 11 or 12 is alone on it: 13-site chain (6,5) 33.6 us
-// with four, 30.7 with two, (5,4) 17.1 and 12.6; 4x4 (4,4), 15 waves, 56.4 and
-// 59.9; 12-site chain (6,6), 15 waves, 13.0 and 13.2).
+// Rows per block: as many as keep kTileWaves waves in flight, up to four (the dn
+// table's entries are read once for all of a block's rows; 12-site chain: 14.1 us
+// with four rows, 15.2 with two, 16.7 with one), four only for kTileFourRows
+// blocks or more (13-site chain (4,4), 179 blocks of four: 10.0 us, 8.3 of two).
 static TilePlan plan_tile(const ed_op* op) {
   TilePlan p{};
   if (!op->packed || op->size == 0) return p;
@@ -1568,9 +1569,13 @@ static TilePlan plan_tile(const ed_op* op) {
   const int64_t iters = (nch + kTileMaxThreads / 64 - 1) / (kTileMaxThreads / 64);
   const int64_t waves = (nch + iters - 1) / iters;
   p.threads = (int)waves * 64;
-  p.rb = waves >= 14 ? 4 : 2;
-  for (; p.rb > 1; p.rb /= 2)
-    if (p.rb * (op->num_dn + 1) * sizeof(double) <= kTileLds - 256 && (op->num_up + p.rb - 1) / p.rb * waves >= kTileWaves) break;
+  p.rb = 4;
+  for (; p.rb > 1; p.rb /= 2) {
+    const int64_t blocks = (op->num_up + p.rb - 1) / p.rb;
+    if (p.rb * (op->num_dn + 1) * sizeof(double) <= kTileLds - 256 && blocks * waves >= kTileWaves &&
+        (p.rb < 4 || blocks >= kTileFourRows))
+      break;
+  }
   p.lds_bytes = p.rb * (op->num_dn + 1) * sizeof(double);
   if (p.lds_bytes > kTileLds - 256) return p;  // the kernel has static LDS of its own
   p.nrg = (int)((op->num_up + p.rb - 1) / p.rb);
