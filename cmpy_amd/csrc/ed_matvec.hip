@@ -1562,6 +1562,15 @@ constexpr int kTileMaxThreads = 1024;
 // table's entries are read once for all of a block's rows; 12-site chain: 14.1 us
 // with four rows, 15.2 with two, 16.7 with one), four only for kTileFourRows
 // blocks or more (13-site chain (4,4), 179 blocks of four: 10.0 us, 8.3 of two).
+// Few rows, each of several chunks a wave, leave most of the chip idle for the
+// length of a row: there k_hv, with a thread a column and row, is the faster
+// sweep, the more so the fewer dn hops gather through the caches (LDS here).  16
+// sites (1,6), chain 17.7 us against 5.7, 4x4 25.7 against 9.1; impurity of 16 sites
+// (2,6) 39.6 against 20.8, of 13 (3,6) 13.7 against 10.9; 16-site chain (2,5) 13.2
+// against 9.8, 15-site (2,7) 16.8 against 17.5; 4x4 (2,5) 18.1 against 22.4.
+constexpr int64_t kTileFewRows = 64, kTileFewRowsFewHops = 384;  // 1/4 and 3/2 of a block a CU
+constexpr int kTileFewHops = 16;
+
 static TilePlan plan_tile(const ed_op* op) {
   TilePlan p{};
   if (!op->packed || op->size == 0) return p;
@@ -1576,6 +1585,9 @@ static TilePlan plan_tile(const ed_op* op) {
         (p.rb < 4 || blocks >= kTileFourRows))
       break;
   }
+  if (p.rb == 1 && iters > 1 &&
+      op->num_up < (op->max_hops_dn <= kTileFewHops ? kTileFewRowsFewHops : kTileFewRows))
+    return p;
   p.lds_bytes = p.rb * (op->num_dn + 1) * sizeof(double);
   if (p.lds_bytes > kTileLds - 256) return p;  // the kernel has static LDS of its own
   p.nrg = (int)((op->num_up + p.rb - 1) / p.rb);
@@ -1761,6 +1773,12 @@ bool matvec_is_fused(const ed_op* op, int64_t ld) { return !plan_two_pass(op, ld
 
 bool matvec_forms_beta(const ed_op* op, int64_t ld) { return matvec_is_fused(op, ld) && plan_tile(op).ok; }
 
+static int matvec_rows_per_block(const ed_op* op, int64_t ld) {
+  if (plan_two_pass(op, ld).ok) return 0;
+  const TilePlan tp = plan_tile(op);
+  return tp.ok ? tp.rb : -1;
+}
+
 int64_t vector_ld(const ed_op* op) {
   const int64_t nd = op->num_dn;
   const int64_t ld = (nd + 15) / 16 * 16;
@@ -1892,5 +1910,14 @@ extern "C" int ed_op_vector_ld(const ed_op* op, int64_t* ld) {
   clear_error();
   ED_REQUIRE(op && ld, "NULL argument");
   *ld = vector_ld(op);
+  return ED_OK;
+}
+
+extern "C" int ed_op_matvec_rows(const ed_op* op, int64_t ld, int32_t* rows) {
+  clear_error();
+  ED_REQUIRE(op && rows, "NULL argument");
+  ED_REQUIRE(ld >= op->num_dn && ld <= op->num_dn + 4096, "ld=%lld outside [num_dn, num_dn + 4096]",
+             (long long)ld);
+  *rows = matvec_rows_per_block(op, ld);
   return ED_OK;
 }

@@ -4,6 +4,8 @@ one, two and four rows per block, uniform and per-bond hopping, several vectors 
 
 Against the oracle's operator to 1e-13 of the largest entry (the bound of every H.v path)."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -66,3 +68,61 @@ def test_infinities_reach_only_coupled_entries(gpu, ns, nu, nd, uniform):
         inf = np.isinf(want)
         assert np.array_equal(got[inf], want[inf])
         assert np.abs(got[~inf] - want[~inf]).max() <= tol
+
+
+def _rows(op, ld=None):
+    from cmpy_amd import _lib as L
+
+    r = C.c_int32()
+    L.call("ed_op_matvec_rows", op.handle, op.num_dn if ld is None else ld, C.byref(r))
+    return r.value
+
+
+def _random_model(ns, uniform, density=0.3):
+    rng = np.random.default_rng(ns)
+    bonds = [(i, j) for i in range(ns) for j in range(i + 1, ns) if j == i + 1 or rng.random() < density]
+    hops = np.full(len(bonds), -0.7) if uniform else rng.uniform(-1, 1, len(bonds))
+    return bonds, hops, rng.uniform(-1, 1, ns), rng.uniform(0, 4, ns)
+
+
+def _check_hv(op, ref, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((2, ref.size))
+    want = np.stack([ref.matvec(v) for v in x])
+    tol = 1e-13 * max(np.abs(want).max(), 1.0)
+    assert np.abs(op.matvec_device(torch.from_numpy(x).cuda()).cpu().numpy() - want).max() <= tol
+    ld = op.num_dn + 5
+    xp = np.full((2, op.num_up, ld), np.nan)
+    xp[:, :, :op.num_dn] = x.reshape(2, op.num_up, op.num_dn)
+    yp = torch.full((2, op.num_up, ld), float("nan"), dtype=torch.float64, device="cuda")
+    op.matvec_device_ld(torch.from_numpy(xp).cuda(), ld, out=yp)
+    yp = yp.cpu().numpy()
+    assert np.all(yp[:, :, op.num_dn:] == 0.0)
+    assert np.abs(yp[:, :, :op.num_dn].reshape(2, -1) - want).max() <= tol
+
+
+def _check_ground(op, ref):
+    """Unreorthogonalised: every step's H.v carries the recurrence's terms (and a beta of its own or a launch for it)."""
+    from cmpy_amd import groundstate
+
+    gs, st = groundstate(op, tol=1e-9, reorth=False, return_stats=True)
+    assert st.converged
+    r = ref.matvec(gs.state) - gs.energy * gs.state
+    assert np.linalg.norm(r) <= 2e-9 and abs(np.linalg.norm(gs.state) - 1.0) <= 1e-12
+    e = groundstate(op, tol=1e-10, reorth=True).energy
+    assert abs(gs.energy - e) <= 1e-9 * max(abs(e), 1.0)
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ns,nu,nd", [(16, 1, 6), (16, 1, 8), (14, 2, 7), (13, 3, 5)])
+def test_few_long_rows_take_columns(gpu, ns, nu, nd, uniform):
+    """Few rows of several chunks a wave, and rows past the staging space (12,870 states): the fused pass on columns,
+    whose beta is formed by a launch of its own."""
+    from cmpy_amd import SectorHamiltonOperator
+
+    args = (ns, nu, nd, *_random_model(ns, uniform, 0.0), ns)
+    op, ref = SectorHamiltonOperator(*args), O.SectorOperator(*args)
+    assert _rows(op) == _rows(op, op.num_dn + 5) == -1
+    _check_hv(op, ref, nu)
+    if uniform:
+        _check_ground(op, ref)
