@@ -1596,29 +1596,50 @@ static TilePlan plan_tile(const ed_op* op) {
   return p;
 }
 
-// Below this many states the single fused pass is the faster sweep: its rows
-// gather their up-hop sources straight from x, which at this size stays in the
-// last-level cache, and it is one launch instead of two.  Measured with
-// k_hv_tile against two passes: 12-site chain (6,6), D = 853,776: 14.1 against
-// 27.1 us; 13-site chain (6,5), 2.2 M: 30.6 against 50.4; 4x4 (4,4), 3.3 M: 57
-// against 73; 14-site chain (7,7), 11.8 M: 165 against 185 (1+13-site impurity:
-// 147 against 192); 4x4 (5,5), 19 M: 439 against 316; 15-site chain (7,7), 41 M:
-// 745 against 634.
+// Where the two passes are the faster sweep; below, the single fused pass, whose
+// rows gather their up-hop sources straight from x, at these sizes from the
+// last-level cache, in one launch.  Measured, fused against two passes, us:
+//  - k_hv_tile from kTwoPassMinStates up: 4x4 (5,5), 19 M: 437 against 315;
+//    15-site chain (7,7), 41 M: 745 against 634.  Below: 13-site chain (6,5),
+//    2.2 M: 30.3 against 50.4; 4x4 (4,4), 3.3 M: 56 against 68; 14-site chain
+//    (7,7), 11.8 M: 136 against 181 (impurity: 127 against 180).
+//  - Rows of 4,096 states and more with uniform hopping, where the row pass has
+//    half-width tables, from kTwoPassMinStatesLongRows up: a block holds one such
+//    row, so the dn table is read anew for every row.  4x4 (3,5), 2.4 M: 71
+//    against 49; (4,5), 7.9 M: 185 against 142; (4,6), 14.6 M: 321 against 228;
+//    16-site chain (4,5) 123 against 123, (4,6) 211 against 201.  (With per-bond
+//    hopping fused: 16-site impurity (4,5) 161 against 198, 4x4 (4,5) 230 each.)
+//    The same for rows that k_hv_tile does not take (4x4 (5,5) by k_hv 1063).
+//  - In a Lanczos step (lz), uniform hopping: u_{j-1} and w of the step pass
+//    through the last-level cache between two reads of x's rows, so the gathers
+//    miss earlier, by states and hops together, and earlier with two rows a block
+//    (the dn table).  Steps with four: 4x4 (5,4), 7.9 M x 36: 212 against 192;
+//    (4,4), 3.3 M x 32: 86.7 against 90.4.  With two: 14-site chain (7,7), 11.8 M x
+//    28: 252 against 235; (5,6), 6.0 M x 22: 116 against 122; 5x3 (4,5), 4.1 M x 36:
+//    116 against 107.  With per-bond hopping fused (14-site impurity (7,7) 234
+//    against 259, 5x3 (5,5) 249 against 346).
 constexpr int64_t kTwoPassMinStates = int64_t(1) << 24;
-// The same for rows that do not fit k_hv_tile's LDS (k_hv otherwise: 4x4 (5,5)
-// 1063 against 316 us, 12-site chain 19.0 against 27.1).
 constexpr int64_t kTwoPassMinStatesLongRows = int64_t(1) << 21;
+constexpr int64_t kTwoPassLzFourRows = int64_t(1) << 28, kTwoPassLzTwoRows = int64_t(1) << 27;  // states x hops
+static bool two_passes_pay(const ed_op* op, bool lz) {
+  const TilePlan tp = plan_tile(op);
+  if (!tp.ok || op->dn.h16) return op->size >= kTwoPassMinStatesLongRows;
+  if (lz && op->uniform_hop && op->size >= kTwoPassMinStatesLongRows &&
+      op->size * (op->max_hops_up + op->max_hops_dn) >= (tp.rb == 4 ? kTwoPassLzFourRows : kTwoPassLzTwoRows))
+    return true;
+  return op->size >= kTwoPassMinStates;
+}
 
 // Two-pass plan.  Kernels: sign-split tables when hopping is uniform and the
 // tables exist (CMPY_AMD_HV_SPLIT=0 turns them off), general packed tables
-// otherwise.  CMPY_AMD_HV_MODE: 0 single fused pass, 1 two passes, unset =
-// two passes from kTwoPassMinStates up.
-static TwoPassPlan plan_two_pass(const ed_op* op, int64_t ld) {
+// otherwise.  CMPY_AMD_HV_MODE: 0 single fused pass, 1 two passes, unset = two
+// passes where they pay.  lz: the H.v of a Lanczos step.
+static TwoPassPlan plan_two_pass(const ed_op* op, int64_t ld, bool lz) {
   TwoPassPlan p{};
   p.ok = false;
   const int mode = op->hv_mode >= 0 ? op->hv_mode : env_int("CMPY_AMD_HV_MODE", -1);
   if (!op->packed || mode == 0) return p;
-  if (mode < 0 && op->size < (plan_tile(op).ok ? kTwoPassMinStates : kTwoPassMinStatesLongRows)) return p;
+  if (mode < 0 && !two_passes_pay(op, lz)) return p;
   const int maxh_up = maxh_for(op->max_hops_up);
   if (!maxh_up || !maxh_for(op->max_hops_dn)) return p;
   bool uni = op->num_bonds > 0;
@@ -1760,7 +1781,7 @@ static void grid_shape(const ed_op* op, int rb, int64_t ld, int64_t* nrb, int64_
 }
 
 int matvec_num_partials(const ed_op* op, int64_t ld) {
-  const TwoPassPlan p = plan_two_pass(op, ld);
+  const TwoPassPlan p = plan_two_pass(op, ld, true);
   if (p.ok) return (int)(p.col_first ? p.grid_r : p.grid_r + p.grid_c);
   const TilePlan tp = plan_tile(op);
   if (tp.ok) return tp.grid();
@@ -1769,12 +1790,12 @@ int matvec_num_partials(const ed_op* op, int64_t ld) {
   return (int)(nrb * nct);
 }
 
-bool matvec_is_fused(const ed_op* op, int64_t ld) { return !plan_two_pass(op, ld).ok; }
+bool matvec_is_fused(const ed_op* op, int64_t ld) { return !plan_two_pass(op, ld, true).ok; }
 
 bool matvec_forms_beta(const ed_op* op, int64_t ld) { return matvec_is_fused(op, ld) && plan_tile(op).ok; }
 
-static int matvec_rows_per_block(const ed_op* op, int64_t ld) {
-  if (plan_two_pass(op, ld).ok) return 0;
+static int matvec_rows_per_block(const ed_op* op, int64_t ld, bool lz) {
+  if (plan_two_pass(op, ld, lz).ok) return 0;
   const TilePlan tp = plan_tile(op);
   return tp.ok ? tp.rb : -1;
 }
@@ -1785,7 +1806,7 @@ int64_t vector_ld(const ed_op* op) {
   if (ld == nd || env_int("CMPY_AMD_HV_PITCH", 1) == 0) return nd;
   // pad only where the two-pass sweep runs on the padded rows (its column
   // slabs then cover whole 128-byte lines)
-  return plan_two_pass(op, ld).ok ? ld : nd;
+  return plan_two_pass(op, ld, true).ok ? ld : nd;
 }
 
 template <bool LZ>
@@ -1815,7 +1836,7 @@ static int launch_tile(const ed_op* op, const TilePlan& p, const double* x, doub
 static int matvec_block(const ed_op* op, const double* x, double* y, int64_t ld, int64_t nvec, hipStream_t s) {
   const HvEpilogue none{nullptr, nullptr, nullptr, nullptr};
   const int64_t n = op->num_up * ld;
-  const TilePlan tp = plan_two_pass(op, ld).ok ? TilePlan{} : plan_tile(op);
+  const TilePlan tp = plan_two_pass(op, ld, false).ok ? TilePlan{} : plan_tile(op);
   const int64_t step = tp.ok ? 65535 : 1;
   for (int64_t v = 0; v < nvec; v += step) {
     if (tp.ok)
@@ -1828,9 +1849,9 @@ static int matvec_block(const ed_op* op, const double* x, double* y, int64_t ld,
 
 int launch_matvec(const ed_op* op, const double* x, double* y, int64_t ld, const HvEpilogue& epi, hipStream_t s,
                   int* num_partials) {
-  const TwoPassPlan p = plan_two_pass(op, ld);
-  if (p.ok) return launch_two_pass(op, p, x, y, ld, epi, s, num_partials);
   const bool lz = epi.xprev || epi.sx || epi.cprev || epi.partial || epi.cself || epi.psi || epi.beta.j >= 0;
+  const TwoPassPlan p = plan_two_pass(op, ld, lz);
+  if (p.ok) return launch_two_pass(op, p, x, y, ld, epi, s, num_partials);
   const TilePlan tp = plan_tile(op);
   if (tp.ok) {
     if (num_partials) *num_partials = tp.grid();
@@ -1913,11 +1934,11 @@ extern "C" int ed_op_vector_ld(const ed_op* op, int64_t* ld) {
   return ED_OK;
 }
 
-extern "C" int ed_op_matvec_rows(const ed_op* op, int64_t ld, int32_t* rows) {
+extern "C" int ed_op_matvec_rows(const ed_op* op, int64_t ld, int32_t lanczos, int32_t* rows) {
   clear_error();
   ED_REQUIRE(op && rows, "NULL argument");
   ED_REQUIRE(ld >= op->num_dn && ld <= op->num_dn + 4096, "ld=%lld outside [num_dn, num_dn + 4096]",
              (long long)ld);
-  *rows = matvec_rows_per_block(op, ld);
+  *rows = matvec_rows_per_block(op, ld, lanczos != 0);
   return ED_OK;
 }

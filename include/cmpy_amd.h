@@ -137,10 +137,11 @@ int ed_op_matvec_ld(ed_op* op, const double* x_dev, double* y_dev, int64_t ld, i
  * (environment CMPY_AMD_HV_PITCH=0: always num_dn).                         */
 int ed_op_vector_ld(const ed_op* op, int64_t* ld);
 
-/* Which sweep an H.v on rows of ld doubles takes: 0 the two passes, 1, 2 or 4
- * the fused pass with that many rows staged per block, -1 the fused pass on
- * columns (a thread a column, nothing staged).                              */
-int ed_op_matvec_rows(const ed_op* op, int64_t ld, int32_t* rows);
+/* Which sweep an H.v on rows of ld doubles takes, by itself or as part of a
+ * Lanczos step: 0 the two passes, 1, 2 or 4 the fused pass with that many rows
+ * staged per block, -1 the fused pass on columns (a thread a column, nothing
+ * staged).                                                                  */
+int ed_op_matvec_rows(const ed_op* op, int64_t ld, int32_t lanczos, int32_t* rows);
 
 /* y = H x for H given as triples sorted by target row (CSR by target):
  * y[t] = sum_{k=ptr[t]}^{ptr[t+1]-1} val[k] * x[src[k]], in stored order.

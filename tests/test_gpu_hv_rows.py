@@ -70,11 +70,11 @@ def test_infinities_reach_only_coupled_entries(gpu, ns, nu, nd, uniform):
         assert np.abs(got[~inf] - want[~inf]).max() <= tol
 
 
-def _rows(op, ld=None):
+def _rows(op, ld=None, lanczos=0):
     from cmpy_amd import _lib as L
 
     r = C.c_int32()
-    L.call("ed_op_matvec_rows", op.handle, op.num_dn if ld is None else ld, C.byref(r))
+    L.call("ed_op_matvec_rows", op.handle, op.num_dn if ld is None else ld, lanczos, C.byref(r))
     return r.value
 
 
@@ -125,4 +125,43 @@ def test_few_long_rows_take_columns(gpu, ns, nu, nd, uniform):
     assert _rows(op) == _rows(op, op.num_dn + 5) == -1
     _check_hv(op, ref, nu)
     if uniform:
+        _check_ground(op, ref)
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ns,nu,nd", [(16, 3, 5), (14, 7, 7)])
+def test_two_passes_for_long_rows_and_large_lanczos_steps(gpu, ns, nu, nd, uniform):
+    """Uniform hopping: rows of 4,096 states and more take two passes, and so do the steps, on padded rows, of a Lanczos
+    run on the 14-site chain's 11.8 M states, whose single H.v is fused.  Per-bond hopping: all fused."""
+    from cmpy_amd import SectorHamiltonOperator, groundstate
+
+    bonds = O.square_bonds(4, 4) if ns == 16 else O.chain_bonds(ns)
+    rng = np.random.default_rng(ns)
+    hops = np.full(len(bonds), 1.0) if uniform else rng.uniform(0.5, 1, len(bonds))
+    op = SectorHamiltonOperator(ns, nu, nd, bonds, hops, np.full(ns, -2.0), np.full(ns, 4.0), ns)
+    if ns == 16:
+        assert _rows(op) == _rows(op, lanczos=1) == (0 if uniform else 1)
+        _check_hv(op, O.SectorOperator(ns, nu, nd, bonds, hops, np.full(ns, -2.0), np.full(ns, 4.0), ns), nu)
+        return
+    assert _rows(op) == 2 and _rows(op, op.vector_ld, 1) == (0 if uniform else 2)
+    assert op.vector_ld == (3440 if uniform else 3432)
+    gs = groundstate(op, tol=1e-7, reorth=False, device=True)
+    r = op.matvec_device(gs.state) - gs.energy * gs.state
+    assert float(torch.linalg.vector_norm(r)) <= 2e-7
+    v0 = torch.rand(op.size, dtype=torch.float64, device="cuda") - 0.5
+    assert gs.energy <= float(torch.dot(v0, op.matvec_device(v0)) / torch.dot(v0, v0))
+
+
+@pytest.mark.parametrize("uniform", [True, False])
+@pytest.mark.parametrize("ns,nu,nd,rows", [(12, 3, 6, 1), (13, 5, 3, 2), (12, 6, 6, 4), (14, 5, 7, 2)])
+def test_each_number_of_rows_per_block(gpu, ns, nu, nd, rows, uniform):
+    """One, two and four rows a block, with a last block that is not full; the form in a Lanczos step below 10^6 states."""
+    from cmpy_amd import SectorHamiltonOperator
+
+    args = (ns, nu, nd, *_random_model(ns, uniform, 0.0), ns)
+    op, ref = SectorHamiltonOperator(*args), O.SectorOperator(*args)
+    assert _rows(op) == rows
+    _check_hv(op, ref, nu)
+    if op.size < 10 ** 6:
+        assert _rows(op, lanczos=1) == rows
         _check_ground(op, ref)
