@@ -302,21 +302,28 @@ __device__ __forceinline__ double beta_share(const HvBeta& b, int at, int step) 
   return S;
 }
 
+// scale_j and the reference |alpha_j| + beta_j of a pending beta.
+struct BetaRef {
+  double scale, ref;
+};
+__device__ __forceinline__ BetaRef beta_ref(const HvBeta& b) {
+  return {b.c.scale[b.j], fabs(b.c.alpha[b.j]) + (b.j > 0 ? b.c.beta[b.j] : 0.0)};
+}
+
 // scale_{j+1} from the whole sum S, and cprev_{j+1} in *cp; one thread of the
 // launch stores the results and the flags of a broken run, which are not read
 // here, so blocks need no order among them.
-__device__ __forceinline__ double beta_scale(const HvBeta& b, double S, bool store, double* cp) {
+__device__ __forceinline__ double beta_scale(const HvBeta& b, BetaRef r, double S, bool store, double* cp) {
   bool bad;
-  const double sj = b.c.scale[b.j];
-  const double bt = lanczos_beta(S, fabs(b.c.alpha[b.j]) + (b.j > 0 ? b.c.beta[b.j] : 0.0), sj == 0.0, &bad);
+  const double bt = lanczos_beta(S, r.ref, r.scale == 0.0, &bad);
   const double sn = bt > 0.0 ? 1.0 / bt : 0.0;
-  *cp = bt * sj;
+  *cp = bt * r.scale;
   if (store) {
     if (bad) b.c.misc[3] = 1.0;
     if (bt == 0.0) b.c.misc[0] = 1.0;
     b.c.beta[b.j + 1] = bt;
     b.c.scale[b.j + 1] = sn;
-    b.c.cprev[b.j + 1] = bt * sj;
+    b.c.cprev[b.j + 1] = bt * r.scale;
   }
   return sn;
 }
@@ -326,7 +333,7 @@ __device__ __forceinline__ double form_beta(const HvBeta& b, bool store, double*
   double S = beta_share(b, threadIdx.x & 63, 64);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) S += __shfl_xor(S, off, 64);
-  return beta_scale(b, S, store && threadIdx.x == 0, cp);
+  return beta_scale(b, beta_ref(b), S, store && threadIdx.x == 0, cp);
 }
 
 // Lanczos epilogue: y = s_j * H x - c_j * xprev, partial <y, x>.

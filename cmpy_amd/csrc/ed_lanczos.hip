@@ -358,10 +358,14 @@ __global__ __launch_bounds__(kVecThreads) void k_gs_update(const double* __restr
   if (threadIdx.x == 0) wpart[blockIdx.x] = t;
 }
 
-// beta_{j+1} of a step whose H.v-formed beta is needed before the next step.
-__global__ __launch_bounds__(64) void k_form_beta(HvBeta b) {
+// beta_{j+1} of a step whose H.v-formed beta is needed before the next step: an
+// update's 512 partials at once, the step's scalars ahead of the sum.
+__global__ __launch_bounds__(512) void k_form_beta(HvBeta b) {
+  __shared__ double sh[8];
+  const BetaRef r = beta_ref(b);
+  const double S = block_sum(beta_share(b, threadIdx.x, 512), sh);
   double cp;
-  form_beta(b, true, &cp);
+  if (threadIdx.x == 0) beta_scale(b, r, S, true, &cp);
 }
 
 // w -= sum_i coef_i V_i   (sign = -1)   or   w = sum_i coef_i V_i (sign = 0)
@@ -625,7 +629,7 @@ struct EventTimer {
 // A beta still held as partials, formed now (before the coefficients are read).
 static int flush_beta(HvBeta& pend, hipStream_t s) {
   if (pend.j < 0) return ED_OK;
-  hipLaunchKernelGGL(k_form_beta, dim3(1), dim3(64), 0, s, pend);
+  hipLaunchKernelGGL(k_form_beta, dim3(1), dim3(512), 0, s, pend);
   pend.j = -1;
   ED_HIP(hipGetLastError());
   return ED_OK;

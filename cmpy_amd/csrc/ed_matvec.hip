@@ -741,7 +741,7 @@ __global__ __launch_bounds__(1024) void k_hv_tile(Hv2Args a, const double* __res
       if (forms) {
         double S = 0.0;
         for (int w = 0; w < nt / 64; ++w) S += red[w];
-        sx = beta_scale(e.beta, S, blockIdx.x == 0 && threadIdx.x == 0, &cp);
+        sx = beta_scale(e.beta, beta_ref(e.beta), S, blockIdx.x == 0 && threadIdx.x == 0, &cp);
       }
       first = false;
     }
