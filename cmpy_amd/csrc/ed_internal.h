@@ -367,12 +367,16 @@ bool matvec_forms_beta(const ed_op* op, int64_t ld);
 // (128-byte rows) where the two-pass sweep runs, num_dn otherwise.
 int64_t vector_ld(const ed_op* op);
 
+// Grants a kernel `bytes` of dynamic LDS on the current device (needed above 64
+// KiB, once per kernel and device); false if refused.  ed_reorth.hip.
+bool grant_lds(const void* kernel, size_t bytes);
+
 // Fully reorthogonalised steps (ed_reorth.hip): blocks of 64 * sub states.
 struct ReorthGrid {
   int blocks, sub;
 };
 ReorthGrid reorth_grid(int64_t D);
-bool reorth_available();                // the kernels' LDS is granted
+bool reorth_available();                // the kernels' LDS is granted on the current device
 constexpr int kReorthMaxVectors = 256;  // basis vectors a step's kernels hold in LDS
 // Step j < kReorthMaxVectors from V_0..V_j (vectors of D doubles, contiguous
 // rows) into V_{j+1}: alpha_j, and |V_{j+1}|^2 as `blocks` partials in nout.

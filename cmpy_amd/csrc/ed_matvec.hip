@@ -1488,23 +1488,6 @@ static bool lds_starts_at_zero(RowKernel k) {
   return ok;
 }
 
-// Grants a row kernel `bytes` of dynamic LDS (needed above 64 KiB); false if refused.
-static bool ensure_row_lds(RowKernel k, size_t bytes) {
-  static std::mutex mu;
-  static std::vector<std::pair<const void*, size_t>> granted;
-  if (bytes <= 65536) return true;
-  std::lock_guard<std::mutex> lk(mu);
-  for (auto& g : granted)
-    if (g.first == (const void*)k && g.second >= bytes) return true;
-  const hipError_t err = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-  if (err != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  granted.emplace_back((const void*)k, bytes);
-  return true;
-}
-
 template <int TW>
 static ColKernel col_kernel_tw(int maxh, bool uni) {
   switch (maxh) {
@@ -1677,7 +1660,7 @@ static TwoPassPlan plan_two_pass(const ed_op* op, int64_t ld, bool lz) {
     p.lds_bytes = row_bytes * R + 8 * 128;
     p.rk = uni ? k_hv_rows<true> : k_hv_rows<false>;
   }
-  if (!ensure_row_lds(p.rk, p.lds_bytes)) return p;
+  if (!grant_lds((const void*)p.rk, p.lds_bytes)) return p;
   p.grid_r = (op->num_up + R - 1) / R;
   if (split) {
     // 64-column tiles: one hop per load instruction, so the source row and
@@ -1734,7 +1717,7 @@ static TwoPassPlan plan_two_pass(const ed_op* op, int64_t ld, bool lz) {
         p.rk = k_hv_rows_off<1, true>;
       else
         p.rk = k_hv_rows_off<4, true>;
-      if (!ensure_row_lds(p.rk, p.lds_bytes)) {
+      if (!grant_lds((const void*)p.rk, p.lds_bytes)) {
         p.ok = false;
         return p;
       }

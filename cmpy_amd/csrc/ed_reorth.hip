@@ -243,18 +243,31 @@ ReorthGrid reorth_grid(int64_t D) {
   return g;
 }
 
+bool grant_lds(const void* kernel, size_t bytes) {
+  struct Grant {
+    int device;
+    const void* kernel;
+    size_t bytes;
+  };
+  static std::mutex mu;
+  static std::vector<Grant> granted;
+  if (bytes <= 65536) return true;
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> lk(mu);
+  for (const Grant& g : granted)
+    if (g.device == dev && g.kernel == kernel && g.bytes >= bytes) return true;
+  if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  granted.push_back({dev, kernel, bytes});
+  return true;
+}
+
 bool reorth_available() {
-  static std::once_flag once;
-  static bool ok = false;
-  std::call_once(once, [] {
-    const int bytes = kReorthMaxVectors * 64 * (int)sizeof(double);
-    ok = hipFuncSetAttribute((const void*)k_reorth_hv, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) ==
-             hipSuccess &&
-         hipFuncSetAttribute((const void*)k_reorth_pass, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) ==
-             hipSuccess;
-    if (!ok) (void)hipGetLastError();
-  });
-  return ok;
+  const size_t bytes = kReorthMaxVectors * 64 * sizeof(double);
+  return grant_lds((const void*)k_reorth_hv, bytes) && grant_lds((const void*)k_reorth_pass, bytes);
 }
 
 int launch_reorth_step(const ed_op* op, const double* V, int64_t D, int j, LzCoef c, double* part, double* part2,
