@@ -196,9 +196,9 @@ __global__ __launch_bounds__(kReorthThreads) void k_reorth_pass(const double* __
     }
     d = group_sum(d, L, lg);
     if ((int)threadIdx.x <= j) {
-      const double s = c.scale[threadIdx.x];
-      cs[threadIdx.x] = s * s * d;
-      if (first && (int)threadIdx.x == j && blockIdx.x == 0) c.alpha[j] = s * d;
+      const double s = c.scale[threadIdx.x], sd = s * d;
+      cs[threadIdx.x] = sd * s;  // (s * s may overflow: the start vector's length is the caller's)
+      if (first && (int)threadIdx.x == j && blockIdx.x == 0) c.alpha[j] = sd;
     }
   }
   double acc = 0.0;

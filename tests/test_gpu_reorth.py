@@ -46,3 +46,19 @@ def test_full_reorthogonalisation_steps(gpu, ns, nu, nd, m):
     T = V @ np.stack([ref.matvec(x) for x in V], axis=1)
     want = np.diag(a) + np.diag(b, 1) + np.diag(b, -1)
     assert np.abs(T - want).max() <= 1e-12 * max(np.abs(want).max(), 1.0)
+
+
+@pytest.mark.parametrize("ns,nu,nd", [(6, 3, 3), (8, 4, 4)])
+@pytest.mark.parametrize("power", [-517, -512, 500])
+def test_start_vectors_of_any_length(gpu, ns, nu, nd, power):
+    """Fully reorthogonalised steps from a start vector whose length is close to the smallest (its square just below the
+    normal numbers, 1 / length squared past the largest) or to the largest with a square: the same ground state."""
+    from cmpy_amd import SectorHamiltonOperator, groundstate
+
+    bonds = O.chain_bonds(ns)
+    op = SectorHamiltonOperator(ns, nu, nd, bonds, np.ones(len(bonds)), np.full(ns, -2.0), np.full(ns, 4.0), ns)
+    v0 = np.random.default_rng(5).uniform(-1, 1, op.size)
+    want = groundstate(op, v0=v0, reorth="full")
+    got = groundstate(op, v0=np.ldexp(v0, power), reorth="full")
+    assert abs(got.energy - want.energy) <= 1e-9 * abs(want.energy)
+    assert 1.0 - abs(got.state @ want.state) <= 1e-9
