@@ -1742,9 +1742,9 @@ __global__ void k_batch_g(Config cf) {
 // One workgroup per model; no orthogonality of Q is assumed (everything is
 // evaluated through K in the sector's state space).
 // ===========================================================================
-// A continued-fraction part whose K products run device-wide (its Krylov
-// basis is long): P = Qt Re W by the grouped matrix-core GEMM, then diag(K)
-// and the bond sums of K over 64-row blocks.
+// A continued-fraction part whose K products run device-wide: P = Qt Re W by the
+// grouped matrix-core GEMM, then diag(K) and the bond sums of K over 64-row
+// blocks.
 struct BwdJob {
   int32_t model, part, m, dt;  // dt: states of the part's sector
   int64_t q_off;               // Krylov basis in the basis store (rows of stride kcap)
@@ -1770,7 +1770,7 @@ constexpr int kRec = 2 * kRecPart + 4 * kMaxBath;    // + dE0/deps_k, psi dH/dep
 
 struct BwdConfig {
   const ModelParams* params;
-  int32_t num_models;
+  int32_t first, last;  // models of this launch
   int32_t* counter;
   char* ws;
   int64_t slot_bytes;
@@ -1802,26 +1802,25 @@ struct BwdConfig {
 
 // Backward slot: the four spin lists (same layout as SlotRef), then
 // N-sector vectors zeta, res, pvec, q; X re/im, Y re/im; diag d; U, U2
-// ([nw][kcap] complex each); ReW [kcap][kcap]; ubar (complex [kcap]);
-// P [vcap][kcap]; scalars.
+// ([nw][kcap] complex each); ubar (complex [kcap]); and, where a part's K
+// products stay in the workgroup, ReW [kcap][kcap] and P [vcap][kcap].
 struct BwdSlot {
   SlotRef lists;  // only the list accessors are used
   __host__ __device__ int64_t vb() const { return align_up(8 * lists.vcap, 256); }
   __host__ __device__ int64_t ub(int nw) const { return align_up(16ll * nw * lists.csteps, 256); }
+  __host__ __device__ int64_t ubarb() const { return align_up(16ll * lists.csteps, 256); }
   __host__ __device__ int64_t wb() const { return align_up(8ll * lists.csteps * lists.csteps, 256); }
   __host__ __device__ int64_t pb() const { return align_up(8ll * lists.vcap * lists.csteps, 256); }
-  __host__ __device__ int64_t bytes(int nw) const {
-    return 4 * lists.list_bytes() + 9 * vb() + 2 * ub(nw) + wb() + align_up(16ll * lists.csteps, 256) + pb() +
-           align_up(8 * 64, 256);
+  __host__ __device__ int64_t bytes(int nw, bool products) const {
+    return 4 * lists.list_bytes() + 9 * vb() + 2 * ub(nw) + ubarb() + (products ? wb() + pb() : 0);
   }
   __device__ char* after_lists() const { return lists.base + 4 * lists.list_bytes(); }
   // 0 zeta, 1 res, 2 pvec, 3 q, 4 Xre, 5 Xim, 6 Yre, 7 Yim, 8 diag
   __device__ double* vec(int i) const { return (double*)(after_lists() + i * vb()); }
   __device__ double* U(int which, int nw) const { return (double*)(after_lists() + 9 * vb() + which * ub(nw)); }
-  __device__ double* ReW(int nw) const { return (double*)(after_lists() + 9 * vb() + 2 * ub(nw)); }
-  __device__ double* ubar(int nw) const { return (double*)((char*)ReW(nw) + wb()); }
-  __device__ double* P(int nw) const { return (double*)((char*)ubar(nw) + align_up(16ll * lists.csteps, 256)); }
-  __device__ double* scal(int nw) const { return (double*)((char*)P(nw) + pb()); }
+  __device__ double* ubar(int nw) const { return U(2, nw); }
+  __device__ double* ReW(int nw) const { return (double*)((char*)ubar(nw) + ubarb()); }
+  __device__ double* P(int nw) const { return (double*)((char*)ReW(nw) + wb()); }
 };
 
 __device__ __forceinline__ cplx cmul(cplx a, cplx b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
@@ -1857,9 +1856,7 @@ constexpr int kBwdLds = 512 * kPc;  // doubles of the backward's LDS staging buf
 constexpr int kBwdMaxSteps = 1024;  // continued-fraction steps a kept basis may hold
 // Parts run their K products device-wide (backward ms, device-wide against one
 // workgroup a model for parts below 96 steps: 4 models x 7 baths 1.8 / 6.4, 64 x
-// 5 1.3 / 1.7, 512 x 5 3.5 / 3.9, 300 x 7 11.9 / 14.2, 16 x 9 54 / 194); those
-// below kBwdSplitM only while the job store leaves half of the free memory.
-constexpr int kBwdSplitM = 96;
+// 5 1.3 / 1.7, 512 x 5 3.5 / 3.9, 300 x 7 11.9 / 14.2, 16 x 9 54 / 194).
 
 // u_n = sigma |phi| (sigma z_n + e0 - T)^-1 e1 by a complex Thomas solve, one
 // thread per frequency, into Uc (Ur holds the eliminated right-hand sides).
@@ -2170,8 +2167,8 @@ __device__ void backward_model(const Group<true>& g, const BwdConfig& bc, int mi
     const double* gre = bc.gre + (int64_t)mi * nw;
     const double* gim = bc.gim + (int64_t)mi * nw;
     if (job >= 0) {
-      // long basis: A and B of Re W = A B^T to the job store (the product
-      // and everything after it run device-wide)
+      // A and B of Re W = A B^T to the job store (the product and everything
+      // after it run device-wide)
       const BwdJob& jb = bc.jobs[job];
       double* const Aj = bc.jstore + jb.a_off;
       double* const Bj = bc.jstore + jb.b_off;
@@ -2466,9 +2463,9 @@ __global__ __launch_bounds__(kBlock) void k_batch_backward(BwdConfig bc) {
   while (true) {
     if (threadIdx.x == 0) popped = atomicAdd(bc.counter, 1);
     __syncthreads();
-    const int q = __builtin_amdgcn_readfirstlane(popped);
+    const int q = bc.first + __builtin_amdgcn_readfirstlane(popped);
     __syncthreads();
-    if (q >= bc.num_models) break;
+    if (q >= bc.last) break;
     backward_model(g, bc, q, bs, wl);
   }
 }
@@ -2664,13 +2661,9 @@ struct ed_batch {
   int32_t* d_bcounter = nullptr;
   // backward: parts whose K products run device-wide (tables and stores)
   std::vector<int64_t> h_off_q;
-  int32_t* d_job_of = nullptr;
-  BwdJob* d_jobs = nullptr;
-  BwdGemm* d_gemms = nullptr;
-  BwdTile* d_tiles = nullptr;
-  BwdBlock* d_blocks = nullptr;
+  char* d_tables = nullptr;  // job of each part, jobs, products, their tiles, row blocks
   double *d_jstore = nullptr, *d_rec = nullptr, *d_partial = nullptr;
-  int64_t cap_jobs = 0, cap_gemms = 0, cap_tiles = 0, cap_blocks = 0, cap_jstore = 0, cap_grad = 0;
+  int64_t cap_tables = 0, cap_partial = 0, cap_jstore = 0, cap_grad = 0;
   char* d_bws = nullptr;
   int64_t bws_bytes = 0;
   int32_t solved_nw = -1;  // frequencies of the last solve (the backward uses them)
@@ -2700,8 +2693,8 @@ static void free_batch(ed_batch* b) {
                   (void*)b->d_resid, (void*)b->d_wn, (void*)b->d_iters, (void*)b->d_ws, (void*)b->d_off_psi,
                   (void*)b->d_off_q, (void*)b->d_store_psi, (void*)b->d_store_q, (void*)b->d_store_coef,
                   (void*)b->d_gre, (void*)b->d_gim, (void*)b->d_grad_eps, (void*)b->d_grad_v, (void*)b->d_cg,
-                  (void*)b->d_bcounter, (void*)b->d_bws, (void*)b->d_gs_store, (void*)b->d_off_gs, (void*)b->d_job_of,
-                  (void*)b->d_jobs, (void*)b->d_gemms, (void*)b->d_tiles, (void*)b->d_blocks, (void*)b->d_jstore, (void*)b->d_rec,
+                  (void*)b->d_bcounter, (void*)b->d_bws, (void*)b->d_gs_store, (void*)b->d_off_gs, (void*)b->d_tables,
+                  (void*)b->d_jstore, (void*)b->d_rec,
                   (void*)b->d_partial})
     if (p) (void)hipFree(p);
   delete b;
@@ -2717,6 +2710,18 @@ static int balloc(T** p, int64_t n) {
     return set_error(ED_ERR_NOMEM, "hipMalloc of %lld bytes failed: %s", (long long)(sizeof(T) * n),
                      hipGetErrorString(e));
   }
+  return ED_OK;
+}
+
+// A buffer that grows to n entries; what it held is lost.
+template <typename T>
+static int grow(T** p, int64_t* cap, int64_t n) {
+  if (n <= *cap) return ED_OK;
+  *cap = 0;
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  ED_TRY(balloc(p, n));
+  *cap = n;
   return ED_OK;
 }
 
@@ -3049,7 +3054,7 @@ extern "C" int ed_batch_create(ed_batch** out, const ed_batch_desc* d, void* str
         (rc = balloc(&b->d_store_psi, np)) != ED_OK || (rc = balloc(&b->d_store_q, nq)) != ED_OK ||
         (rc = balloc(&b->d_grad_eps, M * d->max_bath)) != ED_OK || (rc = balloc(&b->d_grad_v, M * d->max_bath)) != ED_OK ||
         (rc = balloc(&b->d_cg, M)) != ED_OK || (rc = balloc(&b->d_bcounter, 1)) != ED_OK ||
-        (rc = balloc(&b->d_rec, M * kRec)) != ED_OK || (rc = balloc(&b->d_job_of, 2 * M)) != ED_OK) {
+        (rc = balloc(&b->d_rec, M * kRec)) != ED_OK) {
       free_batch(b);
       return rc;
     }
@@ -3225,6 +3230,90 @@ extern "C" int ed_batch_info(const ed_batch* b, int64_t* wave_max_dim, int32_t* 
   return ED_OK;
 }
 
+// The backward's device-wide stage: jobs, products, tiles and row blocks in the
+// order of the models, and the launches, each of a run of models whose parts fit
+// the job store together.
+struct BwdGroup {
+  int64_t model0, model1;
+  int64_t tw0, tw1, t0, t1, b0, b1;  // its Re W tiles, P tiles and row blocks
+};
+struct BwdPlan {
+  std::vector<int32_t> job_of;
+  std::vector<BwdJob> jobs;
+  std::vector<BwdGemm> gemms;  // Re W = A B^T (m x m, K = 2 nw) and P = Qt Re W^T of each job
+  std::vector<BwdTile> tiles_w, tiles;
+  std::vector<BwdBlock> blocks;
+  std::vector<BwdGroup> groups;
+  int64_t store = 0;  // doubles
+};
+
+static int32_t part_states(const ed_batch* b, int64_t i, int part) {
+  const ModelParams& p = b->params[i];
+  return (int32_t)sector_dim(p.nb + 1, p.n_up + (part == 0 ? 1 : -1), p.n_dn);
+}
+
+// Doubles of the job store that a part of m steps takes: A, B, Re W and P.
+static int64_t part_store(const ed_batch* b, int64_t i, int part, int m, int nw) {
+  return 4ll * m * nw + (int64_t)m * m + (int64_t)part_states(b, i, part) * m;
+}
+
+static void plan_backward(const ed_batch* b, const std::vector<int32_t>& iters, int split_m, int32_t nw, int64_t room,
+                          BwdPlan* plan) {
+  const int64_t M = b->num_models;
+  *plan = BwdPlan{};
+  plan->job_of.assign(2 * M, -1);
+  int64_t jst = 0;
+  BwdGroup g{};
+  const auto close = [&](int64_t i) {
+    g.model1 = i;
+    g.tw1 = (int64_t)plan->tiles_w.size();
+    g.t1 = (int64_t)plan->tiles.size();
+    g.b1 = (int64_t)plan->blocks.size();
+    plan->groups.push_back(g);
+    g = BwdGroup{i, i, g.tw1, g.tw1, g.t1, g.t1, g.b1, g.b1};
+    jst = 0;
+  };
+  for (int64_t i = 0; i < M; ++i) {
+    int64_t need = 0;
+    int steps[2];
+    for (int part = 0; part < 2; ++part) {
+      const int m = iters[3 * i + 1 + part];
+      steps[part] = m > 0 && m >= split_m ? m : 0;
+      if (steps[part]) need += part_store(b, i, part, m, nw);
+    }
+    if (jst + need > room && i > g.model0) close(i);
+    for (int part = 0; part < 2; ++part) {
+      const int m = steps[part];
+      if (!m) continue;
+      BwdJob jb{};
+      jb.model = (int32_t)i;
+      jb.part = part;
+      jb.m = m;
+      jb.dt = part_states(b, i, part);
+      jb.q_off = b->h_off_q[2 * i + part];
+      jb.a_off = jst;
+      jb.b_off = jb.a_off + 2ll * m * nw;
+      jb.w_off = jb.b_off + 2ll * m * nw;
+      jb.p_off = jb.w_off + (int64_t)m * m;
+      jst = jb.p_off + (int64_t)jb.dt * m;
+      jb.blk0 = (int32_t)plan->blocks.size();
+      jb.nblk = (jb.dt + 63) / 64;
+      const int32_t j = (int32_t)plan->jobs.size();
+      for (int32_t r0 = 0; r0 < jb.dt; r0 += 64) plan->blocks.push_back(BwdBlock{j, r0});
+      plan->job_of[2 * i + part] = j;
+      plan->jobs.push_back(jb);
+      plan->gemms.push_back(BwdGemm{jb.a_off, jb.b_off, jb.w_off, 2 * nw, 2 * nw, m, m, 2 * nw, 0});
+      plan->gemms.push_back(BwdGemm{jb.q_off, jb.w_off, jb.p_off, b->kcap, m, jb.dt, m, m, 1});
+      for (int32_t r0 = 0; r0 < m; r0 += 64)
+        for (int32_t c0 = 0; c0 < m; c0 += 64) plan->tiles_w.push_back(BwdTile{2 * j, r0, c0, 0});
+      for (int32_t r0 = 0; r0 < jb.dt; r0 += 64)
+        for (int32_t c0 = 0; c0 < m; c0 += 64) plan->tiles.push_back(BwdTile{2 * j + 1, r0, c0, 0});
+      plan->store = std::max(plan->store, jst);
+    }
+  }
+  close(M);
+}
+
 __global__ void k_reset_one(int32_t* c) {
   if (threadIdx.x == 0) *c = 0;
 }
@@ -3244,6 +3333,44 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
   const int grid = (int)std::min<int64_t>(M, 2 * (int64_t)cus);
+  // parts with at least split_m continued-fraction steps run their K products
+  // device-wide (CMPY_AMD_BWD_SPLIT_M)
+  const int split_m = env_flag("CMPY_AMD_BWD_SPLIT_M", 1);
+  std::vector<int32_t> iters(3 * M);
+  ED_HIP(hipMemcpy(iters.data(), b->d_iters, sizeof(int32_t) * 3 * M, hipMemcpyDeviceToHost));
+  BwdPlan plan;
+  bool products = false;  // of a part that stays in its workgroup
+  int64_t total = 0, largest = 0;
+  for (int64_t i = 0; i < M; ++i) {
+    int64_t need = 0;
+    for (int part = 0; part < 2; ++part) {
+      const int m = iters[3 * i + 1 + part];
+      if (m <= 0) continue;
+      if (m < split_m)
+        products = true;
+      else
+        need += part_store(b, i, part, m, nw);
+    }
+    total += need;
+    largest = std::max(largest, need);
+  }
+  // The job store holds all parts at once where they fit what it has, or that and
+  // half of the free memory; else the models of a launch share it in turn, down
+  // to one at a time.  A part's arithmetic does not depend on its launch.
+  int64_t room = total;
+  if (total > b->cap_jstore) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) == hipSuccess)
+      room = b->cap_jstore + (int64_t)(free_b / (2 * sizeof(double)));
+  }
+  for (;;) {
+    plan_backward(b, iters, split_m, nw, std::max(room, largest), &plan);
+    const int rc = grow(&b->d_jstore, &b->cap_jstore, plan.store);
+    if (rc == ED_OK) break;
+    if (room <= largest) return rc;
+    room = std::min(room, plan.store) / 2;
+    clear_error();
+  }
   int32_t lcap = 1;
   int64_t vcap = 1;
   for (int64_t i = 0; i < M; ++i) {
@@ -3253,106 +3380,35 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
     lcap = std::max<int32_t>(lcap, (int32_t)binom_u(ns, p.n_dn));
     vcap = std::max(vcap, b->dmax[i]);
   }
-  const int64_t slot = BwdSlot{SlotRef{nullptr, lcap, vcap, 0, b->kcap}}.bytes(nw);
-  if (slot * grid > b->bws_bytes) {
-    if (b->d_bws) (void)hipFree(b->d_bws);
-    b->d_bws = nullptr;
-    b->bws_bytes = 0;
-    ED_TRY(balloc(&b->d_bws, slot * grid));
-    b->bws_bytes = slot * grid;
+  const int64_t slot = BwdSlot{SlotRef{nullptr, lcap, vcap, 0, b->kcap}}.bytes(nw, products);
+  ED_TRY(grow(&b->d_bws, &b->bws_bytes, slot * grid));
+  ED_TRY(grow(&b->d_partial, &b->cap_partial, (int64_t)plan.blocks.size() * kRecPart));
+  // the tables one after another, each at a multiple of 16 bytes
+  size_t tables = 0;
+  const auto room_for = [&](const auto& v) {
+    const size_t at = (tables + 15) / 16 * 16;
+    tables = at + sizeof(v[0]) * v.size();
+    return at;
+  };
+  const size_t at_of = room_for(plan.job_of), at_jobs = room_for(plan.jobs), at_gemms = room_for(plan.gemms),
+               at_tw = room_for(plan.tiles_w), at_t = room_for(plan.tiles), at_blocks = room_for(plan.blocks);
+  ED_TRY(grow(&b->d_tables, &b->cap_tables, (int64_t)tables));
+  const auto upload = [&](size_t at, const auto& v) {
+    return hipMemcpy(b->d_tables + at, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice);
+  };
+  ED_HIP(upload(at_of, plan.job_of));
+  if (!plan.jobs.empty()) {
+    ED_HIP(upload(at_jobs, plan.jobs));
+    ED_HIP(upload(at_gemms, plan.gemms));
+    ED_HIP(upload(at_tw, plan.tiles_w));
+    ED_HIP(upload(at_t, plan.tiles));
+    ED_HIP(upload(at_blocks, plan.blocks));
   }
+  const BwdGemm* const gemms = (const BwdGemm*)(b->d_tables + at_gemms);
   ED_HIP(hipMemcpyAsync(b->d_gre, dl_dre, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
   ED_HIP(hipMemcpyAsync(b->d_gim, dl_dim, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
-  // parts with at least split_m continued-fraction steps run their K products
-  // device-wide (CMPY_AMD_BWD_SPLIT_M)
-  const int split_m = env_flag("CMPY_AMD_BWD_SPLIT_M", 1);
-  std::vector<int32_t> iters(3 * M);
-  ED_HIP(hipMemcpy(iters.data(), b->d_iters, sizeof(int32_t) * 3 * M, hipMemcpyDeviceToHost));
-  std::vector<int32_t> job_of(2 * M, -1);
-  std::vector<BwdJob> jobs;
-  std::vector<BwdGemm> gemms;                 // Re W products, then P products
-  std::vector<BwdTile> tiles_w, tiles;        // their tiles
-  std::vector<BwdBlock> blocks;
-  int64_t jst = 0;
-  int64_t room = b->cap_jstore;  // doubles a short part may fill the job store to
-  bool asked = false;
-  for (int64_t i = 0; i < M; ++i) {
-    const ModelParams& p = b->params[i];
-    const int ns = p.nb + 1;
-    for (int part = 0; part < 2; ++part) {
-      const int m = iters[3 * i + 1 + part];
-      const int n_t = p.n_up + (part == 0 ? 1 : -1);
-      if (m <= 0 || m < split_m || n_t < 0 || n_t > ns) continue;
-      BwdJob jb{};
-      jb.model = (int32_t)i;
-      jb.part = part;
-      jb.m = m;
-      jb.dt = (int32_t)sector_dim(ns, n_t, p.n_dn);
-      const int64_t need = 4ll * m * nw + (int64_t)m * m + (int64_t)jb.dt * m;
-      if (m < kBwdSplitM && jst + need > room) {
-        size_t free_b = 0, total_b = 0;
-        if (!asked && hipMemGetInfo(&free_b, &total_b) == hipSuccess)
-          room = b->cap_jstore + (int64_t)(free_b / (2 * sizeof(double)));
-        asked = true;
-        if (jst + need > room) continue;
-      }
-      jb.q_off = b->h_off_q[2 * i + part];
-      jb.a_off = jst;
-      jst += 2ll * m * nw;
-      jb.b_off = jst;
-      jst += 2ll * m * nw;
-      jb.w_off = jst;
-      jst += (int64_t)m * m;
-      jb.p_off = jst;
-      jst += (int64_t)jb.dt * m;
-      jb.blk0 = (int32_t)blocks.size();
-      jb.nblk = (jb.dt + 63) / 64;
-      const int32_t j = (int32_t)jobs.size();
-      for (int32_t r0 = 0; r0 < jb.dt; r0 += 64) blocks.push_back(BwdBlock{j, r0});
-      job_of[2 * i + part] = j;
-      jobs.push_back(jb);
-    }
-  }
-  // Re W = A B^T (m x m, K = 2 nw) for every job, then P = Qt Re W^T
-  const int32_t nj = (int32_t)jobs.size();
-  for (int32_t j = 0; j < nj; ++j) {
-    const BwdJob& jb = jobs[j];
-    gemms.push_back(BwdGemm{jb.a_off, jb.b_off, jb.w_off, 2 * nw, 2 * nw, jb.m, jb.m, 2 * nw, 0});
-    for (int32_t r0 = 0; r0 < jb.m; r0 += 64)
-      for (int32_t c0 = 0; c0 < jb.m; c0 += 64) tiles_w.push_back(BwdTile{j, r0, c0, 0});
-  }
-  for (int32_t j = 0; j < nj; ++j) {
-    const BwdJob& jb = jobs[j];
-    gemms.push_back(BwdGemm{jb.q_off, jb.w_off, jb.p_off, b->kcap, jb.m, jb.dt, jb.m, jb.m, 1});
-    for (int32_t r0 = 0; r0 < jb.dt; r0 += 64)
-      for (int32_t c0 = 0; c0 < jb.m; c0 += 64) tiles.push_back(BwdTile{nj + j, r0, c0, 0});
-  }
-  auto grow = [](auto** ptr, int64_t* cap, int64_t n) -> int {
-    if (n <= *cap) return ED_OK;
-    if (*ptr) (void)hipFree(*ptr);
-    *ptr = nullptr;
-    *cap = 0;
-    ED_TRY(balloc(ptr, n));
-    *cap = n;
-    return ED_OK;
-  };
-  ED_TRY(grow(&b->d_jobs, &b->cap_jobs, (int64_t)jobs.size()));
-  ED_TRY(grow(&b->d_gemms, &b->cap_gemms, (int64_t)gemms.size()));
-  ED_TRY(grow(&b->d_tiles, &b->cap_tiles, (int64_t)(tiles_w.size() + tiles.size())));
-  ED_TRY(grow_pair(&b->d_blocks, &b->d_partial, kRecPart, &b->cap_blocks, (int64_t)blocks.size()));
-  ED_TRY(grow(&b->d_jstore, &b->cap_jstore, jst));
-  ED_HIP(hipMemcpy(b->d_job_of, job_of.data(), sizeof(int32_t) * 2 * M, hipMemcpyHostToDevice));
-  if (!jobs.empty()) {
-    ED_HIP(hipMemcpy(b->d_jobs, jobs.data(), sizeof(BwdJob) * jobs.size(), hipMemcpyHostToDevice));
-    ED_HIP(hipMemcpy(b->d_gemms, gemms.data(), sizeof(BwdGemm) * gemms.size(), hipMemcpyHostToDevice));
-    ED_HIP(hipMemcpy(b->d_tiles, tiles_w.data(), sizeof(BwdTile) * tiles_w.size(), hipMemcpyHostToDevice));
-    ED_HIP(hipMemcpy(b->d_tiles + tiles_w.size(), tiles.data(), sizeof(BwdTile) * tiles.size(),
-                     hipMemcpyHostToDevice));
-    ED_HIP(hipMemcpy(b->d_blocks, blocks.data(), sizeof(BwdBlock) * blocks.size(), hipMemcpyHostToDevice));
-  }
   BwdConfig bc{};
   bc.params = b->d_params;
-  bc.num_models = (int32_t)M;
   bc.counter = b->d_bcounter;
   bc.ws = b->d_bws;
   bc.slot_bytes = slot;
@@ -3376,25 +3432,30 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   bc.grad_eps = b->d_grad_eps;
   bc.grad_v = b->d_grad_v;
   bc.cg_iters = b->d_cg;
-  bc.job_of = b->d_job_of;
-  bc.jobs = b->d_jobs;
-  bc.blocks = b->d_blocks;
+  bc.job_of = (const int32_t*)(b->d_tables + at_of);
+  bc.jobs = (const BwdJob*)(b->d_tables + at_jobs);
   bc.jstore = b->d_jstore;
   bc.rec = b->d_rec;
-  bc.partial = b->d_partial;
   hipEvent_t e0, e1;
   ED_HIP(hipEventCreate(&e0));
   ED_HIP(hipEventCreate(&e1));
   (void)hipEventRecord(e0, s);
-  hipLaunchKernelGGL(k_reset_one, dim3(1), dim3(64), 0, s, b->d_bcounter);
-  hipLaunchKernelGGL(k_batch_backward, dim3((unsigned)grid), dim3(kBlock), 0, s, bc);
-  if (!jobs.empty()) {
-    hipLaunchKernelGGL(k_bwd_gemm, dim3((unsigned)tiles_w.size()), dim3(256), 0, s, (const BwdGemm*)b->d_gemms,
-                       (const BwdTile*)b->d_tiles, (const double*)b->d_store_q, b->d_jstore);
-    hipLaunchKernelGGL(k_bwd_gemm, dim3((unsigned)tiles.size()), dim3(256), 0, s, (const BwdGemm*)b->d_gemms,
-                       (const BwdTile*)(b->d_tiles + tiles_w.size()), (const double*)b->d_store_q, b->d_jstore);
-    hipLaunchKernelGGL(k_bwd_sums, dim3((unsigned)blocks.size()), dim3(256), 0, s, bc);
+  for (const BwdGroup& g : plan.groups) {
+    bc.first = (int32_t)g.model0;
+    bc.last = (int32_t)g.model1;
+    bc.blocks = (const BwdBlock*)(b->d_tables + at_blocks) + g.b0;
+    bc.partial = b->d_partial + g.b0 * kRecPart;
+    hipLaunchKernelGGL(k_reset_one, dim3(1), dim3(64), 0, s, b->d_bcounter);
+    hipLaunchKernelGGL(k_batch_backward, dim3((unsigned)std::min<int64_t>(grid, g.model1 - g.model0)), dim3(kBlock), 0,
+                       s, bc);
+    if (g.b1 == g.b0) continue;
+    hipLaunchKernelGGL(k_bwd_gemm, dim3((unsigned)(g.tw1 - g.tw0)), dim3(256), 0, s, gemms,
+                       (const BwdTile*)(b->d_tables + at_tw) + g.tw0, (const double*)b->d_store_q, b->d_jstore);
+    hipLaunchKernelGGL(k_bwd_gemm, dim3((unsigned)(g.t1 - g.t0)), dim3(256), 0, s, gemms,
+                       (const BwdTile*)(b->d_tables + at_t) + g.t0, (const double*)b->d_store_q, b->d_jstore);
+    hipLaunchKernelGGL(k_bwd_sums, dim3((unsigned)(g.b1 - g.b0)), dim3(256), 0, s, bc);
   }
+  bc.partial = b->d_partial;
   hipLaunchKernelGGL(k_bwd_combine, dim3((unsigned)M), dim3(64), 0, s, bc);
   const hipError_t el = hipGetLastError();
   (void)hipEventRecord(e1, s);

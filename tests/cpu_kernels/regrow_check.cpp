@@ -5,7 +5,8 @@
 //
 // Arguments: a script of steps run on one batch of two small models,
 //   sN  solve with N frequencies       b   backward
-//   fN  the N-th allocation from here (0 = the next) fails
+//   fN  the N-th allocation from here (0 = the next) fails; with kK before it,
+//       and the K - 1 after it
 //   z   solve with 3 frequencies, the last of them zero (refused)
 // Output: "solve rc" / "grad rc v..." per step.
 #include <fstream>
@@ -13,10 +14,14 @@
 
 #include <hip/hip_runtime.h>
 
-static long g_fail_in = -1;
+static long g_fail_in = -1, g_fail_count = 1;
 template <class T>
 static hipError_t counted_malloc(T** p, size_t n) {
-  if (g_fail_in >= 0 && g_fail_in-- == 0) return hipErrorOutOfMemory;
+  if (g_fail_in == 0) {
+    if (--g_fail_count == 0) g_fail_in = -1;
+    return hipErrorOutOfMemory;
+  }
+  if (g_fail_in > 0) --g_fail_in;
   return hipMalloc(p, n);
 }
 #define hipMalloc counted_malloc
@@ -56,6 +61,7 @@ int main(int argc, char** argv) {
     const char op = argv[i][0];
     const long n = std::atol(argv[i] + 1);
     if (op == 'f') g_fail_in = n;
+    if (op == 'k') g_fail_count = n;
     if (op == 's' || op == 'z') {
       const int k = op == 'z' ? 3 : (int)n;
       std::vector<double> wn(k), g(2 * M * k);
