@@ -2661,7 +2661,7 @@ struct ed_batch {
   int32_t* d_bcounter = nullptr;
   // backward: parts whose K products run device-wide (tables and stores)
   std::vector<int64_t> h_off_q;
-  char* d_tables = nullptr;  // job of each part, jobs, products, their tiles, row blocks
+  char* d_tables = nullptr;  // one upload: job of each part, jobs, products, their tiles, row blocks
   double *d_jstore = nullptr, *d_rec = nullptr, *d_partial = nullptr;
   int64_t cap_tables = 0, cap_partial = 0, cap_jstore = 0, cap_grad = 0;
   char* d_bws = nullptr;
@@ -3383,27 +3383,18 @@ extern "C" int ed_batch_backward(ed_batch* b, const double* dl_dre, const double
   const int64_t slot = BwdSlot{SlotRef{nullptr, lcap, vcap, 0, b->kcap}}.bytes(nw, products);
   ED_TRY(grow(&b->d_bws, &b->bws_bytes, slot * grid));
   ED_TRY(grow(&b->d_partial, &b->cap_partial, (int64_t)plan.blocks.size() * kRecPart));
-  // the tables one after another, each at a multiple of 16 bytes
-  size_t tables = 0;
-  const auto room_for = [&](const auto& v) {
-    const size_t at = (tables + 15) / 16 * 16;
-    tables = at + sizeof(v[0]) * v.size();
+  // the tables in one upload, each at a multiple of 16 bytes
+  std::vector<char> tables;
+  const auto put = [&](const auto& v) {
+    const size_t at = (tables.size() + 15) / 16 * 16, n = sizeof(v[0]) * v.size();
+    tables.resize(at + n);
+    if (n) std::memcpy(tables.data() + at, v.data(), n);
     return at;
   };
-  const size_t at_of = room_for(plan.job_of), at_jobs = room_for(plan.jobs), at_gemms = room_for(plan.gemms),
-               at_tw = room_for(plan.tiles_w), at_t = room_for(plan.tiles), at_blocks = room_for(plan.blocks);
-  ED_TRY(grow(&b->d_tables, &b->cap_tables, (int64_t)tables));
-  const auto upload = [&](size_t at, const auto& v) {
-    return hipMemcpy(b->d_tables + at, v.data(), sizeof(v[0]) * v.size(), hipMemcpyHostToDevice);
-  };
-  ED_HIP(upload(at_of, plan.job_of));
-  if (!plan.jobs.empty()) {
-    ED_HIP(upload(at_jobs, plan.jobs));
-    ED_HIP(upload(at_gemms, plan.gemms));
-    ED_HIP(upload(at_tw, plan.tiles_w));
-    ED_HIP(upload(at_t, plan.tiles));
-    ED_HIP(upload(at_blocks, plan.blocks));
-  }
+  const size_t at_of = put(plan.job_of), at_jobs = put(plan.jobs), at_gemms = put(plan.gemms),
+               at_tw = put(plan.tiles_w), at_t = put(plan.tiles), at_blocks = put(plan.blocks);
+  ED_TRY(grow(&b->d_tables, &b->cap_tables, (int64_t)tables.size()));
+  ED_HIP(hipMemcpy(b->d_tables, tables.data(), tables.size(), hipMemcpyHostToDevice));
   const BwdGemm* const gemms = (const BwdGemm*)(b->d_tables + at_gemms);
   ED_HIP(hipMemcpyAsync(b->d_gre, dl_dre, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
   ED_HIP(hipMemcpyAsync(b->d_gim, dl_dim, sizeof(double) * M * nw, hipMemcpyHostToDevice, s));
