@@ -45,17 +45,12 @@ namespace batch {
 constexpr int kMaxBath = ED_BATCH_MAX_BATH;
 constexpr int kMaxSites = kMaxBath + 1;
 constexpr int kBlock = 1024;      // threads per workgroup of the backward kernel
-// Solve kernels, per phase (ground-state tasks, continued-fraction tasks):
-// threads per workgroup (the VGPR budget is 512 / waves per SIMD) and whether
-// block-mode sweeps take the wave-private row path, which needs more than the
-// 128 VGPRs of 16 waves: with 12 waves a ground-state step of 63,504 states
-// takes 103 us against 135 on 16, one of 400 states held on chip 2.0 us against
-// 2.2; the 512-model batch (bath sizes 5..9) 62.8 ms against 69.6.
-constexpr int kBlockGround = 768;
-constexpr bool kFastGround = true;
-constexpr int kBlockFrac = 768;
-constexpr bool kFastFrac = true;
-constexpr int kBlockSolveMax = kBlockGround > kBlockFrac ? kBlockGround : kBlockFrac;
+// Threads per workgroup of the solve kernels (the VGPR budget is 512 / waves per
+// SIMD): their sweeps on wave-private rows need more than the 128 VGPRs of 16
+// waves.  With 12 a ground-state step of 63,504 states takes 103 us against 135
+// on 16, one of 400 states held on chip 2.0 us against 2.2; the 512-model batch
+// (bath sizes 5..9) 62.8 ms against 69.6.
+constexpr int kBlockSolve = 768;
 
 struct ModelParams {
   int32_t nb, n_up, n_dn, pad;
@@ -123,13 +118,12 @@ __device__ __forceinline__ const glb_f64* glb(const double* p) { return (const g
 __device__ __forceinline__ glb_f64* glb(double* p) { return (glb_f64*)p; }
 
 constexpr int kLdsChunks = 64;  // 64-state chunks of the dn sector the LDS cache covers
-// LDS sizes: staged rows (solve kernel: one row of at most 256 columns per
-// wave, 4096 doubles; backward kernel: 2048 doubles, one row of at most 128
-// columns per wave or two buffers of R rows of at most 64 * 16 / R columns),
-// cached dn and up hop slots (12 bytes each) and up-state counts
-constexpr int kLdsRows = 2048;
-// (solve kernel: also the current vector of a sector held on chip, 4,900
-// states at 7 bath sites)
+// LDS sizes: staged rows (one row of at most 64 C columns per wave, or two
+// buffers of R rows of at most 64 / R columns per wave), cached dn and up hop
+// slots (12 bytes each) and up-state counts
+constexpr int kLdsRows = 2048;  // backward kernel: 16 waves, C = 2
+// solve kernel: 12 waves, C = 4, or the current vector of a sector held on chip
+// (4,900 states at 7 bath sites)
 constexpr int kLdsRowsSolve = 4904;
 constexpr int kLdsDnSolve = 4096;   // solve kernel: 48 KiB
 constexpr int kLdsUpSolve = 4096;   // 48 KiB
@@ -327,7 +321,7 @@ struct SlotRef {
   // continued-fraction coefficients: 0 ap, 1 bp, 2 am, 3 bm
   __device__ double* cfc(int i) const { return (double*)(coef_base() + 4 * coef_bytes(miter) + i * coef_bytes(csteps)); }
   __device__ double* scal() const { return (double*)(coef_base() + 4 * coef_bytes(miter) + 4 * coef_bytes(csteps)); }
-  __device__ SpinList list(int l, int32_t n) const { 
+  __device__ SpinList list(int l, int32_t n) const {
     return SpinList{(const glb_u32*)st(l), glb((const double*)dg(l)), (const glb_i32*)cnt(l), (const glb_i32*)tgt(l),
                     glb((const double*)val(l)), n};
   }
@@ -462,15 +456,14 @@ __device__ __forceinline__ T* opaque_uniform(T* p) {
 
 constexpr int kUpPre = 6;  // up hops whose loads start before the staging barrier
 
-
 // Block-mode sweep 1 of lanczos_step with staged rows, for dn sectors of at
-// most 64 * 16 states: w = sj H u - bj sp uprev, returning this thread's part
-// of <w, u>.  Each step stages R = 16 / (64-column chunks per row) rows of u
-// in LDS (one barrier per step, two row buffers); wave wv handles chunk wv % chunks of row wv / chunks: diagonal, up
-// hops from the row's list (uniform over the wave, each hop a contiguous
-// 64-column piece of another row, the first kUpPre loads issued before the
-// staging barrier) and dn hops gathered from the staged row through the
-// cached lists.
+// most 64 states a wave: w = sj H u - bj sp uprev, returning this thread's part
+// of <w, u>.  Each step stages R = waves / (64-column chunks per row) rows of u
+// in LDS (one barrier per step, two row buffers); wave wv handles chunk
+// wv % chunks of row wv / chunks: diagonal, up hops from the row's list
+// (uniform over the wave, each hop a contiguous 64-column piece of another row,
+// the first kUpPre loads issued before the staging barrier) and dn hops gathered
+// from the staged row through the cached lists.
 // LEAN: the row's up-hop list is read once (one entry per lane) and broadcast
 // hop by hop, hop sources are addressed from wave-uniform row bases, and the
 // dn hops go four slots at a time (table reads, then gathers, then the sums
@@ -798,13 +791,13 @@ __device__ __forceinline__ void lanczos_step(const Group<BLOCK>& g, const ModelP
 // lanczos_step as a call of its own: its registers are allocated apart from
 // the caller's (the ground-state task keeps more state live across the step
 // than the 768-thread budget leaves beside the wave-private row sweep).
-template <bool BLOCK, bool FAST, bool LEAN>
+template <bool BLOCK>
 __device__ __noinline__ void lanczos_step_call(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U,
                                                const SpinList& Dn, const glb_f64* __restrict__ u,
                                                const glb_f64* __restrict__ uprev, glb_f64* __restrict__ w, double sj,
                                                double sp, double bj, bool known, double a_in, double* a_out,
                                                double* nrm2) {
-  lanczos_step<BLOCK, FAST, LEAN>(g, p, U, Dn, u, uprev, w, sj, sp, bj, known, a_in, a_out, nrm2);
+  lanczos_step<BLOCK, true, true>(g, p, U, Dn, u, uprev, w, sj, sp, bj, known, a_in, a_out, nrm2);
 }
 
 // 1 / d from the hardware estimate and two Newton steps (to rounding).
@@ -1075,7 +1068,8 @@ __device__ cplx cf_value(const double* a, const double* b, int m, double norm2, 
 constexpr int kResGround = 7;  // states per thread: 768 * 7 >= kLdsRowsSolve
 constexpr int kResFrac = 7;
 constexpr int kResHops = 4;    // hops in flight (a half-filled spin sector of 6 or 8 sites has 3 or 4 slots)
-static_assert(kBlockGround * kResGround >= kLdsRowsSolve && kBlockFrac * kResFrac >= kLdsRowsSolve, "resident states");
+static_assert(kBlockSolve * kResGround >= kLdsRowsSolve && kBlockSolve * kResFrac >= kLdsRowsSolve,
+              "resident states");
 
 template <int S>
 struct Resident {
@@ -1248,7 +1242,7 @@ __device__ __noinline__ int ground_resident(const Group<true>& gr, const ModelPa
 
 // solve_ground's Lanczos loop: the step count, with the Ritz value and its
 // residual.
-template <bool BLOCK, bool FAST>
+template <bool BLOCK>
 __device__ __forceinline__ int ground_loop(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U,
                                            const SpinList& Dn, const SlotRef& sl, double* V, int check_every, int cap,
                                            double tol, double s0, double* theta, double* ritz) {
@@ -1259,7 +1253,7 @@ __device__ __forceinline__ int ground_loop(const Group<BLOCK>& g, const ModelPar
   for (int m = 0;;) {
     const int next = (m / check_every + 1) * check_every < cap ? (m / check_every + 1) * check_every : cap;
     bool done = false;
-    if constexpr (BLOCK && FAST) {
+    if constexpr (BLOCK) {
       if (resident_fits(g, U, Dn)) {
         m = ground_resident(g, p, U, Dn, glb(V), glb(alpha), glb(beta), m, next, s0);
         done = true;
@@ -1268,7 +1262,7 @@ __device__ __forceinline__ int ground_loop(const Group<BLOCK>& g, const ModelPar
     while (!done) {
       double aj, nn;
       const glb_f64* u = glb(V + (int64_t)m * D);
-      lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, u, m > 0 ? u - D : u, glb(V + (int64_t)(m + 1) * D), sj, sp, bj,
+      lanczos_step_call<BLOCK>(g, p, U, Dn, u, m > 0 ? u - D : u, glb(V + (int64_t)(m + 1) * D), sj, sp, bj,
                                            false, 0.0, &aj, &nn);
       const double bn = sqrt(nn);
       if (g.rank == 0) {
@@ -1424,12 +1418,12 @@ __device__ __noinline__ int cf_resident(const Group<true>& gr, const ModelParams
 // continued fraction s n2 / (s z + e0 - a0 - ...) at z = i wmin has converged
 // (CfTrack; the fraction converges last at the frequency closest to the real
 // axis).  Returns the step count.
-template <bool BLOCK, bool FAST>
+template <bool BLOCK>
 __device__ int cf_coeffs(const Group<BLOCK>& g, const ModelParams& p, const SpinList& U, const SpinList& Dn,
                          const SlotRef& sl, double n2, int cap, double e0, double sgn, double wmin, double cf_tol,
                          double* a, double* b, double* qt, int kcap) {
   double* u = sl.vec(1);
-  if constexpr (BLOCK && FAST) {
+  if constexpr (BLOCK) {
     if (resident_fits(g, U, Dn))
       return qt ? cf_resident<true>(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap)
                 : cf_resident<false>(g, p, U, Dn, glb(u), n2, cap, e0, sgn, wmin, cf_tol, glb(a), glb(b), glb(qt), kcap);
@@ -1444,7 +1438,7 @@ __device__ int cf_coeffs(const Group<BLOCK>& g, const ModelParams& p, const Spin
     double aj, nn;
     if (qt)  // keep the normalised Krylov vector v_j = sj u, state-major
       for (int64_t k = g.rank; k < D; k += g.size) qt[k * kcap + j] = sj * u[k];
-    lanczos_step<BLOCK, FAST, true>(g, p, U, Dn, glb(u), glb(up), glb(w), sj, sp, bj, false, 0.0, &aj, &nn);
+    lanczos_step<BLOCK, true, true>(g, p, U, Dn, glb(u), glb(up), glb(w), sj, sp, bj, false, 0.0, &aj, &nn);
     a[j] = aj;
     m = j + 1;
     const double bn = sqrt(nn);
@@ -1495,7 +1489,7 @@ __device__ __noinline__ void combine_psi(const Group<BLOCK>& g, glb_f64* V, cons
   }
 }
 
-template <bool BLOCK, bool FAST>
+template <bool BLOCK>
 __device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config& cf, int mi, SlotRef sl) {
   sl.base = opaque_uniform(sl.base);  // its pointers are not computed ahead of the task loop and kept
   const ModelParams& p = cf.params[mi];
@@ -1527,7 +1521,7 @@ __device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config
   const double s0 = 1.0 / sqrt(n2);
   double theta = 1e300, ritz = 1e300;
   const int cap = (int)((int64_t)cf.max_iter < D ? (int64_t)cf.max_iter : D);
-  const int m = ground_loop<BLOCK, FAST>(g, p, U, Dn, sl, V, cf.check_every, cap, cf.tol, s0, &theta, &ritz);
+  const int m = ground_loop<BLOCK>(g, p, U, Dn, sl, V, cf.check_every, cap, cf.tol, s0, &theta, &ritz);
   // psi = sum_j sv_j s_j V_j in step order, over V_0: each state's entries of
   // every V_j are read by the one member that then overwrites V_0 there
   double* const psi = V;
@@ -1553,7 +1547,7 @@ __device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config
     double aj, nn;
     // w = H psi - theta psi (unit scale, no previous vector, known coefficient)
     double* wr = sl.vec(2);
-    lanczos_step_call<BLOCK, FAST, true>(g, p, U, Dn, glb(psi), glb(sl.vec(0)), glb(wr), 1.0, 0.0, 0.0, true, theta, &aj, &nn);
+    lanczos_step_call<BLOCK>(g, p, U, Dn, glb(psi), glb(sl.vec(0)), glb(wr), 1.0, 0.0, 0.0, true, theta, &aj, &nn);
     double r2 = 0.0;
     for (int64_t k = g.rank; k < D; k += g.size) r2 += wr[k] * wr[k];
     res2 = g.sum(r2);
@@ -1579,7 +1573,7 @@ __device__ __forceinline__ void solve_ground(const Group<BLOCK>& g, const Config
 // coefficients (zero past the step count), |phi|^2 and the step count go to
 // the part's half of the model's coefficient record
 // [a+ | b+ | a- | b- (kcap each) | e0, n2+, n2-, m+, m-].
-template <bool BLOCK, bool FAST>
+template <bool BLOCK>
 __device__ void solve_fraction(const Group<BLOCK>& g, const Config& cf, int mi, int part, const SlotRef& sl) {
   const ModelParams& p = cf.params[mi];
   const int ns = p.nb + 1;
@@ -1619,7 +1613,7 @@ __device__ void solve_fraction(const Group<BLOCK>& g, const Config& cf, int mi, 
       }
     }
     double* qt = cf.keep ? cf.store_q + cf.off_q[2 * mi + part] : nullptr;
-    m = cf_coeffs<BLOCK, FAST>(g, p, T, Dn, sl, nn, cf.cf_steps, theta, part == 0 ? 1.0 : -1.0, cf.wmin, cf.cf_tol, a, b,
+    m = cf_coeffs<BLOCK>(g, p, T, Dn, sl, nn, cf.cf_steps, theta, part == 0 ? 1.0 : -1.0, cf.wmin, cf.cf_tol, a, b,
                          qt, kc);
   }
   // coefficient arrays were written by one member, or by every one with the same values
@@ -1640,7 +1634,7 @@ __device__ void solve_fraction(const Group<BLOCK>& g, const Config& cf, int mi, 
 // fraction tasks, two per model (queue position q >> 1, part q & 1), in the
 // same order.  Each phase pops its own pair of counters.
 template <int PHASE>
-__global__ __launch_bounds__(PHASE ? kBlockFrac : kBlockGround) void k_batch_solve(Config cf) {
+__global__ __launch_bounds__(kBlockSolve) void k_batch_solve(Config cf) {
   __shared__ double red[32];
   __shared__ int popped;
   int32_t* const counters = cf.counters + 2 * PHASE;
@@ -1658,9 +1652,9 @@ __global__ __launch_bounds__(PHASE ? kBlockFrac : kBlockGround) void k_batch_sol
       q = __builtin_amdgcn_readfirstlane(__shfl(q, 0, 64));  // uniform task index
       if (q >= n) break;
       if (PHASE == 0)
-        solve_ground<false, kFastGround>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_wave[q]), sl);
+        solve_ground<false>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_wave[q]), sl);
       else
-        solve_fraction<false, kFastFrac>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_wave[q >> 1]), q & 1, sl);
+        solve_fraction<false>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_wave[q >> 1]), q & 1, sl);
     }
   } else {
     __shared__ double s_rows[kLdsRowsSolve];
@@ -1692,9 +1686,9 @@ __global__ __launch_bounds__(PHASE ? kBlockFrac : kBlockGround) void k_batch_sol
       __syncthreads();
       if (q >= n) break;
       if (PHASE == 0)
-        solve_ground<true, kFastGround>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_block[q]), sl);
+        solve_ground<true>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_block[q]), sl);
       else
-        solve_fraction<true, kFastFrac>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_block[q >> 1]), q & 1, sl);
+        solve_fraction<true>(g, cf, __builtin_amdgcn_readfirstlane(cf.queue_block[q >> 1]), q & 1, sl);
     }
   }
 }
@@ -2784,7 +2778,7 @@ static int configure(ed_batch* b, int64_t wave_max_dim, int grid_blocks, int wav
   if (!qb.empty() && wave_blocks >= grid_blocks) grid_blocks = wave_blocks + 1;
   const int64_t sw = SlotRef{nullptr, lw, vw, b->max_iter, b->cf_steps}.bytes();
   const int64_t sb = SlotRef{nullptr, lb, vb, b->max_iter, b->cf_steps}.bytes();
-  const int64_t n_wave_slots = (int64_t)wave_blocks * (kBlockSolveMax / 64);
+  const int64_t n_wave_slots = (int64_t)wave_blocks * (kBlockSolve / 64);
   const int64_t n_block_slots = grid_blocks - wave_blocks;
   const int64_t bytes = n_wave_slots * sw + n_block_slots * sb + 256;
   if (bytes > b->ws_bytes) {
@@ -2854,8 +2848,8 @@ static int launch(ed_batch* b, hipStream_t s) {
     c.queue_block = b->d_queues + cq[2];
     c.n_block = cq[3];
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, s, b->d_counters);
-    hipLaunchKernelGGL(k_batch_solve<0>, dim3((unsigned)b->grid), dim3(kBlockGround), 0, s, c);
-    hipLaunchKernelGGL(k_batch_solve<1>, dim3((unsigned)b->grid), dim3(kBlockFrac), 0, s, c);
+    hipLaunchKernelGGL(k_batch_solve<0>, dim3((unsigned)b->grid), dim3(kBlockSolve), 0, s, c);
+    hipLaunchKernelGGL(k_batch_solve<1>, dim3((unsigned)b->grid), dim3(kBlockSolve), 0, s, c);
   }
   const int64_t nt = b->num_models * (int64_t)b->cfg.nw;
   if (nt > 0) hipLaunchKernelGGL(k_batch_g, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, s, b->cfg);

@@ -385,7 +385,4 @@ constexpr int kReorthMaxVectors = 256;  // basis vectors a step's kernels hold i
 int launch_reorth_step(const ed_op* op, const double* V, int64_t D, int j, LzCoef c, double* part, double* part2,
                        const HvBeta& prev, double* nout, hipStream_t s);
 
-// Deterministic reductions (ed_lanczos.hip).
-int launch_reduce(const double* partial, int n, double* out, int op_kind, hipStream_t stream);
-
 }  // namespace ed

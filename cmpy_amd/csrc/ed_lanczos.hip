@@ -26,14 +26,14 @@
 
 namespace ed {
 
-enum RedKind { RED_NORM0 = 0, RED_ALPHA = 1, RED_SUM_TO = 3, RED_SQRT_TO = 4 };
+enum RedKind { RED_NORM0, RED_SQRT_TO };
 
 constexpr int kRedThreads = 1024;
 constexpr int kVecThreads = 256;
 typedef double v2d __attribute__((ext_vector_type(2)));
 
 __global__ __launch_bounds__(kRedThreads) void k_reduce(const double* __restrict__ partial, int n,
-                                                        int kind, LzCoef c, int j, double* out) {
+                                                        int kind, LzCoef c, double* out) {
   __shared__ double sh[kRedThreads / 64];
   double v = 0.0;
   for (int i = threadIdx.x; i < n; i += kRedThreads) v += partial[i];
@@ -54,12 +54,6 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce(const double* __restrict
       c.misc[0] = b > 0.0 ? 0.0 : 1.0;
       break;
     }
-    case RED_ALPHA:
-      c.alpha[j] = c.scale[j] * S;
-      break;
-    case RED_SUM_TO:
-      *out = S;
-      break;
     case RED_SQRT_TO:
       *out = sqrt(fmax(S, 0.0));
       break;
@@ -233,10 +227,8 @@ __global__ __launch_bounds__(kVecThreads) void k_scale(double* dst, const double
   }
 }
 
-// partial |w|^2; gate (optional): skip the launch unless *gate != 0
-__global__ __launch_bounds__(kVecThreads) void k_norm2(const double* __restrict__ w, int64_t D, double* partial,
-                                                       const int* gate) {
-  if (gate && *gate == 0) return;
+// partial |w|^2
+__global__ __launch_bounds__(kVecThreads) void k_norm2(const double* __restrict__ w, int64_t D, double* partial) {
   __shared__ double sh[kVecThreads / 64];
   double acc = 0.0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -331,7 +323,7 @@ __global__ __launch_bounds__(kVecThreads) void k_multidot(const double* __restri
 // coef_i = scale_i^2 sum_c dots[i][c] (the ng partials of <V_i, w> per vector
 // that k_multidot left, summed by every block in the same order), then
 // w -= sum_i coef_i V_i, and the partial |w|^2 of this block into
-// wpart[blockIdx.x].  gate as in k_multidot.
+// wpart[blockIdx.x].  gate (optional): skip the launch unless *gate != 0.
 __global__ __launch_bounds__(kVecThreads) void k_gs_update(const double* __restrict__ V, int nv, int64_t D,
                                                            const double* __restrict__ dots, int ng,
                                                            const double* __restrict__ scale, double* __restrict__ w,
@@ -368,11 +360,9 @@ __global__ __launch_bounds__(512) void k_form_beta(HvBeta b) {
   if (threadIdx.x == 0) beta_scale(b, r, S, true, &cp);
 }
 
-// w -= sum_i coef_i V_i   (sign = -1)   or   w = sum_i coef_i V_i (sign = 0)
-__global__ __launch_bounds__(kVecThreads) void k_axpy_multi(const double* __restrict__ V, int nv, int64_t D,
-                                                            const double* __restrict__ coef,
-                                                            double* __restrict__ w, int assign, const int* gate) {
-  if (gate && *gate == 0) return;
+// w = sum_i coef_i V_i
+__global__ __launch_bounds__(kVecThreads) void k_combine(const double* __restrict__ V, int nv, int64_t D,
+                                                         const double* __restrict__ coef, double* __restrict__ w) {
   extern __shared__ double cs[];
   for (int i = threadIdx.x; i < nv; i += blockDim.x) cs[i] = coef[i];
   __syncthreads();
@@ -380,7 +370,7 @@ __global__ __launch_bounds__(kVecThreads) void k_axpy_multi(const double* __rest
   for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < D; k += stride) {
     double acc = 0.0;
     for (int i = 0; i < nv; ++i) acc += cs[i] * V[(int64_t)i * D + k];
-    w[k] = assign ? acc : w[k] - acc;
+    w[k] = acc;
   }
 }
 
@@ -404,13 +394,6 @@ static void launch_update(int vb, hipStream_t s, double* w, const double* u, int
   else
     hipLaunchKernelGGL(k_update, dim3(vb), dim3(kVecThreads), 0, s, w, u, D, alpha, scale, psi, yj, partial,
                        hv_part, np);
-}
-
-int launch_reduce(const double* partial, int n, double* out, int kind, hipStream_t stream) {
-  LzCoef c{};
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, stream, partial, n, kind, c, 0, out);
-  ED_HIP(hipGetLastError());
-  return ED_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -731,7 +714,7 @@ static int reorth_start(const LzLayout& L, LzCoef c, double* part, const ReorthC
   const int vb = vec_blocks(L.D);
   // V_0 = the start vector, unnormalised (v_0 = scale_0 V_0)
   launch_start(L, s, r.V, v0, seed, part);
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, 0, nullptr);
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, nullptr);
   ED_HIP(hipGetLastError());
   return ED_OK;
 }
@@ -975,7 +958,7 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
     double* u[3] = {vec_ptr(base, L, 0), vec_ptr(base, L, 1), vec_ptr(base, L, 2)};
     double* psi = cfg->want_vector ? vec_ptr(base, L, 3) : nullptr;
     launch_start(L, s, u[0], v0_dev, cfg->seed, part);
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, 0, nullptr);
+    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, nullptr);
     ED_HIP(hipGetLastError());
     int ip = 2, ic = 0, iw = 1;  // u_prev, u_cur, w
     int steps = 0;
@@ -1049,8 +1032,8 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
       std::vector<double> yc(m);
       for (int k = 0; k < m; ++k) yc[k] = y[k] / hb[k];
       ED_HIP(hipMemcpyAsync(coefs, yc.data(), sizeof(double) * m, hipMemcpyHostToDevice, s));
-      hipLaunchKernelGGL(k_axpy_multi, dim3(vb), dim3(kVecThreads), sizeof(double) * m, s, V, m, D, coefs,
-                         vec_ptr(base, L, M + 1), 1, nullptr);
+      hipLaunchKernelGGL(k_combine, dim3(vb), dim3(kVecThreads), sizeof(double) * m, s, V, m, D, coefs,
+                         vec_ptr(base, L, M + 1));
       ED_HIP(hipStreamSynchronize(s));  // yc goes out of scope
       ED_HIP(hipGetLastError());
     }
@@ -1065,14 +1048,14 @@ extern "C" int ed_lanczos_groundstate(ed_op* op, const ed_lanczos_cfg* cfg, cons
     // normalise psi (in place, padded layout), compute the explicit residual
     // |H psi - e0 psi|, and write psi into psi_dev in the contiguous layout
     double* psi = cfg->reorth ? vec_ptr(base, L, M + 1) : vec_ptr(base, L, 3);
-    hipLaunchKernelGGL(k_norm2, dim3(vb), dim3(kVecThreads), 0, s, psi, D, part, nullptr);
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_SQRT_TO, c, 0, c.misc + 4);
+    hipLaunchKernelGGL(k_norm2, dim3(vb), dim3(kVecThreads), 0, s, psi, D, part);
+    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_SQRT_TO, c, c.misc + 4);
     hipLaunchKernelGGL(k_scale, dim3(vb), dim3(kVecThreads), 0, s, psi, psi, D, c.misc + 4, 1, nullptr);
     double* w = vec_ptr(base, L, 0);
     HvEpilogue none{nullptr, nullptr, nullptr, nullptr};
     ED_TRY(launch_matvec(op, psi, w, L.ld, none, s, nullptr));
     hipLaunchKernelGGL(k_resid, dim3(vb), dim3(kVecThreads), 0, s, w, psi, D, e0, part);
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_SQRT_TO, c, 0, c.misc + 5);
+    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_SQRT_TO, c, c.misc + 5);
     launch_compact(L, s, psi_dev, psi, 0, 1, nullptr, 0);
     ED_HIP(hipGetLastError());
     double r[2];
@@ -1130,7 +1113,7 @@ extern "C" int ed_lanczos_coeffs(ed_op* op, const double* v0_dev, int32_t nsteps
   } else {
     double* u[3] = {vec_ptr(base, L, 0), vec_ptr(base, L, 1), vec_ptr(base, L, 2)};
     launch_start(L, s, u[0], v0_dev, 0, part);
-    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, 0, nullptr);
+    hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kRedThreads), 0, s, part, vb, (int)RED_NORM0, c, nullptr);
     ED_HIP(hipGetLastError());
     int ip = 2, ic = 0, iw = 1;
     HvBeta pend;
