@@ -1605,9 +1605,10 @@ constexpr int64_t kTwoPassMinStates = int64_t(1) << 24;
 constexpr int64_t kTwoPassMinStatesLongRows = int64_t(1) << 21;
 constexpr int64_t kTwoPassLzFourRows = int64_t(1) << 28, kTwoPassLzTwoRows = int64_t(1) << 27;  // states x hops
 static bool two_passes_pay(const ed_op* op, bool lz) {
+  if (op->size < kTwoPassMinStatesLongRows) return false;
   const TilePlan tp = plan_tile(op);
-  if (!tp.ok || op->dn.h16) return op->size >= kTwoPassMinStatesLongRows;
-  if (lz && op->uniform_hop && op->size >= kTwoPassMinStatesLongRows &&
+  if (!tp.ok || op->dn.h16) return true;
+  if (lz && op->uniform_hop &&
       op->size * (op->max_hops_up + op->max_hops_dn) >= (tp.rb == 4 ? kTwoPassLzFourRows : kTwoPassLzTwoRows))
     return true;
   return op->size >= kTwoPassMinStates;
