@@ -642,11 +642,11 @@ __global__ __launch_bounds__(kRowThreads) void k_hv_rows_held(Hv2Args a, int row
 // 64-column piece of another row, UP of them in flight a row), dn hops are LDS
 // gathers through the packed column-major table, whose entries serve all RB
 // rows.  Slots past a state's count take nothing from x, so that an infinity
-// reaches only the entries that H couples to it: an up slot is branched over (a
-// row's count is uniform; a load in its place costs as much as half of a star's
-// hops, whose rows have 3 and 13 of them: 13-site impurity (4,5) 24.0 us, 16.5
-// without), a dn slot gathers the zero past its
-// row.  Blocks go to XCDs in contiguous runs of rows, whose hop sources lie
+// reaches only the entries that H couples to it: a dn slot gathers the zero past
+// its row, an up slot is branched over (a row's count is uniform).  Where rows
+// differ in length its load is left out too: it costs as much as half of a star's
+// hops, whose rows have 3 and 13 of them (13-site impurity (4,5) 24.0 us, 16.5
+// without).  Blocks go to XCDs in contiguous runs of rows, whose hop sources lie
 // mostly near them.  blockIdx.y picks the vector.  Every wave has a chunk (at
 // most nch waves a block).
 // ---------------------------------------------------------------------------
@@ -1542,9 +1542,10 @@ constexpr size_t kTileLds = 64 * 1024;  // granted without an attribute, and two
 constexpr int kTileMaxThreads = 1024;
 
 // Rows per block: as many as keep kTileWaves waves in flight, up to four (the dn
-// table's entries are read once for all of a block's rows; 12-site chain: 14.1 us
-// with four rows, 15.2 with two, 16.7 with one), four only for kTileFourRows
-// blocks or more (13-site chain (4,4), 179 blocks of four: 10.0 us, 8.3 of two).
+// table's entries are read once for all of a block's rows: a Lanczos step on the
+// 12-site chain (6,5) 25.5 us with four rows, 27.3 with two, on 5x3 (5,4) 96 and
+// 111; 4x4 (4,4) 56.3 and 59.9), four only for kTileFourRows blocks or more
+// (13-site chain (4,4), 179 blocks of four: 10.0 us, 8.3 of two).
 // Few rows, each of several chunks a wave, leave most of the chip idle for the
 // length of a row: there k_hv, with a thread a column and row, is the faster
 // sweep, the more so the fewer dn hops gather through the caches (LDS here).  16
@@ -1593,14 +1594,14 @@ static TilePlan plan_tile(const ed_op* op) {
 //    16-site chain (4,5) 123 against 123, (4,6) 211 against 201.  (With per-bond
 //    hopping fused: 16-site impurity (4,5) 161 against 198, 4x4 (4,5) 230 each.)
 //    The same for rows that k_hv_tile does not take (4x4 (5,5) by k_hv 1063).
-//  - In a Lanczos step (lz), uniform hopping: u_{j-1} and w of the step pass
-//    through the last-level cache between two reads of x's rows, so the gathers
-//    miss earlier, by states and hops together, and earlier with two rows a block
-//    (the dn table).  Steps with four: 4x4 (5,4), 7.9 M x 36: 212 against 192;
-//    (4,4), 3.3 M x 32: 86.7 against 90.4.  With two: 14-site chain (7,7), 11.8 M x
-//    28: 252 against 235; (5,6), 6.0 M x 22: 116 against 122; 5x3 (4,5), 4.1 M x 36:
-//    116 against 107.  With per-bond hopping fused (14-site impurity (7,7) 234
-//    against 259, 5x3 (5,5) 249 against 346).
+//  - In a Lanczos step (lz) with uniform hopping, where u_{j-1}, w and the
+//    update's streams share the caches with x: earlier, by states and hops
+//    together, and earlier still with two rows a block.  Steps with four: 4x4
+//    (5,4), 7.9 M x 36: 212 against 192; (4,4), 3.3 M x 32: 86.7 against 90.4.
+//    With two: 14-site chain (7,7), 11.8 M x 28: 252 against 235; (5,6), 6.0 M x
+//    22: 116 against 122; 5x3 (4,5), 4.1 M x 36: 116 against 107.  With per-bond
+//    hopping fused (14-site impurity (7,7) 234 against 259, 5x3 (5,5) 249 against
+//    346).
 constexpr int64_t kTwoPassMinStates = int64_t(1) << 24;
 constexpr int64_t kTwoPassMinStatesLongRows = int64_t(1) << 21;
 constexpr int64_t kTwoPassLzFourRows = int64_t(1) << 28, kTwoPassLzTwoRows = int64_t(1) << 27;  // states x hops
